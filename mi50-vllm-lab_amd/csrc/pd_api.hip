@@ -153,9 +153,7 @@ hipError_t pth_dec_launch_noalloc(const void* q, int q_st, const void* kc, int k
     x.part_o = static_cast<float*>(base);
     x.part_m = x.part_o + rows * kDim;
     x.part_l = x.part_m + rows;
-    e = launch_partial(x, stream);
-    if (e != hipSuccess) return e;
-    return launch_combine(x, stream);
+    return launch_both(x, stream);
 }
 
 hipError_t pth_dec_launch_partial(const void* q, int q_st, const void* kc, int k_sb, int k_ss, int k_sh,

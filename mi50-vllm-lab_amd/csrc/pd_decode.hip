@@ -76,6 +76,7 @@ constexpr int kBtCache = 1024;                     // block-table entries of a s
 // is smaller:
 constexpr int kBtEarly = 384;                      // per-block row offsets (48 tiles per wave)
 constexpr int kBtRaw = 384;                        // raw block-table entries (96 per wave)
+constexpr int kMaxBalancedSegments = 128;          // segments per item of a balanced launch
 constexpr int kBtWave = kBtEarly / 4;              // 16-key blocks staged per wave
 
 // The 17 DMAs of one tile into the slot at LDS address `slot` (8 K blocks, 8 V blocks, tail).
@@ -130,10 +131,34 @@ struct TileOps {
 // 16), so every K/V byte is loaded and widened once. Each wave double-buffers its tiles in LDS:
 // tile n + 1 is copied while tile n is computed, and tile n + 2 is issued as soon as tile n is
 // done, so while the wave waits it has two tiles in flight.
+template <int NRB, bool kEarly>
+struct PartialLds {
+    static constexpr int kStats = kWaves * kWaveLds;      // m, l: [wave][NRB][16]
+    static constexpr int kBt = kStats + 2 * kWaves * NRB * 16 * 4;
+    static constexpr int kRaw = kBt + (kEarly ? kBtEarly : kBtCache) * 8;
+    static constexpr int kQ = kRaw + (kEarly ? kBtRaw * 4 : 0);
+    // (three row blocks: Q is staged in the V images of slot 1 of waves 0..2 instead, 16 rows
+    // each; those slots receive their V copies only after Q is in registers)
+    static constexpr bool kQInSlots = NRB >= 3;
+    static constexpr int kBytes = kQ + (kEarly && !kQInSlots ? 16 * NRB * 2 * kDim : 0);
+    static_assert(2 * 17 * 1024 <= kWaveLds && kWaveLds % 16 == 0,
+                  "two row blocks of accumulator blocks fit the slots of their wave");
+    static_assert(kBytes <= 160 * 1024, "gfx950 has 160 KiB of LDS per CU");
+};
+
+// What a workgroup computes: rows [row0, row0 + R) of one GQA group of one sequence over the key tiles
+// of one split, and the segment of the partial buffers it writes.
+struct Work {
+    int g, b, row0;            // kv head, sequence, first row of the group
+    int q0, q_len, seq_len;    // first query token, query tokens, keys (the new tokens' among them)
+    int seg;                   // segment of the partial buffers
+    int tb, te;                // tiles [tb, te) of the split
+    bool interleave;           // the waves instead take every W-th tile from t_first + gw of the ntiles
+    int t_first, ntiles, W;
+};
+
 template <int NRB, bool kFast>
-__global__ void __launch_bounds__(kThreads, 1) pd_partial_kernel(const PartialParams a) {
-    constexpr int kLdsWaves = kWaves * kWaveLds;
-    constexpr int kLdsStats = kLdsWaves;                  // m, l: [wave][NRB][16]
+__device__ __forceinline__ void partial_body(const PartialParams& a, const Work& wk, unsigned char* lds) {
     // kEarly (block sizes that are multiples of 16): Q and the block-table slice are copied into
     // LDS like the tiles, and each wave's
     // first tile is issued before anything is waited for (addressed with scalar block-table
@@ -141,75 +166,27 @@ __global__ void __launch_bounds__(kThreads, 1) pd_partial_kernel(const PartialPa
     // tile's K copies follow at once, its other copies after the set-up (a copy issue stalls
     // while the memory queues are full).
     constexpr bool kEarly = kFast;
-    constexpr int kLdsBt = kLdsStats + 2 * kWaves * NRB * 16 * 4;
-    constexpr int kLdsRaw = kLdsBt + (kEarly ? kBtEarly : kBtCache) * 8;
-    constexpr int kLdsQ = kLdsRaw + (kEarly ? kBtRaw * 4 : 0);
-    // (three row blocks: Q is staged in the V images of slot 1 of waves 0..2 instead, 16 rows
-    // each; those slots receive their V copies only after Q is in registers)
-    constexpr bool kQInSlots = NRB >= 3;
-    constexpr int kQBytes = kEarly && !kQInSlots ? 16 * NRB * 2 * kDim : 0;
-    constexpr int kLdsBytes = kLdsQ + kQBytes;
-    static_assert(2 * 17 * 1024 <= kWaveLds && kWaveLds % 16 == 0,
-                  "two row blocks of accumulator blocks fit the slots of their wave");
-    static_assert(kLdsBytes <= 160 * 1024, "gfx950 has 160 KiB of LDS per CU");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kLdsBytes];
+    using Lds = PartialLds<NRB, kEarly>;
+    constexpr int kLdsStats = Lds::kStats, kLdsBt = Lds::kBt, kLdsRaw = Lds::kRaw, kLdsQ = Lds::kQ;
+    constexpr bool kQInSlots = Lds::kQInSlots;
 
-    // grid z = row slice x sequence: with rslices > 1 the workgroup takes rows [row0, row0 + 16 NRB)
-    // of its GQA group, and the group's other slices read the same tiles
-    const int s = blockIdx.x, g = blockIdx.y;
-    const int rs = a.rslices > 1 ? (int)blockIdx.z / a.num_seqs : 0;
-    const int b = (int)blockIdx.z - rs * a.num_seqs;
-    const int row0 = 16 * NRB * rs;
+    const int g = wk.g, b = wk.b, row0 = wk.row0, q0 = wk.q0, q_len = wk.q_len, seq_len = wk.seq_len;
+    const int tb = wk.tb, te = wk.te, t_first = wk.t_first, ntiles = wk.ntiles, W = wk.W;
+    const bool interleave = wk.interleave;
     const int tid = threadIdx.x, l = tid & 63, lg = l >> 4, li = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform by construction
-
-    // The set-up is a chain of dependent scalar loads (arguments, sequence, block table) before
-    // the first copy: make each link one round trip. Every argument the set-up reads is
-    // requested at once, then the three sequence words together.
-    asm volatile("" ::"s"(a.qsl), "s"(a.seq_lens), "s"(a.block_table), "s"(a.bt_stride), "s"(a.kc), "s"(a.k_sb),
-                 "s"(a.k_ss), "s"(a.k_sh), "s"(a.q), "s"(a.q_st), "s"(a.qmax), "s"(a.G), "s"(a.window),
-                 "s"(a.nsplit), "s"(a.block_size), "s"(a.bs_shift));
-    // (read-only for the kernel's lifetime: scalar loads through the constant address space)
-    const int q0 = ((const_int_ptr)(uintptr_t)a.qsl)[b];
-    const int q_end = ((const_int_ptr)(uintptr_t)a.qsl)[b + 1];
-    const int seq_len = ((const_int_ptr)(uintptr_t)a.seq_lens)[b];
-    asm volatile("" ::"s"(q0), "s"(q_end), "s"(seq_len));
-    const int q_len = q_end - q0;
-    if (q_len <= 0 || seq_len <= 0) return;
     const int ql = min(q_len, a.qmax);
     const int G = a.G;
     const int R = min(16 * NRB, ql * G - row0);  // rows of this workgroup: group rows row0 + [0, R)
-    if (R <= 0) return;                          // a slice past the sequence's rows
     const int ctx0 = seq_len - q_len;  // absolute position of query token 0
     const int lo = a.window > 0 ? max(0, ctx0 - a.window + 1) : 0;
     const int hi = seq_len;
-    const int t_first = lo / kTile;
-    const int ntiles = (hi - 1) / kTile - t_first + 1;
-    // Tiles of each wave. Split s owns a contiguous run of tiles [tb, te) and its waves take every
-    // kWaves-th tile of it, unless the block size is a multiple of 16 and there are at least as
-    // many tiles as the W = kWaves * nsplit waves of a (sequence, kv head): then the waves
-    // interleave over all the tiles, wave gw = kWaves * s + w taking tiles t_first + gw + W n, so
-    // that every split has work and the waves' counts differ by at most one. (Fewer tiles than
-    // waves: the contiguous runs measured faster, fewer workgroups with more waves busy.)
-    const int per_split = (ntiles + a.nsplit - 1) / a.nsplit;
-    const int tb = t_first + s * per_split;
-    const int te = min(t_first + ntiles, tb + per_split);
-    const int W = kWaves * a.nsplit, gw = kWaves * s + w;
-    const bool interleave = kFast && ntiles >= W;
-    const bool empty = interleave ? kWaves * s >= ntiles : tb >= te;
+    const int gw = kWaves * wk.seg + w;  // interleaved: this wave among the W of the (sequence, kv head)
 
     auto prow = [&](int r) -> int64_t {  // partial row index of query row r
         const int i = (row0 + r) / G, hh = (row0 + r) - i * G;
-        return ((int64_t)(q0 + i) * a.Hq + (g * G + hh)) * a.nseg + s;
+        return ((int64_t)(q0 + i) * a.Hq + (g * G + hh)) * a.nseg + wk.seg;
     };
-
-    if (empty) {  // no tiles: mark the split empty for the combine
-        for (int r = tid; r < R; r += kThreads) {
-            a.part_m[prow(r)] = kNegInf;
-            a.part_l[prow(r)] = 0.f;
-        }
-        return;
-    }
 
     const int nt = interleave ? (gw < ntiles ? (ntiles - 1 - gw) / W + 1 : 0)
                               : max(0, (te - tb - w + kWaves - 1) / kWaves);  // tiles of this wave
@@ -844,6 +821,229 @@ __global__ void __launch_bounds__(kThreads, 1) pd_partial_kernel(const PartialPa
     }
 }
 
+// One split of one (sequence, kv head) per workgroup: grid (nsplit, Hkv, num_seqs x slices).
+template <int NRB, bool kFast>
+__global__ void __launch_bounds__(kThreads, 1) pd_partial_kernel(const PartialParams a) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[PartialLds<NRB, kFast>::kBytes];
+
+    // grid z = row slice x sequence: with rslices > 1 the workgroup takes rows [row0, row0 + 16 NRB)
+    // of its GQA group, and the group's other slices read the same tiles
+    const int s = blockIdx.x, g = blockIdx.y;
+    const int rs = a.rslices > 1 ? (int)blockIdx.z / a.num_seqs : 0;
+    const int b = (int)blockIdx.z - rs * a.num_seqs;
+    const int row0 = 16 * NRB * rs;
+
+    // The set-up is a chain of dependent scalar loads (arguments, sequence, block table) before
+    // the first copy: make each link one round trip. Every argument the set-up reads is
+    // requested at once, then the three sequence words together.
+    asm volatile("" ::"s"(a.qsl), "s"(a.seq_lens), "s"(a.block_table), "s"(a.bt_stride), "s"(a.kc), "s"(a.k_sb),
+                 "s"(a.k_ss), "s"(a.k_sh), "s"(a.q), "s"(a.q_st), "s"(a.qmax), "s"(a.G), "s"(a.window),
+                 "s"(a.nsplit), "s"(a.block_size), "s"(a.bs_shift));
+    // (read-only for the kernel's lifetime: scalar loads through the constant address space)
+    const int q0 = ((const_int_ptr)(uintptr_t)a.qsl)[b];
+    const int q_end = ((const_int_ptr)(uintptr_t)a.qsl)[b + 1];
+    const int seq_len = ((const_int_ptr)(uintptr_t)a.seq_lens)[b];
+    asm volatile("" ::"s"(q0), "s"(q_end), "s"(seq_len));
+    const int q_len = q_end - q0;
+    if (q_len <= 0 || seq_len <= 0) return;
+    const int R = min(16 * NRB, min(q_len, a.qmax) * a.G - row0);
+    if (R <= 0) return;                          // a slice past the sequence's rows
+    const int lo = a.window > 0 ? max(0, seq_len - q_len - a.window + 1) : 0;
+    const int t_first = lo / kTile;
+    const int ntiles = (seq_len - 1) / kTile - t_first + 1;
+    // Tiles of each wave. Split s owns a contiguous run of tiles [tb, te) and its waves take every
+    // kWaves-th tile of it, unless the block size is a multiple of 16 and there are at least as
+    // many tiles as the W = kWaves * nsplit waves of a (sequence, kv head): then the waves
+    // interleave over all the tiles, wave gw = kWaves * s + w taking tiles t_first + gw + W n, so
+    // that every split has work and the waves' counts differ by at most one. (Fewer tiles than
+    // waves: the contiguous runs measured faster, fewer workgroups with more waves busy.)
+    const int per_split = (ntiles + a.nsplit - 1) / a.nsplit;
+    Work wk;
+    wk.g = g;
+    wk.b = b;
+    wk.row0 = row0;
+    wk.q0 = q0;
+    wk.q_len = q_len;
+    wk.seq_len = seq_len;
+    wk.seg = s;
+    wk.tb = t_first + s * per_split;
+    wk.te = min(t_first + ntiles, wk.tb + per_split);
+    wk.t_first = t_first;
+    wk.ntiles = ntiles;
+    wk.W = kWaves * a.nsplit;
+    wk.interleave = kFast && ntiles >= wk.W;
+    if (wk.interleave ? kWaves * s >= ntiles : wk.tb >= wk.te) {  // no tiles: mark the split empty
+        for (int r = threadIdx.x; r < R; r += kThreads) {
+            const int i = (row0 + r) / a.G, hh = (row0 + r) - i * a.G;
+            const int64_t pr = ((int64_t)(q0 + i) * a.Hq + (g * a.G + hh)) * a.nseg + s;
+            a.part_m[pr] = kNegInf;
+            a.part_l[pr] = 0.f;
+        }
+        return;
+    }
+    partial_body<NRB, kFast>(a, wk, lds);
+}
+
+// ---------------------------------------------------------------------------------------
+// Batches: one launch of a workgroup per CU over every (sequence, kv head), the tiles dealt by the
+// sequence lengths on the device.
+//
+// The items (sequence, kv head) of a batch lie one after the other on a line of total = sum of their
+// tiles. In the even split each workgroup takes `share` consecutive tiles of the line, which may end one item
+// and begin another (a segment each); in the aligned split each item is cut into ns equal pieces, one
+// workgroup each. A fixed split count per sequence, which the host has to choose, leaves the chip
+// waiting for the longest sequence or pays set-up and merge (~10 us) for thousands of pieces of the
+// short ones. 48 sequences of 200 to 16,384 keys, one token each (24 q / 4 kv heads, 370 MB): 250 us at the 64
+// splits that a captured graph gets, 108 us here (this kernel 97, the merge 5.4); it is bound by the page
+// read (3.8 TB/s here; 71 us at the 5.2 TB/s of long streams) and ~1.75 segments' set-up and merge per
+// workgroup. Equal lengths take the aligned split, which has no second segment.
+// Segment s of an item is its s-th workgroup; the last one marks the item's other segments (up to
+// a.nsplit) empty, so the partial buffers mean the same as after pd_partial_kernel.
+constexpr unsigned kSegmentTiles = 12;  // set-up and merge of a segment in tiles of a workgroup (~0.8 us each)
+constexpr unsigned kSnapTiles = 6;      // a share's end this close to an item's boundary moves onto it
+
+__device__ __forceinline__ unsigned wave_add(unsigned v) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += (unsigned)__shfl_xor((int)v, o, 64);
+    return v;
+}
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, o, 64));
+    return v;
+}
+__device__ __forceinline__ unsigned wave_scan(unsigned v, int lane) {  // inclusive
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned u = (unsigned)__shfl_up((int)v, o, 64);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
+template <int NRB, bool kFast>
+__global__ void __launch_bounds__(kThreads, 1) pd_balanced_kernel(const PartialParams a) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[PartialLds<NRB, kFast>::kBytes];
+    asm volatile("" ::"s"(a.qsl), "s"(a.seq_lens), "s"(a.block_table), "s"(a.bt_stride), "s"(a.kc), "s"(a.k_sb),
+                 "s"(a.k_ss), "s"(a.k_sh), "s"(a.q), "s"(a.q_st), "s"(a.qmax), "s"(a.G), "s"(a.window),
+                 "s"(a.nsplit), "s"(a.block_size), "s"(a.bs_shift));
+    const int lane = threadIdx.x & 63;
+    const unsigned Hkv = (unsigned)(a.Hq / a.G), nwg = gridDim.x, wg = blockIdx.x;
+    // tiles that any row of sequence i sees (0 past the batch)
+    auto tiles_of = [&](int i) __attribute__((always_inline)) -> unsigned {
+        const int c = min(i, a.num_seqs - 1);
+        const int q_len = a.qsl[c + 1] - a.qsl[c], len = a.seq_lens[c];
+        const int lo = a.window > 0 ? max(0, len - q_len - a.window + 1) : 0;
+        return i < a.num_seqs && q_len > 0 && len > 0 ? (unsigned)((len - 1) / kTile - lo / kTile + 1) : 0u;
+    };
+    const unsigned t0 = tiles_of(lane), incl0 = wave_scan(t0, lane);  // the first 64 sequences
+    unsigned total = (unsigned)__builtin_amdgcn_readlane((int)incl0, 63), longest = wave_umax(t0);
+    for (int c = 64; c < a.num_seqs; c += 64) {
+        const unsigned t = tiles_of(c + lane);
+        total += wave_add(t);
+        longest = max(longest, wave_umax(t));
+    }
+    total = (unsigned)__builtin_amdgcn_readfirstlane((int)total) * Hkv;
+    longest = (unsigned)__builtin_amdgcn_readfirstlane((int)longest);
+    if (total == 0) return;
+    const unsigned items = (unsigned)a.num_seqs * Hkv, cap = (unsigned)a.nsplit;
+    // an item reaches into at most ceil(tiles / share) + 1 <= cap shares
+    const unsigned share = max(max((total + nwg - 1) / nwg, (longest + cap - 2) / (cap - 1)), 2u);
+    const unsigned ns = min(nwg / items, cap);
+    const bool aligned = ns >= 1 && (longest + ns - 1) / ns <= share + kSegmentTiles;
+    const unsigned snap = min(kSnapTiles, share / 8);
+
+    // the item that holds tile `pos` of the line: sequence, first tile of the sequence, its tiles
+    unsigned at_seq, at_start, at_tiles;
+    auto locate = [&](unsigned pos) __attribute__((always_inline)) {
+        unsigned before = 0;
+        for (int c = 0;; c += 64) {
+            const unsigned t = c == 0 ? t0 : tiles_of(c + lane);
+            const unsigned incl = c == 0 ? incl0 : wave_scan(t, lane);
+            const int k = __popcll(__ballot(Hkv * (before + incl) <= pos));
+            if (k < 64) {
+                at_seq = (unsigned)(c + k);
+                at_tiles = (unsigned)__builtin_amdgcn_readlane((int)t, k);
+                at_start = Hkv * (before + (unsigned)__builtin_amdgcn_readlane((int)(incl - t), k));
+                return;
+            }
+            before += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+        }
+    };
+    // start of share x of the even split
+    auto bound = [&](unsigned x) __attribute__((always_inline)) -> unsigned {
+        const unsigned raw = (unsigned)min((uint64_t)x * share, (uint64_t)total);
+        if (raw == 0 || raw == total) return raw;
+        locate(raw);
+        const unsigned off = (raw - at_start) % at_tiles;
+        if (off <= snap) return raw - off;
+        return at_tiles - off <= snap ? raw + (at_tiles - off) : raw;
+    };
+
+    unsigned pos = 0, end = 0;
+    if (!aligned) {
+        pos = bound(wg);
+        end = bound(wg + 1);
+        if (pos >= end) return;
+    } else if (wg >= items * ns) {
+        return;
+    }
+    while (true) {
+        unsigned first, last, seg;  // tiles [first, last) of the item, and its segment
+        Work wk;
+        if (aligned) {
+            const unsigned item = wg / ns;
+            seg = wg - item * ns;
+            wk.b = (int)(item / Hkv);
+            wk.g = (int)(item - (unsigned)wk.b * Hkv);
+        } else {
+            locate(pos);
+            const unsigned g = (pos - at_start) / at_tiles, item = at_start + g * at_tiles;
+            first = pos - item;
+            last = min(at_tiles, end - item);
+            // the item's first workgroup: the one whose share holds its first tile, or the next if that
+            // one's start has moved onto the item's
+            const unsigned x = item / share, next = (x + 1) * share;
+            seg = wg - (x + (next - item <= snap && next < item + at_tiles ? 1u : 0u));
+            wk.b = (int)at_seq;
+            wk.g = (int)g;
+        }
+        wk.q0 = ((const_int_ptr)(uintptr_t)a.qsl)[wk.b];
+        const int q_end = ((const_int_ptr)(uintptr_t)a.qsl)[wk.b + 1];
+        wk.seq_len = ((const_int_ptr)(uintptr_t)a.seq_lens)[wk.b];
+        asm volatile("" ::"s"(wk.q0), "s"(q_end), "s"(wk.seq_len));
+        wk.q_len = q_end - wk.q0;
+        const int lo = a.window > 0 ? max(0, wk.seq_len - wk.q_len - a.window + 1) : 0;
+        wk.t_first = lo / kTile;
+        wk.ntiles = (wk.seq_len - 1) / kTile - wk.t_first + 1;
+        if (aligned) {
+            if (wk.q_len <= 0 || wk.seq_len <= 0) return;
+            const unsigned per = ((unsigned)wk.ntiles + ns - 1) / ns;
+            first = seg * per;
+            last = min((unsigned)wk.ntiles, first + per);
+            if (first >= last) return;
+        }
+        wk.row0 = 0;
+        wk.seg = (int)seg;
+        wk.tb = wk.t_first + (int)first;
+        wk.te = wk.t_first + (int)last;
+        wk.W = 0;
+        wk.interleave = false;
+        if (last == (unsigned)wk.ntiles) {  // the item's last workgroup: no other segments
+            const int R = min(16 * NRB, min(wk.q_len, a.qmax) * a.G), spare = a.nsplit - 1 - wk.seg;
+            for (int k = threadIdx.x; k < R * spare; k += kThreads) {
+                const int r = k / spare, i = r / a.G, hh = r - i * a.G;
+                a.part_m[((int64_t)(wk.q0 + i) * a.Hq + (wk.g * a.G + hh)) * a.nseg + wk.seg + 1 + (k - r * spare)] = kNegInf;
+            }
+        }
+        partial_body<NRB, kFast>(a, wk, lds);
+        if (aligned) return;
+        pos += last - first;
+        if (pos >= end) return;
+        __syncthreads();  // every wave has read the merge's blocks: the slots can be refilled
+    }
+}
+
 // Cross-row lane exchanges of gfx950 (v_permlane16/32_swap), as asm with both registers read and
 // written. With a = b = x on entry: permlane16: a = rows (0, 0, 2, 2) of x, b = rows (1, 1, 3, 3);
 // permlane32: a = (low, low) halves, b = (high, high). So a op b is x op x^16 (resp. x^32) in
@@ -914,7 +1114,9 @@ __device__ __forceinline__ float group_sum(float v) {
 // kCols: float4 columns per workgroup, 16 (a 64-dim quarter) or 32 (a half row); kPer: splits
 // per lane loaded up front (the first kPer * 64 / (kCols / 4) splits), the smallest power of two
 // that covers nsplit up to 64, so that few splits do not cost loads of clamped duplicates.
-template <int kCols, int kPer>
+// kLive (after pd_balanced_kernel, whose items have few segments each): the partial rows are loaded
+// once the m of the first 64 splits have said which of them hold anything.
+template <int kCols, int kPer, bool kLive>
 __global__ void __launch_bounds__(256) pd_combine_kernel(const CombineParams a) {
     constexpr int kCW = kCols / 4;  // float4 columns per wave
     constexpr int kSG = 64 / kCW;   // lanes sharing a column (segment groups)
@@ -942,13 +1144,15 @@ __global__ void __launch_bounds__(256) pd_combine_kernel(const CombineParams a) 
     const float m_ld = pm[min(lane, ns1)], l_ld = pl[min(lane, ns1)];  // lane s: split s
     float mv[kPer];
     float4_t ov[kPer];
+    if constexpr (!kLive) {
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const int si = min(sg + kSG * i, ns1);
-        const float m = pm[si];
-        const float4_t o = po[(int64_t)si * (kDim / 4)];
-        mv[i] = sg + kSG * i <= ns1 ? m : kNegInf;
-        ov[i] = o;
+        for (int i = 0; i < kPer; ++i) {
+            const int si = min(sg + kSG * i, ns1);
+            const float m = pm[si];
+            const float4_t o = po[(int64_t)si * (kDim / 4)];
+            mv[i] = sg + kSG * i <= ns1 ? m : kNegInf;
+            ov[i] = o;
+        }
     }
 
     const int q_end0 = lane + 1 <= a.num_seqs ? q_end_ld : 0x7fffffff;
@@ -975,12 +1179,30 @@ __global__ void __launch_bounds__(256) pd_combine_kernel(const CombineParams a) 
             const float mp = pm[p];
             if (mp != kNegInf) lw += exp2f(mp - M) * pl[p];
         }
+        if constexpr (kLive) {
+            // (the segments that hold anything are the first few)
+            const int n = 64 - __builtin_clzll(__ballot(m_s != kNegInf) | 1);
+            for (int i = 0; i < n; i += kSG * kPer) {
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const float w = mv[i] != kNegInf ? exp2f(mv[i] - M) : 0.f;
-            acc += w != 0.f ? w * ov[i] : (float4_t)0.f;  // empty splits leave part_o unwritten
+                for (int j = 0; j < kPer; ++j) {
+                    const int si = i + sg + kSG * j;
+                    mv[j] = __shfl(m_s, min(si, 63), 64);
+                    if (si >= n || mv[j] == kNegInf) mv[j] = kNegInf;
+                    ov[j] = (float4_t)0.f;
+                    if (mv[j] != kNegInf) ov[j] = po[(int64_t)si * (kDim / 4)];
+                }
+#pragma unroll
+                for (int j = 0; j < kPer; ++j)
+                    if (mv[j] != kNegInf) acc += exp2f(mv[j] - M) * ov[j];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                const float w = mv[i] != kNegInf ? exp2f(mv[i] - M) : 0.f;
+                acc += w != 0.f ? w * ov[i] : (float4_t)0.f;  // empty splits leave part_o unwritten
+            }
         }
-        for (int p = sg + kSG * kPer; p <= ns1; p += kSG) {
+        for (int p = kLive ? 64 + sg : sg + kSG * kPer; p <= ns1; p += kSG) {
             const float mp = pm[p];
             if (mp != kNegInf) acc += exp2f(mp - M) * po[(int64_t)p * (kDim / 4)];
         }
@@ -1041,7 +1263,28 @@ hipError_t launch_partial_nrb(const PartialParams& p, dim3 grid, hipStream_t str
     return hipGetLastError();
 }
 
-hipError_t launch_partial(const LaunchArgs& x, hipStream_t stream) {
+template <int NRB>
+static hipError_t launch_balanced_nrb(const PartialParams& p, int wgs, hipStream_t stream, bool fast) {
+    if (fast)
+        hipLaunchKernelGGL((pd_balanced_kernel<NRB, true>), dim3(wgs), dim3(kThreads), 0, stream, p);
+    else
+        hipLaunchKernelGGL((pd_balanced_kernel<NRB, false>), dim3(wgs), dim3(kThreads), 0, stream, p);
+    return hipGetLastError();
+}
+
+// Segments per item that a balanced launch may use (0: the batch is not one for it). More than one
+// sequence, since one alone is dealt evenly by pd_partial_kernel; at least two segments for the shares' ends;
+// at most two row blocks (three do not fit the registers beside the line's state); and, with a block table of this width, a line of tiles that 32 bits number.
+static int balanced_segments(const LaunchArgs& x) {
+    const int64_t tiles = ((int64_t)x.bt_stride * x.block_size + kTile - 1) / kTile + 1;
+    if (x.num_seqs < 2 || x.nseg < 2 || x.bt_stride < 1 || x.qmax * (x.heads_q / x.heads_kv) > 32) return 0;
+    if (tiles > INT32_MAX || tiles * x.num_seqs > INT32_MAX / x.heads_kv) return 0;
+    return x.nseg < kMaxBalancedSegments ? x.nseg : kMaxBalancedSegments;
+}
+
+// The partial pass. `balanced` (may be null): allows pd_balanced_kernel, and says how many segments per row it
+// was given (0 if pd_partial_kernel ran instead).
+hipError_t launch_partial(const LaunchArgs& x, hipStream_t stream, int* balanced) {
     PartialParams p;
     p.q = static_cast<const _Float16*>(x.q);
     p.q_st = x.q_st;
@@ -1080,26 +1323,39 @@ hipError_t launch_partial(const LaunchArgs& x, hipStream_t stream) {
                     : 1;
     const dim3 grid(x.nsplit, x.heads_kv, x.num_seqs * p.rslices);
     const bool fast = fast_block_table(x.block_size, x.k_ss);
+    if (balanced) {
+        const int cus = compute_units(stream);
+        *balanced = p.rslices == 1 && cus > 0 ? balanced_segments(x) : 0;
+        if (*balanced) {
+            p.nsplit = *balanced;
+            if (rows <= 16) return launch_balanced_nrb<1>(p, cus, stream, fast);
+            return launch_balanced_nrb<2>(p, cus, stream, fast);
+        }
+    }
     if (rows <= 16 || p.rslices > 1) return launch_partial_nrb<1>(p, grid, stream, fast);
     if (rows <= 32) return launch_partial_nrb<2>(p, grid, stream, fast);
     return launch_partial_nrb<3>(p, grid, stream, fast);
 }
 
 template <int kCols>
-static void launch_combine_cols(const CombineParams& c, dim3 grid, hipStream_t stream) {
-    constexpr int kSG = 64 / (kCols / 4);
+static void launch_combine_cols(const CombineParams& c, dim3 grid, hipStream_t stream, bool live) {
+    constexpr int kSG = 64 / (kCols / 4), kMost = 64 / kSG;  // lanes per column; splits per lane for 64
     const int need = (min(c.nsplit, 64) + kSG - 1) / kSG;  // splits per lane to cover
-    if (need <= 1)
-        hipLaunchKernelGGL((pd_combine_kernel<kCols, 1>), grid, dim3(256), 0, stream, c);
+    const dim3 block(256);
+    if (live)
+        hipLaunchKernelGGL((pd_combine_kernel<kCols, 2, true>), grid, block, 0, stream, c);
+    else if (need <= 1)
+        hipLaunchKernelGGL((pd_combine_kernel<kCols, 1, false>), grid, block, 0, stream, c);
     else if (need <= 2)
-        hipLaunchKernelGGL((pd_combine_kernel<kCols, 2>), grid, dim3(256), 0, stream, c);
-    else if (need <= 4 || 64 / kSG < 8)
-        hipLaunchKernelGGL((pd_combine_kernel<kCols, (64 / kSG < 4 ? 64 / kSG : 4)>), grid, dim3(256), 0, stream, c);
+        hipLaunchKernelGGL((pd_combine_kernel<kCols, 2, false>), grid, block, 0, stream, c);
+    else if (need <= 4 || kMost < 8)
+        hipLaunchKernelGGL((pd_combine_kernel<kCols, (kMost < 4 ? kMost : 4), false>), grid, block, 0, stream, c);
     else
-        hipLaunchKernelGGL((pd_combine_kernel<kCols, (64 / kSG < 8 ? 64 / kSG : 8)>), grid, dim3(256), 0, stream, c);
+        hipLaunchKernelGGL((pd_combine_kernel<kCols, (kMost < 8 ? kMost : 8), false>), grid, block, 0, stream, c);
 }
 
-hipError_t launch_combine(const LaunchArgs& x, hipStream_t stream) {
+// `balanced`: the segments per row of a balanced partial pass, 0 after pd_partial_kernel.
+hipError_t launch_combine(const LaunchArgs& x, hipStream_t stream, int balanced) {
     CombineParams c;
     c.part_o = x.part_o;
     c.part_m = x.part_m;
@@ -1111,25 +1367,29 @@ hipError_t launch_combine(const LaunchArgs& x, hipStream_t stream) {
     c.o_sh = x.o_sh;
     c.num_seqs = x.num_seqs;
     c.nseg = x.nseg;
-    c.nsplit = x.nsplit;
+    c.nsplit = balanced ? balanced : x.nsplit;
     c.qmax = x.qmax;
     // Few rows: a quarter row per workgroup for parallelism; many rows: half rows, fewer
     // workgroups (4 windowed sequences x 8 tokens x 24 heads, 768 rows: 31.3 -> 29.7 us per layer;
     // 24 rows: 12.2 against 12.6).
     if ((int64_t)x.num_tokens * x.heads_q <= 256)
-        launch_combine_cols<16>(c, dim3(x.num_tokens, x.heads_q, 4), stream);
+        launch_combine_cols<16>(c, dim3(x.num_tokens, x.heads_q, 4), stream, balanced != 0);
     else
-        launch_combine_cols<32>(c, dim3(x.num_tokens, x.heads_q, 2), stream);
+        launch_combine_cols<32>(c, dim3(x.num_tokens, x.heads_q, 2), stream, balanced != 0);
     return hipGetLastError();
 }
 
+hipError_t launch_both(const LaunchArgs& x, hipStream_t stream) {
+    int balanced = 0;
+    const hipError_t e = launch_partial(x, stream, &balanced);
+    if (e != hipSuccess) return e;
+    return launch_combine(x, stream, balanced);
+}
+
 hipError_t launch_all(const LaunchArgs& x, hipStream_t stream, bool strict) {
-    hipError_t e = check_args(x, strict);
+    const hipError_t e = check_args(x, strict);
     if (e != hipSuccess) return e;
-    if (x.num_tokens == 0) return hipSuccess;
-    e = launch_partial(x, stream);
-    if (e != hipSuccess) return e;
-    return launch_combine(x, stream);
+    return x.num_tokens == 0 ? hipSuccess : launch_both(x, stream);
 }
 
 // Partials of pth_dec_launch_noalloc: part_o [T, Hq, nsplit, 256], then part_m and part_l

@@ -127,8 +127,9 @@ inline bool fast_block_table(int bs, int64_t k_ss) { return bs % 16 == 0 && k_ss
 
 // decode (pd_decode.hip)
 hipError_t check_args(const LaunchArgs& x, bool strict_reference);
-hipError_t launch_partial(const LaunchArgs& x, hipStream_t stream);
-hipError_t launch_combine(const LaunchArgs& x, hipStream_t stream);
+hipError_t launch_partial(const LaunchArgs& x, hipStream_t stream, int* balanced = nullptr);
+hipError_t launch_combine(const LaunchArgs& x, hipStream_t stream, int balanced = 0);
+hipError_t launch_both(const LaunchArgs& x, hipStream_t stream);
 hipError_t launch_all(const LaunchArgs& x, hipStream_t stream, bool strict);
 // the device array behind pth_dec_launch_noalloc, and its address on the current device
 constexpr size_t kScratchBytes = size_t(32) << 20;
