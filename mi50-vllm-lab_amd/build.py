@@ -2,19 +2,22 @@
 
     python mi50-vllm-lab_amd/build.py [--save-temps DIR]
 
-The library is the C ABI declared in include/pth_dec.h. It is always rebuilt: hipcc takes
-about half a minute and a stale library is worse than a slow build.
+The library is the C ABI declared in include/pth_dec.h. Beside it pd_native.so, the Python extension
+through which pth_dec.py calls it on torch tensors (host code only, torch's headers). Both are
+always rebuilt: hipcc takes about half a minute and a stale library is worse than a slow build.
 """
 import argparse
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libpthdec.so")
+NATIVE_PATH = os.path.join(LIB_DIR, "pd_native.so")
 # the C ABI, then the kernels (each file compiles on its own; they share csrc/pd_*.hpp)
 SOURCES = [os.path.join(HERE, "csrc", f) for f in
            ("pd_api.hip", "pd_decode.hip", "pd_prefill.hip", "pd_cache_write.hip")]
@@ -57,9 +60,32 @@ def build(save_temps: str | None = None, verbose: bool = False) -> str:
     return LIB_PATH
 
 
+def build_native() -> str:
+    """pd_native.so: pd_python.cpp against the installed torch's headers and libraries."""
+    from torch.utils import cpp_extension
+
+    os.makedirs(LIB_DIR, exist_ok=True)
+    tmp = NATIVE_PATH + ".tmp"
+    rocm = os.path.dirname(os.path.dirname(hipcc()))
+    includes = [os.path.join(ROOT, "include"), sysconfig.get_paths()["include"], os.path.join(rocm, "include"),
+                *cpp_extension.include_paths()]
+    libs = cpp_extension.library_paths()
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", *[x for i in includes for x in ("-isystem", i)],
+           os.path.join(HERE, "csrc", "pd_python.cpp"), "-o", tmp, *[x for p in libs for x in ("-L" + p,)],
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        sys.stderr.write(res.stdout + res.stderr)
+        raise RuntimeError(f"g++ failed ({res.returncode}) building {NATIVE_PATH}")
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 if __name__ == "__main__":
     ap = argparse.ArgumentParser()
     ap.add_argument("--save-temps", default=None, help="directory for hipcc -save-temps output")
     ap.add_argument("-v", "--verbose", action="store_true")
     args = ap.parse_args()
     print(build(args.save_temps, args.verbose))
+    print(build_native())

@@ -1,0 +1,306 @@
+// pd_native: the Python face of libpthdec.so's operator calls (pth_dec.py, vllm_shim.py) in C++. A call
+// fills the pd_tensor descriptors from its torch tensors, takes torch's current stream and calls
+// the C entry whose address it is given; the entry does every check and reports its message.
+// In Python with ctypes that work took 20-30 us per call, and the split plans, which are evaluated on every
+// call too, 50-100 us: more than a decode layer of one user takes on the GPU. One eager layer step
+// (cache write, routing, decode; 4,096 keys) 116 -> 19 us, a 16-token cache write 18.6 -> 3.7.
+//
+// The module holds no state: the library that is active is pth_dec.load_library()'s business.
+#include <Python.h>
+
+#include <algorithm>
+#include <cmath>
+#include <exception>
+
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "pth_dec.h"
+
+namespace {
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kChar: return PD_DTYPE_INT8;
+        case at::kHalf: return PD_DTYPE_FP16;
+        case at::kFloat: return PD_DTYPE_FP32;
+        case at::kInt: return PD_DTYPE_INT32;
+        case at::kBFloat16: return PD_DTYPE_BF16;
+        case at::kLong: return PD_DTYPE_INT64;
+        default: return 0;
+    }
+}
+
+// Descriptor of a tensor argument; false with a Python error set.
+bool describe(PyObject* o, pd_tensor& d) {
+    if (!THPVariable_Check(o)) {
+        PyErr_Format(PyExc_TypeError, "expected a tensor, got %s", Py_TYPE(o)->tp_name);
+        return false;
+    }
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (t.dim() > PD_MAX_DIMS) {
+        PyErr_Format(PyExc_RuntimeError, "tensor rank %lld exceeds %d", (long long)t.dim(), PD_MAX_DIMS);
+        return false;
+    }
+    d = pd_tensor{};
+    d.data = t.data_ptr();
+    d.dtype = dtype_code(t.scalar_type());
+    d.ndim = (int)t.dim();
+    for (int i = 0; i < d.ndim; ++i) {
+        d.sizes[i] = t.size(i);
+        d.strides[i] = t.stride(i);
+    }
+    return true;
+}
+
+bool describe_all(PyObject* const* o, pd_tensor* d, int n) {
+    for (int i = 0; i < n; ++i)
+        if (!describe(o[i], d[i])) return false;
+    return true;
+}
+
+// torch's current stream on a tensor's device, with that device current while this object lives.
+class OnDevice {
+public:
+    explicit OnDevice(PyObject* o) {
+        const c10::Device dev = THPVariable_Unpack(o).device();
+        if (!dev.is_cuda()) return;  // the entry gets no further than its checks
+        before_ = c10::hip::current_device();
+        const c10::DeviceIndex index = dev.has_index() ? dev.index() : before_;
+        if (index != before_) c10::hip::set_device(index);
+        now_ = index;
+        stream = c10::hip::getCurrentHIPStream(index).stream();
+    }
+    ~OnDevice() {
+        try {
+            if (now_ != before_) c10::hip::set_device(before_);
+        } catch (...) {  // the call itself has already been made
+        }
+    }
+    OnDevice(const OnDevice&) = delete;
+    hipStream_t stream = nullptr;
+
+private:
+    c10::DeviceIndex before_ = -1, now_ = -1;
+};
+
+bool as_int64(PyObject* o, int64_t& v) {
+    v = PyLong_AsLongLong(o);
+    return !(v == -1 && PyErr_Occurred());
+}
+bool as_double(PyObject* o, double& v) {
+    v = PyFloat_AsDouble(o);
+    return !(v == -1.0 && PyErr_Occurred());
+}
+template <class F>
+bool entry(PyObject* o, F& f) {
+    f = reinterpret_cast<F>(PyLong_AsVoidPtr(o));
+    return f != nullptr || (PyErr_Occurred() ? false : (PyErr_SetString(PyExc_ValueError, "null entry point"), false));
+}
+bool count_is(Py_ssize_t n, Py_ssize_t want) {
+    if (n == want) return true;
+    PyErr_Format(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
+    return false;
+}
+PyObject* done(int rc, const char* err) {
+    if (rc == 0) Py_RETURN_NONE;
+    PyErr_SetString(PyExc_RuntimeError, err);
+    return nullptr;
+}
+// No C++ exception crosses into Python (torch's accessors throw for tensors without storage).
+template <class F>
+PyObject* guarded(F&& f) {
+    try {
+        return f();
+    } catch (const c10::Error& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+
+// decode(entry, q, key_cache, value_cache, k_scale, v_scale, block_table, seq_lens, query_start_loc, out, scale,
+//        part_o, part_m, part_l, num_seqs, qmax, nsplit, window, causal)
+PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        decltype(&pth_dec_decode) fn;
+        pd_tensor t[9], p[3];
+        double scale;
+        int64_t v[5];
+        if (!count_is(n, 19) || !entry(a[0], fn) || !describe_all(a + 1, t, 9) || !as_double(a[10], scale) ||
+            !describe_all(a + 11, p, 3))
+            return nullptr;
+        for (int i = 0; i < 5; ++i)
+            if (!as_int64(a[14 + i], v[i])) return nullptr;
+        char err[256] = "";
+        OnDevice dev(a[1]);
+        int rc;
+        Py_BEGIN_ALLOW_THREADS;
+        rc = fn(&t[0], &t[1], &t[2], &t[3], &t[4], &t[5], &t[6], &t[7], &t[8], scale, &p[0], &p[1], &p[2], v[0], v[1],
+                v[2], v[3], v[4], dev.stream, err, (int)sizeof err);
+        Py_END_ALLOW_THREADS;
+        return done(rc, err);
+    });
+}
+
+// prefill(entry, q, key_cache, value_cache, block_table, seq_lens, scale, q_abs_offset, out)
+PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        decltype(&pth_fa_forward) fn;
+        pd_tensor t[5], p[2];
+        double scale;
+        if (!count_is(n, 9) || !entry(a[0], fn) || !describe_all(a + 1, t, 5) || !as_double(a[6], scale) ||
+            !describe_all(a + 7, p, 2))
+            return nullptr;
+        char err[256] = "";
+        OnDevice dev(a[1]);
+        int rc;
+        Py_BEGIN_ALLOW_THREADS;
+        rc = fn(&t[0], &t[1], &t[2], &t[3], &t[4], scale, &p[0], &p[1], dev.stream, err, (int)sizeof err);
+        Py_END_ALLOW_THREADS;
+        return done(rc, err);
+    });
+}
+
+// prefill_split(entry, q, key_cache, value_cache, block_table, seq_lens, scale, q_abs_offset, out, workspace, nsplit, exact)
+PyObject* prefill_split(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        decltype(&pth_fa_forward_split) fn;
+        pd_tensor t[5], p[3];
+        double scale;
+        int64_t nsplit, exact;
+        if (!count_is(n, 12) || !entry(a[0], fn) || !describe_all(a + 1, t, 5) || !as_double(a[6], scale) ||
+            !describe_all(a + 7, p, 3) || !as_int64(a[10], nsplit) || !as_int64(a[11], exact))
+            return nullptr;
+        char err[256] = "";
+        OnDevice dev(a[1]);
+        int rc;
+        Py_BEGIN_ALLOW_THREADS;
+        rc = fn(&t[0], &t[1], &t[2], &t[3], &t[4], scale, &p[0], &p[1], &p[2], nsplit, exact, dev.stream, err,
+                (int)sizeof err);
+        Py_END_ALLOW_THREADS;
+        return done(rc, err);
+    });
+}
+
+// cache_write(entry, key, value, key_cache, value_cache, k_scale, v_scale, slot_mapping)
+PyObject* cache_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        decltype(&pth_cache_write) fn;
+        pd_tensor t[7];
+        if (!count_is(n, 8) || !entry(a[0], fn) || !describe_all(a + 1, t, 7)) return nullptr;
+        char err[256] = "";
+        OnDevice dev(a[1]);
+        int rc;
+        Py_BEGIN_ALLOW_THREADS;
+        rc = fn(&t[0], &t[1], &t[2], &t[3], &t[4], &t[5], &t[6], dev.stream, err, (int)sizeof err);
+        Py_END_ALLOW_THREADS;
+        return done(rc, err);
+    });
+}
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// plan_decode(lens, num_seqs, num_kv_heads, rows, max_q, window, cap, cus, tile_us, fixed_us, empty_us, merge_us_per_mb,
+//             row_bytes): vllm_shim.decode_splits' makespan model; lens is a contiguous int32 or int64 CPU tensor.
+PyObject* plan_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        int64_t num_seqs, hkv, rows, max_q, window, cap, cus;
+        double tile_us, fixed_us, empty_us, merge_us, row_bytes;
+        if (!count_is(n, 13) || !as_int64(a[1], num_seqs) || !as_int64(a[2], hkv) || !as_int64(a[3], rows) ||
+            !as_int64(a[4], max_q) || !as_int64(a[5], window) || !as_int64(a[6], cap) || !as_int64(a[7], cus) ||
+            !as_double(a[8], tile_us) || !as_double(a[9], fixed_us) || !as_double(a[10], empty_us) ||
+            !as_double(a[11], merge_us) || !as_double(a[12], row_bytes))
+            return nullptr;
+        if (!THPVariable_Check(a[0])) {
+            PyErr_SetString(PyExc_TypeError, "lens must be a tensor");
+            return nullptr;
+        }
+        const at::Tensor& lens = THPVariable_Unpack(a[0]);
+        const bool wide = lens.scalar_type() == at::kLong;
+        if (!lens.device().is_cpu() || !lens.is_contiguous() || (!wide && lens.scalar_type() != at::kInt)) {
+            PyErr_SetString(PyExc_ValueError, "lens must be a contiguous int32 or int64 CPU tensor");
+            return nullptr;
+        }
+        const void* data = lens.const_data_ptr();
+        const int64_t count = std::min<int64_t>(lens.numel(), num_seqs);
+        // visible keys in 32-key tiles (+ 1: alignment)
+        auto tiles_of = [&](int64_t i) -> int64_t {
+            int64_t len = wide ? static_cast<const int64_t*>(data)[i] : static_cast<const int32_t*>(data)[i];
+            if (window > 0) len = std::min(len, window + max_q);
+            return len > 0 ? ceil_div(len, 32) + 1 : 0;
+        };
+        bool live = false;
+        for (int64_t i = 0; i < count; ++i) live = live || tiles_of(i) > 0;
+        if (!live) return PyLong_FromLong(1);
+        int64_t best_s = cap;
+        double best_t = HUGE_VAL;
+        for (int64_t s = 1;; s = s * 2 < cap ? s * 2 : cap) {  // powers of two, and the cap
+            double total = 0.0, longest = 0.0;
+            for (int64_t i = 0; i < count; ++i) {
+                const int64_t t = tiles_of(i), per = std::max<int64_t>(ceil_div(t, s), 1);
+                const int64_t filled = t > 0 ? ceil_div(t, per) : 0;  // splits holding tiles
+                const double us = fixed_us + tile_us * (double)ceil_div(per, 4);
+                total += (double)filled * us + (double)(s - filled) * empty_us;
+                if (t > 0) longest = std::max(longest, us);
+            }
+            const double span = std::max((double)hkv * total / (double)cus, longest) +
+                                merge_us * (double)rows * (double)s * row_bytes / 1e6;
+            if (span < best_t - 1e-9) best_s = s, best_t = span;
+            if (s >= cap) break;
+        }
+        return PyLong_FromLongLong(best_s);
+    });
+}
+
+// plan_prefill(work_items, rows, max_keys, block_size, cus, tile_us, wg_us, mb_us, merge_us, max_splits, min_tiles,
+//              max_workspace, lds_table, global_factor): pth_dec.prefill_splits' makespan model.
+PyObject* plan_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        int64_t v[5], max_splits, min_tiles, max_workspace, lds_table;
+        double tile_us, wg_us, mb_us, merge_us, factor;
+        if (!count_is(n, 14)) return nullptr;
+        for (int i = 0; i < 5; ++i)
+            if (!as_int64(a[i], v[i])) return nullptr;
+        if (!as_double(a[5], tile_us) || !as_double(a[6], wg_us) || !as_double(a[7], mb_us) || !as_double(a[8], merge_us) ||
+            !as_int64(a[9], max_splits) || !as_int64(a[10], min_tiles) || !as_int64(a[11], max_workspace) ||
+            !as_int64(a[12], lds_table) || !as_double(a[13], factor))
+            return nullptr;
+        const int64_t items = v[0], rows = v[1], keys = std::max<int64_t>(0, v[2]), bs = std::max<int64_t>(1, v[3]), cus = v[4];
+        const int64_t tiles = ceil_div(keys, 32);
+        auto cost = [&](int64_t s) {
+            const int64_t rounds = ceil_div(items * s, cus), per = ceil_div(tiles, s);
+            const bool in_lds = v[3] % 16 == 0 ? 2 * per <= lds_table : ceil_div(keys, bs) <= lds_table;
+            double t = (double)rounds * ((double)per * (tile_us * (in_lds ? 1.0 : factor)) + wg_us);
+            if (s > 1) t += merge_us + mb_us * (double)rows * (double)s * 1032 / 1e6;
+            return t;
+        };
+        int64_t best = 1;
+        double best_t = cost(1);
+        const int64_t top = std::max<int64_t>(1, std::min(max_splits, tiles / min_tiles));
+        for (int64_t s = 2; s <= top && rows * s * 1032 <= max_workspace; ++s) {
+            const double t = cost(s);
+            if (t < best_t) best = s, best_t = t;
+        }
+        return PyLong_FromLongLong(best);
+    });
+}
+
+#define PD_METHOD(f, doc) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, doc}
+PyMethodDef methods[] = {
+    PD_METHOD(decode, "pth_dec_decode on torch tensors"),
+    PD_METHOD(prefill, "pth_fa_forward / pth_fa_forward_exact on torch tensors"),
+    PD_METHOD(prefill_split, "pth_fa_forward_split on torch tensors"),
+    PD_METHOD(cache_write, "pth_cache_write on torch tensors"),
+    PD_METHOD(plan_decode, "split count of a decode batch"),
+    PD_METHOD(plan_prefill, "key splits of a prefill launch"),
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "pd_native", "operator calls of libpthdec.so on torch tensors", -1, methods,
+                      nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_pd_native() { return PyModule_Create(&module); }

@@ -8,12 +8,15 @@ nothing and launches on torch's current stream, so it is safe inside HIP-graph c
 non-causal sliding-window rows, patches/vllm/gfx906_fa_paged.patch:7-20).
 
 Tensors cross the C ABI as `pd_tensor` descriptors (data pointer, dtype code, sizes, strides);
-no torch type appears in the ABI. The library has no CPU fallback: if it is not built, every
-entry point raises.
+no torch type appears in the ABI. The operator calls go through pd_native (csrc/pd_python.cpp), which
+fills the descriptors and calls the loaded library's entries. Neither has a CPU fallback: if one is
+not built, every entry point raises.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -67,6 +70,22 @@ class PdTensor(ctypes.Structure):
 
 _lib = None
 _lib_path = None
+_entries = {}  # addresses of the loaded library's operator entries
+_native = None
+
+
+def native():
+    """The pd_native extension module, loaded on first use; raises if it is not built."""
+    global _native
+    if _native is None:
+        path = os.path.join(_HERE, "lib", "pd_native.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"pd_native.so not found at {path}; build it with mi50-vllm-lab_amd/build.py")
+        loader = importlib.machinery.ExtensionFileLoader("pd_native", path)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("pd_native", loader))
+        loader.exec_module(mod)
+        _native = mod
+    return _native
 
 
 def load_library(path: str | None = None) -> ctypes.CDLL:
@@ -116,8 +135,18 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
     lib.pth_cache_write.restype = c_int
     lib.pth_dec_version.argtypes = []
     lib.pth_dec_version.restype = ctypes.c_char_p
+    _entries.update({name: ctypes.cast(getattr(lib, name), vp).value
+                     for name in ("pth_dec_decode", "pth_fa_forward", "pth_fa_forward_exact", "pth_fa_forward_split",
+                                  "pth_cache_write")})
     _lib, _lib_path = lib, os.path.realpath(p)
     return lib
+
+
+def _entry(name: str) -> int:
+    """Address of an operator entry of the active library (loaded if none is)."""
+    if _lib is None:
+        load_library()
+    return _entries[name]
 
 
 def describe(t: torch.Tensor) -> PdTensor:
@@ -159,18 +188,9 @@ def decode(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, 
     """
     if not q.is_cuda:
         raise RuntimeError("q must be fp16 [T, Hq, 256] with contiguous heads")
-    lib = load_library()
-    tensors = (q, key_cache, value_cache, k_scale, v_scale, block_table, seq_lens, query_start_loc, out)
-    descs = [describe(t) for t in tensors]
-    pdescs = [describe(t) for t in (part_o, part_m, part_l)]
-    err = ctypes.create_string_buffer(256)
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        rc = lib.pth_dec_decode(*[ctypes.byref(x) for x in descs], float(scale),
-                                *[ctypes.byref(x) for x in pdescs], int(num_seqs), int(qmax), int(nsplit),
-                                int(window), 1 if causal else 0, ctypes.c_void_p(stream), err, len(err))
-    if rc != 0:
-        raise RuntimeError(err.value.decode())
+    native().decode(_entry("pth_dec_decode"), q, key_cache, value_cache, k_scale, v_scale, block_table, seq_lens,
+                    query_start_loc, out, scale, part_o, part_m, part_l, int(num_seqs), int(qmax), int(nsplit),
+                    int(window), 1 if causal else 0)
 
 
 PREFILL_ROWS_PER_WORKGROUP = 192  # query rows (tokens x heads of one kv head) per prefill workgroup
@@ -226,16 +246,12 @@ def prefill_splits(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: i
     the keys a row can see; the device splits each row's actual keys evenly."""
     if batch <= 0 or sq <= 0 or heads_q <= 0 or heads_kv <= 0:
         return 1
-    tiles = -(-max(0, max_keys) // 32)
-    top = max(1, min(PREFILL_MAX_SPLITS, tiles // PREFILL_MIN_TILES_PER_SPLIT))
-    best, best_t = 1, prefill_cost_us(batch, sq, heads_q, heads_kv, max_keys, 1, block_size)
-    for ns in range(2, top + 1):
-        if batch * sq * heads_q * ns * 1032 > PREFILL_MAX_WORKSPACE:
-            break
-        t = prefill_cost_us(batch, sq, heads_q, heads_kv, max_keys, ns, block_size)
-        if t < best_t:
-            best, best_t = ns, t
-    return best
+    g = max(1, heads_q // heads_kv)
+    qtiles = -(-sq // max(1, PREFILL_ROWS_PER_WORKGROUP // g))
+    return native().plan_prefill(qtiles * heads_kv * batch, batch * sq * heads_q, max_keys, block_size, PREFILL_CUS,
+                                 PREFILL_US_PER_TILE, PREFILL_US_PER_WORKGROUP, PREFILL_US_PER_PARTIAL_MB,
+                                 PREFILL_US_MERGE_LAUNCH, PREFILL_MAX_SPLITS, PREFILL_MIN_TILES_PER_SPLIT,
+                                 PREFILL_MAX_WORKSPACE, PREFILL_LDS_TABLE, PREFILL_GLOBAL_TABLE_FACTOR)
 
 
 def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, block_table: torch.Tensor,
@@ -259,32 +275,21 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
     """
     if not q.is_cuda:
         raise RuntimeError("q must be contiguous fp32 [B, Hq, Sq, D]")
-    lib = load_library()
     if out is None:
         out = torch.empty((q.shape[0], q.shape[2], q.shape[1], q.shape[3]), dtype=torch.float32, device=q.device)
-    descs = [describe(t) for t in (q, key_cache, value_cache, block_table, seq_lens)]
-    qa, od = describe(q_abs_offset), describe(out)
-    err = ctypes.create_string_buffer(256)
     if nsplit is None:
         if max_keys is None:
             max_keys = block_table.shape[1] * key_cache.shape[1] if block_table.dim() == 2 else 0
         nsplit = prefill_splits(q.shape[0], q.shape[2], q.shape[1], key_cache.shape[2], int(max_keys),
                                 key_cache.shape[1] if key_cache.dim() == 4 else 16)
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        if nsplit > 1:
-            ws = torch.empty((q.shape[0] * q.shape[2] * q.shape[1] * nsplit * (q.shape[3] + 2),), dtype=torch.float32,
-                             device=q.device)
-            wd = describe(ws)
-            rc = lib.pth_fa_forward_split(*[ctypes.byref(x) for x in descs], float(scale), ctypes.byref(qa),
-                                          ctypes.byref(od), ctypes.byref(wd), nsplit, 1 if exact else 0,
-                                          ctypes.c_void_p(stream), err, len(err))
-        else:
-            fn = lib.pth_fa_forward_exact if exact else lib.pth_fa_forward
-            rc = fn(*[ctypes.byref(x) for x in descs], float(scale), ctypes.byref(qa), ctypes.byref(od),
-                    ctypes.c_void_p(stream), err, len(err))
-    if rc != 0:
-        raise RuntimeError(err.value.decode())
+    if nsplit > 1:
+        ws = torch.empty((q.shape[0] * q.shape[2] * q.shape[1] * nsplit * (q.shape[3] + 2),), dtype=torch.float32,
+                         device=q.device)
+        native().prefill_split(_entry("pth_fa_forward_split"), q, key_cache, value_cache, block_table, seq_lens, scale,
+                               q_abs_offset, out, ws, int(nsplit), 1 if exact else 0)
+    else:
+        native().prefill(_entry("pth_fa_forward_exact" if exact else "pth_fa_forward"), q, key_cache, value_cache,
+                         block_table, seq_lens, scale, q_abs_offset, out)
     return out
 
 
@@ -298,14 +303,7 @@ def cache_write(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor,
     """
     if not key.is_cuda:
         raise RuntimeError("key and value must be fp16, bf16 or fp32 of the same dtype")
-    lib = load_library()
-    descs = [describe(t) for t in (key, value, key_cache, value_cache, k_scale, v_scale, slot_mapping)]
-    err = ctypes.create_string_buffer(256)
-    with torch.cuda.device(key.device):
-        stream = torch.cuda.current_stream(key.device).cuda_stream
-        rc = lib.pth_cache_write(*[ctypes.byref(x) for x in descs], ctypes.c_void_p(stream), err, len(err))
-    if rc != 0:
-        raise RuntimeError(err.value.decode())
+    native().cache_write(_entry("pth_cache_write"), key, value, key_cache, value_cache, k_scale, v_scale, slot_mapping)
 
 
 def _ptr(t: torch.Tensor, ctype):

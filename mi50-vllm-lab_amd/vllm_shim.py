@@ -31,7 +31,6 @@ few fields the routing reads.
 from __future__ import annotations
 
 import logging
-import math
 import os
 from dataclasses import dataclass
 from typing import Any, Callable, Optional
@@ -128,26 +127,13 @@ def decode_splits(nseg: int, window: int, num_kv_heads: int, num_seqs: int, devi
         if window > 0:
             return max(1, min(cap, cus // max(1, num_kv_heads * num_seqs)))
         return cap
-    lens = np.asarray(seq_lens_host, dtype=np.int64).reshape(-1)[:num_seqs]
-    if window > 0:
-        lens = np.minimum(lens, window + max_q)
-    tiles = (lens + 31) // 32 + (lens > 0)  # visible keys in 32-key tiles (+1: alignment)
-    live = tiles > 0
-    if not live.any():
-        return 1
+    lens = seq_lens_host
+    if not (isinstance(lens, torch.Tensor) and lens.dtype in (torch.int32, torch.int64) and lens.device.type == "cpu"
+            and lens.is_contiguous()):
+        lens = torch.from_numpy(np.array(seq_lens_host, dtype=np.int64).reshape(-1))
     rows = num_seqs * max(1, max_q) * (num_q_heads if num_q_heads else 6 * num_kv_heads)
-    cands = sorted({1 << k for k in range(int(math.log2(cap)) + 1)} | {cap})
-    best_s, best_t = cap, float("inf")
-    for s in cands:
-        per = np.maximum(-(-tiles // s), 1)              # tiles per split
-        n = np.where(live, -(-tiles // per), 0)         # splits holding tiles
-        t = SPLIT_FIXED_US + SPLIT_TILE_US * -(-per // 4)
-        total = num_kv_heads * float(np.sum(n * t + (s - n) * SPLIT_EMPTY_US))
-        span = max(total / cus, float(t[live].max()))
-        span += COMBINE_US_PER_MB * rows * s * PARTIAL_ROW_BYTES / 1e6
-        if span < best_t - 1e-9:
-            best_s, best_t = s, span
-    return best_s
+    return _pd.native().plan_decode(lens, num_seqs, num_kv_heads, rows, max_q, window, cap, cus, SPLIT_TILE_US,
+                                    SPLIT_FIXED_US, SPLIT_EMPTY_US, COMBINE_US_PER_MB, PARTIAL_ROW_BYTES)
 
 
 def _capturing(device) -> bool:
