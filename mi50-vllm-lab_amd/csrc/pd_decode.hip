@@ -888,37 +888,47 @@ __global__ void __launch_bounds__(kThreads, 1) pd_partial_kernel(const PartialPa
 // Batches: one launch of a workgroup per CU over every (sequence, kv head), the tiles dealt by the
 // sequence lengths on the device.
 //
-// The items (sequence, kv head) of a batch lie one after the other on a line of total = sum of their
-// tiles. In the even split each workgroup takes `share` consecutive tiles of the line, which may end one item
-// and begin another (a segment each); in the aligned split each item is cut into ns equal pieces, one
-// workgroup each. A fixed split count per sequence, which the host has to choose, leaves the chip
+// The items (sequence, kv head) of a batch lie one after the other on a line, each as long as its tiles and
+// the set-up and merge of a segment (kSegmentUnits tiles' time). In the even split each workgroup takes `share`
+// consecutive units of the line, which may end one item and begin others (a segment each); in the
+// aligned split each item is cut into ns equal pieces, one workgroup each. A fixed split count per sequence, which the host has to choose, leaves the chip
 // waiting for the longest sequence or pays set-up and merge (~10 us) for thousands of pieces of the
-// short ones. 48 sequences of 200 to 16,384 keys, one token each (24 q / 4 kv heads, 370 MB): 250 us at the 64
-// splits that a captured graph gets, 108 us here (this kernel 97, the merge 5.4); it is bound by the page
-// read (3.8 TB/s here; 71 us at the 5.2 TB/s of long streams) and ~1.75 segments' set-up and merge per
-// workgroup. Equal lengths take the aligned split, which has no second segment.
+// short ones. Measured per layer (24 q / 4 kv heads, one token each): 48 sequences of 200 to 16,384 keys
+// 254 us at the 64 splits that a captured graph gets, 115 at the 4 that the host plans with the
+// lengths, 85 here (4.3 TB/s; the page read alone 71 us at the 5.2 TB/s of long streams); without the segments'
+// cost in the line 113, since the workgroups of the shortest sequences then took up to a dozen
+// segments. 120,000 + 7 x 2,048 keys (4 tokens): 119 / 90.7 / 70.3 us. Equal lengths take the aligned split, which
+// has no second segment (16 x 8,192 keys, 4 tokens: 192 / 68.4 / 65.9).
 // Segment s of an item is its s-th workgroup; the last one marks the item's other segments (up to
 // a.nsplit) empty, so the partial buffers mean the same as after pd_partial_kernel.
-constexpr unsigned kSegmentTiles = 12;  // set-up and merge of a segment in tiles of a workgroup (~0.8 us each)
+constexpr unsigned kSegmentUnits = 12;  // set-up and merge of a segment, ~10 us, in tiles of a workgroup (~0.8 us each)
 constexpr unsigned kSnapTiles = 6;      // a share's end this close to an item's boundary moves onto it
 
-__device__ __forceinline__ unsigned wave_add(unsigned v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += (unsigned)__shfl_xor((int)v, o, 64);
+// DPP move with 0 in lanes that have no source (kRows: the 16-lane rows that take part).
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ unsigned dpp_or_zero(unsigned v) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xf, false);
+}
+// Inclusive sum over the lanes: shifts inside 16-lane rows, then the last lane of row 0 into row 1 and of row
+// 2 into row 3, then the last lane of the lower half into the upper.
+__device__ __forceinline__ unsigned wave_scan(unsigned v) {
+    v += dpp_or_zero<0x111>(v);       // row_shr:1
+    v += dpp_or_zero<0x112>(v);       // row_shr:2
+    v += dpp_or_zero<0x114>(v);       // row_shr:4
+    v += dpp_or_zero<0x118>(v);       // row_shr:8
+    v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15
+    v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31
     return v;
 }
+// Largest value of the wave, uniform (the same steps; the last lane has seen every other).
 __device__ __forceinline__ unsigned wave_umax(unsigned v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, o, 64));
-    return v;
-}
-__device__ __forceinline__ unsigned wave_scan(unsigned v, int lane) {  // inclusive
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const unsigned u = (unsigned)__shfl_up((int)v, o, 64);
-        if (lane >= o) v += u;
-    }
-    return v;
+    v = max(v, dpp_or_zero<0x111>(v));
+    v = max(v, dpp_or_zero<0x112>(v));
+    v = max(v, dpp_or_zero<0x114>(v));
+    v = max(v, dpp_or_zero<0x118>(v));
+    v = max(v, dpp_or_zero<0x142, 0xa>(v));
+    v = max(v, dpp_or_zero<0x143, 0xc>(v));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 template <int NRB, bool kFast>
@@ -936,48 +946,48 @@ __global__ void __launch_bounds__(kThreads, 1) pd_balanced_kernel(const PartialP
         const int lo = a.window > 0 ? max(0, len - q_len - a.window + 1) : 0;
         return i < a.num_seqs && q_len > 0 && len > 0 ? (unsigned)((len - 1) / kTile - lo / kTile + 1) : 0u;
     };
-    const unsigned t0 = tiles_of(lane), incl0 = wave_scan(t0, lane);  // the first 64 sequences
+    auto units_of = [&](unsigned t) __attribute__((always_inline)) { return t ? t + kSegmentUnits : 0u; };
+    const unsigned t0 = tiles_of(lane), incl0 = wave_scan(units_of(t0));  // the first 64 sequences
     unsigned total = (unsigned)__builtin_amdgcn_readlane((int)incl0, 63), longest = wave_umax(t0);
     for (int c = 64; c < a.num_seqs; c += 64) {
         const unsigned t = tiles_of(c + lane);
-        total += wave_add(t);
+        total += (unsigned)__builtin_amdgcn_readlane((int)wave_scan(units_of(t)), 63);
         longest = max(longest, wave_umax(t));
     }
-    total = (unsigned)__builtin_amdgcn_readfirstlane((int)total) * Hkv;
-    longest = (unsigned)__builtin_amdgcn_readfirstlane((int)longest);
+    total *= Hkv;
     if (total == 0) return;
     const unsigned items = (unsigned)a.num_seqs * Hkv, cap = (unsigned)a.nsplit;
     // an item reaches into at most ceil(tiles / share) + 1 <= cap shares
     const unsigned share = max(max((total + nwg - 1) / nwg, (longest + cap - 2) / (cap - 1)), 2u);
     const unsigned ns = min(nwg / items, cap);
-    const bool aligned = ns >= 1 && (longest + ns - 1) / ns <= share + kSegmentTiles;
-    const unsigned snap = min(kSnapTiles, share / 8);
+    const bool aligned = ns >= 1 && (longest + ns - 1) / ns <= share;
+    const unsigned snap = min(kSnapTiles, share / 8), lead = kSegmentUnits + snap;
 
-    // the item that holds tile `pos` of the line: sequence, first tile of the sequence, its tiles
+    // the sequence that holds unit `pos` of the line, where it starts, and its tiles
     unsigned at_seq, at_start, at_tiles;
     auto locate = [&](unsigned pos) __attribute__((always_inline)) {
         unsigned before = 0;
         for (int c = 0;; c += 64) {
             const unsigned t = c == 0 ? t0 : tiles_of(c + lane);
-            const unsigned incl = c == 0 ? incl0 : wave_scan(t, lane);
+            const unsigned incl = c == 0 ? incl0 : wave_scan(units_of(t));
             const int k = __popcll(__ballot(Hkv * (before + incl) <= pos));
             if (k < 64) {
                 at_seq = (unsigned)(c + k);
                 at_tiles = (unsigned)__builtin_amdgcn_readlane((int)t, k);
-                at_start = Hkv * (before + (unsigned)__builtin_amdgcn_readlane((int)(incl - t), k));
+                at_start = Hkv * (before + (unsigned)__builtin_amdgcn_readlane((int)incl, k) - units_of(at_tiles));
                 return;
             }
             before += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
         }
     };
-    // start of share x of the even split
+    // start of share x of the even split: on an item's start, or past its first `lead` units
     auto bound = [&](unsigned x) __attribute__((always_inline)) -> unsigned {
         const unsigned raw = (unsigned)min((uint64_t)x * share, (uint64_t)total);
         if (raw == 0 || raw == total) return raw;
         locate(raw);
-        const unsigned off = (raw - at_start) % at_tiles;
-        if (off <= snap) return raw - off;
-        return at_tiles - off <= snap ? raw + (at_tiles - off) : raw;
+        const unsigned units = units_of(at_tiles), off = (raw - at_start) % units;
+        if (off <= lead) return raw - off;
+        return units - off <= snap ? raw + (units - off) : raw;
     };
 
     unsigned pos = 0, end = 0;
@@ -998,13 +1008,12 @@ __global__ void __launch_bounds__(kThreads, 1) pd_balanced_kernel(const PartialP
             wk.g = (int)(item - (unsigned)wk.b * Hkv);
         } else {
             locate(pos);
-            const unsigned g = (pos - at_start) / at_tiles, item = at_start + g * at_tiles;
-            first = pos - item;
-            last = min(at_tiles, end - item);
-            // the item's first workgroup: the one whose share holds its first tile, or the next if that
-            // one's start has moved onto the item's
-            const unsigned x = item / share, next = (x + 1) * share;
-            seg = wg - (x + (next - item <= snap && next < item + at_tiles ? 1u : 0u));
+            const unsigned units = units_of(at_tiles), g = (pos - at_start) / units, item = at_start + g * units;
+            first = pos - item <= lead ? 0 : pos - item - kSegmentUnits;
+            last = end - item >= units ? at_tiles : end - item - kSegmentUnits;
+            // the item's first workgroup is the last one whose share starts at or before the item: the last
+            // whose start lies in the item's first `lead` units, if any does
+            seg = wg - min(item + lead, item + units - 1) / share;
             wk.b = (int)at_seq;
             wk.g = (int)g;
         }
@@ -1037,8 +1046,8 @@ __global__ void __launch_bounds__(kThreads, 1) pd_balanced_kernel(const PartialP
             }
         }
         partial_body<NRB, kFast>(a, wk, lds);
-        if (aligned) return;
-        pos += last - first;
+        if (aligned || last < (unsigned)wk.ntiles) return;
+        pos = (first ? pos - first - kSegmentUnits : pos) + units_of((unsigned)wk.ntiles);  // the next item
         if (pos >= end) return;
         __syncthreads();  // every wave has read the merge's blocks: the slots can be refilled
     }
@@ -1272,10 +1281,15 @@ static hipError_t launch_balanced_nrb(const PartialParams& p, int wgs, hipStream
     return hipGetLastError();
 }
 
-// Segments per item that a balanced launch may use (0: the batch is not one for it). More than one
+// Segments per item that a balanced launch may use (0: the batch is not one for it). A split count whose
+// workgroups fit one round of the CUs has been planned for the batch's lengths, and its kernel starts ~1.5 us earlier
+// (16 x 300 keys at 4 splits 11.5 us against 12.6, 64 x 4,096 at 1 split 109.2 against 111.3); past one
+// round the balanced kernel won at every batch measured (the figures at
+// pd_balanced_kernel) but at many short equal ones (128 x 1,024 keys at 1 split 74.4 against 77.3). More than one
 // sequence, since one alone is dealt evenly by pd_partial_kernel; at least two segments for the shares' ends;
 // at most two row blocks (three do not fit the registers beside the line's state); and, with a block table of this width, a line of tiles that 32 bits number.
-static int balanced_segments(const LaunchArgs& x) {
+static int balanced_segments(const LaunchArgs& x, int cus) {
+    if ((int64_t)x.nsplit * x.heads_kv * x.num_seqs <= cus) return 0;
     const int64_t tiles = ((int64_t)x.bt_stride * x.block_size + kTile - 1) / kTile + 1;
     if (x.num_seqs < 2 || x.nseg < 2 || x.bt_stride < 1 || x.qmax * (x.heads_q / x.heads_kv) > 32) return 0;
     if (tiles > INT32_MAX || tiles * x.num_seqs > INT32_MAX / x.heads_kv) return 0;
@@ -1325,7 +1339,7 @@ hipError_t launch_partial(const LaunchArgs& x, hipStream_t stream, int* balanced
     const bool fast = fast_block_table(x.block_size, x.k_ss);
     if (balanced) {
         const int cus = compute_units(stream);
-        *balanced = p.rslices == 1 && cus > 0 ? balanced_segments(x) : 0;
+        *balanced = p.rslices == 1 && cus > 0 ? balanced_segments(x, cus) : 0;
         if (*balanced) {
             p.nsplit = *balanced;
             if (rows <= 16) return launch_balanced_nrb<1>(p, cus, stream, fast);
