@@ -201,6 +201,34 @@ int pth_fa_forward_split(const pd_tensor* q, const pd_tensor* key_cache, const p
                          int64_t nsplit, int64_t exact, hipStream_t stream, char* err, int errlen);
 
 /*
+ * No counterpart in the reference. The prefill with the key tiles of all query tiles dealt evenly over the GPU by
+ * the lengths on the device, for chunks whose query tiles see different numbers of keys (fresh prompts), do not
+ * fill the GPU, or belong to several sequences. Two forms:
+ *   query_start == NULL: pth_fa_forward's arguments, checks and messages (num_seqs is ignored).
+ *   query_start (host, int[num_seqs + 1], num_seqs <= 32): q fp16 [T, Hq, 256] with unit dim stride, rows
+ *     16-byte aligned; sequence i has rows [query_start[i], query_start[i + 1]) of q and out, the last tokens
+ *     of its seq_lens[i] keys; block_table and seq_lens have a row per sequence; out fp16 [T, Hq, 256],
+ *     rows 8-byte aligned. The rows outside the sequences are left alone. q_abs_offset is ignored.
+ *   workspace  fp32, contiguous, 16-byte aligned, of pth_fa_balanced_workspace floats (fewer, down to
+ *              2 x 192 x 258, only lower the number of workgroups)
+ *   max_keys   a bound on the keys any row sees, to size the launch; a wrong one costs time only
+ *   nsplit     0; or, in the rows form with one sequence, 1..64: pth_fa_forward_split's kernels on the rows
+ *              instead (workspace rows x Hq x nsplit x 258 floats when above 1)
+ * Numerics and return codes are those of pth_fa_forward (exact != 0: pth_fa_forward_exact); the results equal
+ * theirs within rounding (partial sums are merged in another order).
+ */
+int pth_fa_forward_balanced(const pd_tensor* q, const pd_tensor* key_cache, const pd_tensor* value_cache,
+                            const pd_tensor* block_table, const pd_tensor* seq_lens, double scale,
+                            const pd_tensor* q_abs_offset, const int* query_start, int64_t num_seqs, const pd_tensor* out,
+                            const pd_tensor* workspace, int64_t max_keys, int64_t nsplit, int64_t exact, hipStream_t stream,
+                            char* err, int errlen);
+/* Workspace floats for pth_fa_forward_balanced on the current device; 0 if it does not take such a call (no query
+ * tokens, more than 32 sequences in the rows form, more than 2^31 key tiles). table_keys: block_table columns x
+ * block size. */
+int64_t pth_fa_balanced_workspace(int64_t num_seqs, const int* query_start, int64_t sq, int64_t heads_q, int64_t heads_kv,
+                                  int64_t max_keys, int64_t table_keys);
+
+/*
  * KV-cache writer and quantiser: the producer of the 520-byte rows the two operators read.
  * Replaces vLLM's cache update for int8 per-token-head KV, which the reference calls as
  * do_kv_cache_update(layer, key, value, kv_cache, slot_mapping)

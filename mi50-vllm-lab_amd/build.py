@@ -4,7 +4,7 @@
 
 The library is the C ABI declared in include/pth_dec.h. Beside it pd_native.so, the Python extension
 through which pth_dec.py calls it on torch tensors (host code only, torch's headers). Both are
-always rebuilt: hipcc takes about half a minute and a stale library is worse than a slow build.
+always rebuilt: hipcc takes about a minute and a stale library is worse than a slow build.
 """
 import argparse
 import os
@@ -12,6 +12,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -43,16 +44,25 @@ def hipcc() -> str:
 def build(save_temps: str | None = None, verbose: bool = False) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     tmp = LIB_PATH + ".tmp"
-    cmd = [hipcc(), *HIP_FLAGS, "-I", os.path.join(ROOT, "include"), *SOURCES, "-o", tmp]
     if save_temps:
         os.makedirs(save_temps, exist_ok=True)
-        cmd.insert(1, f"-save-temps={'obj'}")
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    cwd = save_temps if save_temps else None
-    if save_temps:
-        cmd[-1] = os.path.abspath(tmp)
-    res = subprocess.run(cmd, cwd=cwd, capture_output=True, text=True)
+    with tempfile.TemporaryDirectory() as objdir:
+        # one compiler per source, side by side (the prefill kernels take longest)
+        jobs = []
+        for src in SOURCES:
+            obj = os.path.join(objdir, os.path.basename(src) + ".o")
+            cmd = [hipcc(), *(["-save-temps=obj"] if save_temps else []), *(f for f in HIP_FLAGS if f != "-shared"), "-c", "-I",
+                   os.path.join(ROOT, "include"), src, "-o", os.path.join(save_temps, os.path.basename(obj)) if save_temps else obj]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            jobs.append((cmd[-1], subprocess.Popen(cmd, cwd=save_temps, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+        outs = [(obj, p.communicate()[0], p.returncode) for obj, p in jobs]
+        for _, text, rc in outs:
+            if rc != 0:
+                sys.stderr.write(text)
+                raise RuntimeError(f"hipcc failed ({rc}) building {LIB_PATH}")
+        res = subprocess.run([hipcc(), *HIP_FLAGS, *(obj for obj, _, _ in outs), "-o", os.path.abspath(tmp)],
+                             capture_output=True, text=True)
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
         raise RuntimeError(f"hipcc failed ({res.returncode}) building {LIB_PATH}")

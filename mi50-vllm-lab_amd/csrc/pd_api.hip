@@ -7,6 +7,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+
 #pragma GCC visibility push(default)
 #include "pth_dec.h"
 #pragma GCC visibility pop
@@ -250,10 +252,45 @@ int pth_dec_decode(const pd_tensor* q, const pd_tensor* key_cache, const pd_tens
     return 0;
 }
 
+static int fa_result(hipError_t e, char* err, int errlen) {
+    if (e == hipSuccess) return 0;
+    char msg[256];
+    snprintf(msg, sizeof msg, "pth_fa launch failed: %s", hipGetErrorString(e));
+    fail(err, errlen, msg);
+    return 2;
+}
+
+// bytes from the cache base to the last K row's scale
+static int64_t cache_span(const pd_tensor* kc) {
+    return (kc->sizes[0] - 1) * kc->strides[0] + (kc->sizes[1] - 1) * kc->strides[1] + (kc->sizes[2] - 1) * kc->strides[2] + 8;
+}
+
+// Whether 32 bits number the line of a balanced prefill: items x the key tiles that a block table can hold.
+static bool balanced_ok(int64_t items, int64_t table_keys) {
+    const int64_t tiles = table_keys / 32 + 64;
+    return items <= INT32_MAX / 2 && tiles <= INT32_MAX / 2 && items * tiles <= INT32_MAX;
+}
+static const char* balanced_workspace(FaParams& p, FaRowsParams& r, const pd_tensor* ws, int64_t items, int64_t max_keys,
+                                      hipStream_t stream) {
+    if (!(ws && ws->dtype == PD_DTYPE_FP32 && ws->ndim == 1 && is_contig(ws) &&
+          reinterpret_cast<uintptr_t>(ws->data) % 16 == 0 && ws->sizes[0] >= 2 * kFaSlotFloats))
+        return "workspace must be contiguous 16-byte aligned fp32 of pth_fa_balanced_workspace";
+    const int cus = compute_units(stream);
+    r.nwg = (int)std::min(ws->sizes[0] / (2 * kFaSlotFloats),
+                          balanced_prefill_workgroups(items, std::max<int64_t>(0, max_keys), cus > 0 ? cus : 256));
+    float* f = static_cast<float*>(const_cast<void*>(ws->data));
+    const int64_t rows = 2ll * r.nwg * kFaRows;
+    p.part_o = f;
+    p.part_m = f + rows * kDim;
+    p.part_l = p.part_m + rows;
+    return nullptr;
+}
+
 static int fa_forward(const pd_tensor* q, const pd_tensor* key_cache, const pd_tensor* value_cache,
                       const pd_tensor* block_table, const pd_tensor* seq_lens, double scale,
                       const pd_tensor* q_abs_offset, const pd_tensor* out, hipStream_t stream, char* err, int errlen,
-                      bool exact, int64_t nsplit = 1, const pd_tensor* workspace = nullptr) {
+                      bool exact, int64_t nsplit = 1, const pd_tensor* workspace = nullptr,
+                      const int64_t* balanced_keys = nullptr) {
     if (!q || !key_cache || !value_cache || !block_table || !seq_lens || !q_abs_offset || !out)
         return fail(err, errlen, "null tensor descriptor");
     if (!(q->dtype == PD_DTYPE_FP32 && q->ndim == 4 && is_contig(q)))
@@ -309,7 +346,7 @@ static int fa_forward(const pd_tensor* q, const pd_tensor* key_cache, const pd_t
     }
     if (B == 0 || Sq == 0) return 0;
     FaParams p;
-    p.q = static_cast<const float*>(q->data);
+    p.q = q->data;
     p.q_sb = q->strides[0];
     p.q_sh = q->strides[1];
     p.q_st = q->strides[2];
@@ -321,7 +358,7 @@ static int fa_forward(const pd_tensor* q, const pd_tensor* key_cache, const pd_t
     p.bt_stride = block_table->strides[0];
     p.seq_lens = static_cast<const int*>(seq_lens->data);
     p.q_abs = static_cast<const int*>(q_abs_offset->data);
-    p.out = static_cast<float*>(const_cast<void*>(out->data));
+    p.out = const_cast<void*>(out->data);
     p.o_sb = out->strides[0];
     p.o_st = out->strides[1];
     p.o_sh = out->strides[2];
@@ -334,9 +371,7 @@ static int fa_forward(const pd_tensor* q, const pd_tensor* key_cache, const pd_t
     p.scale_log2 = (float)scale * 1.4426950408889634f;
     // 16-key block offsets fit the LDS table's 32 bits (in 8-byte units) when the cache spans
     // less than 2^35 bytes
-    const int64_t span = (key_cache->sizes[0] - 1) * key_cache->strides[0] + (bs - 1) * key_cache->strides[1] +
-                         (Hkv - 1) * key_cache->strides[2] + 8;
-    p.bt32 = span < ((int64_t)1 << 35);
+    p.bt32 = cache_span(key_cache) < ((int64_t)1 << 35);
     p.nsplit = (int)nsplit;
     p.part_o = nullptr;
     p.part_m = nullptr;
@@ -348,14 +383,113 @@ static int fa_forward(const pd_tensor* q, const pd_tensor* key_cache, const pd_t
         p.part_m = ws + prow * kDim;
         p.part_l = p.part_m + prow;
     }
-    const hipError_t e = launch_prefill(p, (int)B, (int)Hkv, stream, exact);
-    if (e != hipSuccess) {
-        char msg[256];
-        snprintf(msg, sizeof msg, "pth_fa launch failed: %s", hipGetErrorString(e));
-        fail(err, errlen, msg);
-        return 2;
+    if (balanced_keys) {
+        FaRowsParams r = {};
+        const int64_t qtiles = (Sq + p.tok_per_wg - 1) / p.tok_per_wg;
+        r.first_tile[0] = (int)B;
+        r.tiles = (int)(B * qtiles);
+        const char* why = nullptr;
+        if (!balanced_ok(B * qtiles * Hkv, block_table->sizes[1] * bs) || Hq == 0)
+            why = "a balanced prefill takes at most 2^31 key tiles";
+        else
+            why = balanced_workspace(p, r, workspace, r.tiles * Hkv, *balanced_keys, stream);
+        if (why) return fail(err, errlen, why);
+        return fa_result(launch_prefill_balanced(p, r, (int)Hkv, PD_DTYPE_FP32, stream, exact), err, errlen);
     }
-    return 0;
+    return fa_result(launch_prefill(p, (int)B, (int)Hkv, PD_DTYPE_FP32, stream, exact), err, errlen);
+}
+
+// The rows form: sequence i has rows [query_start[i], query_start[i + 1]) of q and out [T, Hq, 256], the last
+// tokens of its seq_lens[i] keys. nsplit 0: balanced; else one sequence with its keys in nsplit splits.
+static int fa_forward_rows(const pd_tensor* q, const pd_tensor* kc, const pd_tensor* vc, const pd_tensor* bt,
+                           const pd_tensor* seq_lens, double scale, const int* query_start, int64_t num_seqs,
+                           const pd_tensor* out, const pd_tensor* workspace, int64_t max_keys, int64_t nsplit,
+                           bool exact, hipStream_t stream, char* err, int errlen) {
+    if (!(q->ndim == 3 && q->dtype == PD_DTYPE_FP16 && q->sizes[2] == kDim &&
+          q->strides[2] == 1 && q->sizes[0] <= INT32_MAX && q->sizes[1] <= INT32_MAX))
+        return fail(err, errlen, "q must be fp16 [T, Hq, 256] with unit dim stride");
+    if (!(out->ndim == 3 && out->dtype == q->dtype && out->sizes[0] == q->sizes[0] && out->sizes[1] == q->sizes[1] &&
+          out->sizes[2] == kDim && out->strides[2] == 1))
+        return fail(err, errlen, "out must be fp16 [T, Hq, 256] with unit dim stride");
+    if (!(reinterpret_cast<uintptr_t>(q->data) % 16 == 0 && q->strides[0] % 8 == 0 && q->strides[1] % 8 == 0 &&
+          reinterpret_cast<uintptr_t>(out->data) % 8 == 0 && out->strides[0] % 4 == 0 && out->strides[1] % 4 == 0))
+        return fail(err, errlen, "q rows must be 16-byte aligned and out rows 8-byte aligned");
+    if (!(kc->dtype == PD_DTYPE_INT8 && vc->dtype == PD_DTYPE_INT8 && kc->ndim == 4 && vc->ndim == 4 &&
+          kc->strides[3] == 1 && vc->strides[3] == 1 && kc->sizes[3] >= kDim + 4 && vc->sizes[3] >= kDim + 4))
+        return fail(err, errlen, "key/value cache views must be 4D int8 rows of D values and a fp32 scale");
+    const uintptr_t kb = reinterpret_cast<uintptr_t>(kc->data);
+    bool rows_ok = kb % 8 == 0 && reinterpret_cast<uintptr_t>(vc->data) == kb + 260;
+    for (int i = 0; i < 3; ++i)
+        rows_ok = rows_ok && kc->strides[i] == vc->strides[i] && kc->sizes[i] == vc->sizes[i] && kc->strides[i] % 8 == 0 &&
+                  kc->strides[i] <= INT32_MAX;
+    if (!rows_ok) return fail(err, errlen, "value_cache must view the same 8-byte aligned cache rows as key_cache, 260 bytes in");
+    const int64_t T = q->sizes[0], Hq = q->sizes[1], bs = kc->sizes[1], Hkv = kc->sizes[2];
+    if (!(Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && Hq / Hkv <= kFaRows))
+        return fail(err, errlen, "heads_q must be a multiple of heads_kv, at most 192 times");
+    if (!(num_seqs >= 1 && num_seqs <= kFaMaxSeqs && query_start[0] >= 0 && query_start[num_seqs] <= T))
+        return fail(err, errlen, "1 to 32 sequences within the rows of q");
+    for (int64_t i = 0; i < num_seqs; ++i)
+        if (query_start[i] > query_start[i + 1]) return fail(err, errlen, "query_start must not decrease");
+    if (!(bt->dtype == PD_DTYPE_INT32 && bt->ndim == 2 && bt->sizes[0] >= num_seqs && bt->strides[1] == 1 &&
+          seq_lens->dtype == PD_DTYPE_INT32 && seq_lens->ndim == 1 && seq_lens->sizes[0] >= num_seqs && is_contig(seq_lens)))
+        return fail(err, errlen, "block_table / seq_lens must be int32 with a row per sequence");
+    FaParams p = {};
+    p.q = q->data;
+    p.q_sh = q->strides[1];
+    p.q_st = q->strides[0];
+    p.kc = static_cast<const int8_t*>(kc->data);
+    p.k_sb = kc->strides[0];
+    p.k_ss = kc->strides[1];
+    p.k_sh = kc->strides[2];
+    p.block_table = static_cast<const int*>(bt->data);
+    p.bt_stride = bt->strides[0];
+    p.seq_lens = static_cast<const int*>(seq_lens->data);
+    p.out = const_cast<void*>(out->data);
+    p.o_st = out->strides[0];
+    p.o_sh = out->strides[1];
+    p.Hq = (int)Hq;
+    p.G = (int)(Hq / Hkv);
+    p.tok_per_wg = kFaRows / p.G;
+    p.block_size = (int)bs;
+    p.bs_shift = (bs & (bs - 1)) == 0 ? __builtin_ctz((unsigned)bs) : -1;
+    p.scale_log2 = (float)scale * 1.4426950408889634f;
+    p.bt32 = cache_span(kc) < ((int64_t)1 << 35);
+    p.nsplit = 1;
+    if (nsplit != 0) {
+        const int64_t n = query_start[1] - query_start[0];
+        if (!(num_seqs == 1 && nsplit >= 1 && nsplit <= 64 && (nsplit == 1 || n * Hq * nsplit <= INT32_MAX)))
+            return fail(err, errlen, "nsplit must be 0, or in [1, 64] for one sequence");
+        if (n == 0) return 0;
+        if (nsplit > 1) {
+            const int64_t rows = n * Hq * nsplit;
+            if (!(workspace && workspace->dtype == PD_DTYPE_FP32 && workspace->ndim == 1 && is_contig(workspace) &&
+                  workspace->sizes[0] >= prefill_workspace_floats(1, n, Hq, nsplit) &&
+                  reinterpret_cast<uintptr_t>(workspace->data) % 16 == 0))
+                return fail(err, errlen, "workspace must be contiguous 16-byte aligned fp32 of rows * Hq * nsplit * 258");
+            p.part_o = static_cast<float*>(const_cast<void*>(workspace->data));
+            p.part_m = p.part_o + rows * kDim;
+            p.part_l = p.part_m + rows;
+        }
+        p.q = static_cast<const _Float16*>(p.q) + query_start[0] * p.q_st;
+        p.out = static_cast<_Float16*>(p.out) + query_start[0] * p.o_st;
+        p.Sq = (int)n;
+        p.nsplit = (int)nsplit;
+        return fa_result(launch_prefill(p, 1, (int)Hkv, PD_DTYPE_FP16, stream, exact), err, errlen);
+    }
+    FaRowsParams r = {};
+    r.n = (int)num_seqs;
+    int64_t tiles = 0;
+    for (int64_t i = 0; i < num_seqs; ++i) {
+        r.first_tok[i] = query_start[i];
+        r.first_tile[i] = (int)tiles;
+        tiles += (query_start[i + 1] - query_start[i] + p.tok_per_wg - 1) / p.tok_per_wg;
+    }
+    r.first_tok[num_seqs] = query_start[num_seqs];
+    r.first_tile[num_seqs] = r.tiles = (int)tiles;
+    if (tiles == 0) return 0;
+    if (!balanced_ok(tiles * Hkv, bt->sizes[1] * bs)) return fail(err, errlen, "a balanced prefill takes at most 2^31 key tiles");
+    if (const char* why = balanced_workspace(p, r, workspace, tiles * Hkv, max_keys, stream)) return fail(err, errlen, why);
+    return fa_result(launch_prefill_balanced(p, r, (int)Hkv, q->dtype, stream, exact), err, errlen);
 }
 
 int pth_fa_forward(const pd_tensor* q, const pd_tensor* key_cache, const pd_tensor* value_cache,
@@ -379,6 +513,42 @@ int pth_fa_forward_split(const pd_tensor* q, const pd_tensor* key_cache, const p
                          int64_t nsplit, int64_t exact, hipStream_t stream, char* err, int errlen) {
     return fa_forward(q, key_cache, value_cache, block_table, seq_lens, scale, q_abs_offset, out, stream, err, errlen,
                       exact != 0, nsplit, workspace);
+}
+
+int64_t pth_fa_balanced_workspace(int64_t num_seqs, const int* query_start, int64_t sq, int64_t heads_q, int64_t heads_kv,
+                                  int64_t max_keys, int64_t table_keys) {
+    if (num_seqs < 1 || heads_kv < 1 || heads_q < 1 || heads_q % heads_kv != 0 || heads_q / heads_kv > kFaRows) return 0;
+    const int64_t tok = kFaRows / (heads_q / heads_kv);
+    int64_t tiles = 0;
+    if (query_start) {
+        if (num_seqs > kFaMaxSeqs) return 0;
+        for (int64_t i = 0; i < num_seqs; ++i) tiles += (query_start[i + 1] - query_start[i] + tok - 1) / tok;
+    } else {
+        if (sq < 0 || sq > INT32_MAX || num_seqs > INT32_MAX) return 0;
+        tiles = num_seqs * ((sq + tok - 1) / tok);
+    }
+    if (tiles < 1 || tiles > INT32_MAX / heads_kv || !balanced_ok(tiles * heads_kv, std::max<int64_t>(0, table_keys))) return 0;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    return 2 * kFaSlotFloats * balanced_prefill_workgroups(tiles * heads_kv, std::max<int64_t>(0, max_keys), cus);
+}
+
+int pth_fa_forward_balanced(const pd_tensor* q, const pd_tensor* key_cache, const pd_tensor* value_cache,
+                            const pd_tensor* block_table, const pd_tensor* seq_lens, double scale,
+                            const pd_tensor* q_abs_offset, const int* query_start, int64_t num_seqs, const pd_tensor* out,
+                            const pd_tensor* workspace, int64_t max_keys, int64_t nsplit, int64_t exact, hipStream_t stream,
+                            char* err, int errlen) {
+    if (query_start) {
+        if (!q || !key_cache || !value_cache || !block_table || !seq_lens || !out)
+            return fail(err, errlen, "null tensor descriptor");
+        return fa_forward_rows(q, key_cache, value_cache, block_table, seq_lens, scale, query_start, num_seqs, out, workspace,
+                               max_keys, nsplit, exact != 0, stream, err, errlen);
+    }
+    if (nsplit != 0) return fail(err, errlen, "nsplit must be 0 in the batch form");
+    return fa_forward(q, key_cache, value_cache, block_table, seq_lens, scale, q_abs_offset, out, stream, err, errlen,
+                      exact != 0, 1, workspace, &max_keys);
 }
 
 int pth_cache_write(const pd_tensor* key, const pd_tensor* value, const pd_tensor* key_cache,

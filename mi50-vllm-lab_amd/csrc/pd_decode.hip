@@ -904,33 +904,6 @@ __global__ void __launch_bounds__(kThreads, 1) pd_partial_kernel(const PartialPa
 constexpr unsigned kSegmentUnits = 12;  // set-up and merge of a segment, ~10 us, in tiles of a workgroup (~0.8 us each)
 constexpr unsigned kSnapTiles = 6;      // a share's end this close to an item's boundary moves onto it
 
-// DPP move with 0 in lanes that have no source (kRows: the 16-lane rows that take part).
-template <int kCtrl, int kRows = 0xf>
-__device__ __forceinline__ unsigned dpp_or_zero(unsigned v) {
-    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xf, false);
-}
-// Inclusive sum over the lanes: shifts inside 16-lane rows, then the last lane of row 0 into row 1 and of row
-// 2 into row 3, then the last lane of the lower half into the upper.
-__device__ __forceinline__ unsigned wave_scan(unsigned v) {
-    v += dpp_or_zero<0x111>(v);       // row_shr:1
-    v += dpp_or_zero<0x112>(v);       // row_shr:2
-    v += dpp_or_zero<0x114>(v);       // row_shr:4
-    v += dpp_or_zero<0x118>(v);       // row_shr:8
-    v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15
-    v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31
-    return v;
-}
-// Largest value of the wave, uniform (the same steps; the last lane has seen every other).
-__device__ __forceinline__ unsigned wave_umax(unsigned v) {
-    v = max(v, dpp_or_zero<0x111>(v));
-    v = max(v, dpp_or_zero<0x112>(v));
-    v = max(v, dpp_or_zero<0x114>(v));
-    v = max(v, dpp_or_zero<0x118>(v));
-    v = max(v, dpp_or_zero<0x142, 0xa>(v));
-    v = max(v, dpp_or_zero<0x143, 0xc>(v));
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-
 template <int NRB, bool kFast>
 __global__ void __launch_bounds__(kThreads, 1) pd_balanced_kernel(const PartialParams a) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[PartialLds<NRB, kFast>::kBytes];
@@ -1249,7 +1222,7 @@ hipError_t check_args(const LaunchArgs& x, bool strict_reference) {
 }
 
 // Compute units of the device a stream belongs to (looked up once per device; 0 if unknown).
-static int compute_units(hipStream_t stream) {
+int compute_units(hipStream_t stream) {
     constexpr int kDevices = 64;
     static std::atomic<int> cached[kDevices];
     int dev = -1;

@@ -64,15 +64,15 @@ struct CombineParams {
 
 // Chunked prefill (pd_prefill_kernel).
 struct FaParams {
-    const float* q;
+    const void* q;             // fp32 or fp16
     int64_t q_sb, q_sh, q_st;  // elements between batches / heads / tokens of q [B, Hq, Sq, 256]
     const int8_t* kc;
     int64_t k_sb, k_ss, k_sh;
     const int* block_table;
     int64_t bt_stride;
     const int* seq_lens;
-    const int* q_abs;
-    float* out;
+    const int* q_abs;          // null: the last Sq keys' positions
+    void* out;                 // q's type
     int64_t o_sb, o_st, o_sh;  // elements between batches / tokens / heads of out [B, Sq, Hq, 256]
     int Sq, Hq, G, tok_per_wg, block_size, bs_shift;
     int bt32;                  // every K row lies within 2^35 bytes of the cache base
@@ -84,6 +84,18 @@ struct FaParams {
     float* part_o;
     float* part_m;
     float* part_l;
+};
+
+// The sequences of a balanced prefill. Batch form (n == 0): q [B, Hq, Sq, 256], every sequence Sq tokens at
+// q_abs. Rows form: n sequences of consecutive rows of q [T, Hq, 256], the last tokens of their keys;
+// sequence i has rows [first_tok[i], first_tok[i + 1]) and query tiles [first_tile[i], first_tile[i + 1]).
+constexpr int kFaMaxSeqs = 32;
+struct FaRowsParams {
+    int n;
+    int first_tok[kFaMaxSeqs + 1];
+    int first_tile[kFaMaxSeqs + 1];
+    int tiles;                       // query tiles of a kv head, all sequences
+    int nwg;                         // workgroups of the launch
 };
 
 // KV-cache writer (pd_cache_write_kernel).
@@ -137,7 +149,18 @@ hipError_t scratch_address(void** out);
 
 // chunked prefill (pd_prefill.hip)
 // exact: K converted to fp16 without the widening bias and P' as fp16 hi + lo (pth_fa_forward_exact)
-hipError_t launch_prefill(const FaParams& p, int batch, int heads_kv, hipStream_t stream, bool exact);
+// dtype: PD_DTYPE_FP32 or _FP16 of q and out
+hipError_t launch_prefill(const FaParams& p, int batch, int heads_kv, int dtype, hipStream_t stream, bool exact);
+// the same with the key tiles of all query tiles dealt evenly over r.nwg workgroups; dtype: of q and
+// out (fp32 in the batch form, fp16 in the rows form); partials in p.part_o/m/l (2 slots of kFaRows rows
+// per workgroup)
+hipError_t launch_prefill_balanced(const FaParams& p, const FaRowsParams& r, int heads_kv, int dtype, hipStream_t stream,
+                                   bool exact);
+// workgroups of such a launch on `cus` CUs: as many as the work pays for, at least one per item while CUs last
+int64_t balanced_prefill_workgroups(int64_t items, int64_t max_keys, int cus);
+constexpr int64_t kFaSlotFloats = (int64_t)kFaRows * (kDim + 2);
+// compute units of a stream's device (0 if unknown)
+int compute_units(hipStream_t stream);
 // workspace floats a split prefill needs: B * Sq * Hq rows x nsplit x (256 + 2)
 inline int64_t prefill_workspace_floats(int64_t B, int64_t Sq, int64_t Hq, int64_t nsplit) {
     return B * Sq * Hq * nsplit * (kDim + 2);

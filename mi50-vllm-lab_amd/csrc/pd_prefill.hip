@@ -15,9 +15,11 @@
 // products as fp16 hi + lo, which doubles them. The default instance keeps the bias in K and V
 // and removes it per row (sum_d q_d (k_d + 1152) - 1152 sum_d q_d, sum_k P'_k (v_k + 1152) -
 // 1152 sum_k P'_k).
+#include <algorithm>
 #include <type_traits>
 
 #include "pd_tile.hpp"
+#include "pth_dec.h"
 
 namespace pd {
 
@@ -78,49 +80,62 @@ __device__ __forceinline__ void wait_quarters(int later, bool tail) {
     }
 }
 
-template <bool kFast, bool kExact, bool kSplit>
-__global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaParams a) {
-    constexpr int kLdsRaw = 0;
-    constexpr int kLdsH = kLdsRaw + kFaRaw * kSlot;
+// Eight consecutive query values as fp16. Q is rounded to fp16 unscaled: fp16-valued queries enter the
+// matrix cores exactly.
+template <class T>
+__device__ __forceinline__ half8_t load_q8(const T* p) {
+    if constexpr (sizeof(T) == 4) {
+        const float4_t x0 = *reinterpret_cast<const float4_t*>(p), x1 = *reinterpret_cast<const float4_t*>(p + 4);
+        return half8_t{(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w,
+                       (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
+    } else {
+        return *reinterpret_cast<const half8_t*>(p);
+    }
+}
+template <class T>
+__device__ __forceinline__ void store_out4(T* p, float4_t v) {
+    if constexpr (sizeof(T) == 4) {
+        *reinterpret_cast<float4_t*>(p) = v;
+    } else {
+        typedef T out4_t __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<out4_t*>(p) = out4_t{(T)v.x, (T)v.y, (T)v.z, (T)v.w};
+    }
+}
+
+// LDS of a prefill workgroup: raw ring, two fp16 buffers, block table.
+constexpr int kFaLdsH = kFaRaw * kSlot;
+constexpr int kFaLdsBt = kFaLdsH + 2 * kFaHBuf;
+constexpr int kFaLdsBytes = kFaLdsBt + kFaBt * 4;
+static_assert(kFaLdsBytes <= 160 * 1024, "gfx950 has 160 KiB of LDS per CU");
+
+// What a workgroup computes: query tokens [tq0, tq0 + ntok) of sequence b and the heads of kv head g, over
+// key tiles [t0, t1).
+struct FaWork {
+    int b, g, tq0, ntok;
+    int seq_len, qabs;         // keys; position of the sequence's query token 0
+    int64_t qrow0, orow0;      // elements to the sequence's query token 0 in q and in out
+    int t0, t1;
+    int part;                  // segment of the partials (kParts 1: split; 2: slot, or -1 for the output itself)
+};
+
+// kParts: 0 the rows are finished and stored; 1 partials of split wk.part; 2 either, as wk.part says.
+template <bool kFast, bool kExact, int kParts, class T>
+__device__ __forceinline__ void prefill_body(const FaParams& a, const FaWork& wk, unsigned char* lds) {
+    constexpr int kLdsRaw = 0, kLdsH = kFaLdsH, kLdsBt = kFaLdsBt;
     // The unsplit default instance addresses its widening stores from bases held per tile (see
     // widen_load), starts its row sums from the first term and forms P' by v_fma_mix; the split
     // and exact instances measured slower with these (the split one 4.14 -> 4.23 ms at 2,560
     // tokens x 4 splits, fma_mix being the part that costs it) and keep per-store addresses and
     // a multiply and a conversion for P'.
-    constexpr bool kPinned = !kExact && !kSplit;
-    constexpr int kLdsBt = kLdsH + 2 * kFaHBuf;
-    constexpr int kLdsBytes = kLdsBt + kFaBt * 4;
-    static_assert(kLdsBytes <= 160 * 1024, "gfx950 has 160 KiB of LDS per CU");
-    __shared__ __attribute__((aligned(16))) unsigned char lds[kLdsBytes];
-
-    // Workgroups are dispatched to the 8 XCDs round robin (linear id L to XCD L % 8), and each XCD
-    // has its own L2. Every query tile of a (sequence, kv head) streams the same keys, so the
-    // logical workgroup index (query tile fastest) is laid out XCD by XCD: XCD x takes a
-    // contiguous range of it, and the query tiles sharing a kv head mostly share an L2 (a 2,048-token
-    // chunk at 24 q / 4 kv heads: each kv head's 64 query tiles on two XCDs).
-    const unsigned nx = gridDim.x, ny = gridDim.y, nwg = nx * ny * gridDim.z;
-    const unsigned lin = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
-    const unsigned xcd = lin % 8u;
-    const unsigned lidx = xcd * (nwg / 8u) + min(xcd, nwg % 8u) + lin / 8u;
-    // x = split * (query tiles) + query tile: the query tiles of one split and kv head (which
-    // stream the same keys) stay neighbours in the XCD order
-    const int x = (int)(lidx % nx), g = (int)((lidx / nx) % ny), b = (int)(lidx / (nx * ny));
-    const int nqt = kSplit ? (int)nx / a.nsplit : (int)nx;
-    const int qt = kSplit ? x % nqt : x, split = kSplit ? x / nqt : 0;
+    constexpr bool kPinned = !kExact && kParts == 0;
+    const int b = wk.b, g = wk.g, tq0 = wk.tq0, ntok = wk.ntok, seq_len = wk.seq_len, qabs = wk.qabs;
+    const int t0 = wk.t0, t1 = wk.t1;
     const int tid = threadIdx.x, l = tid & 63, lg = l >> 4, li = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = a.G;
-    const int tq0 = qt * a.tok_per_wg;                 // first query token of the workgroup
-    const int ntok = min(a.tok_per_wg, a.Sq - tq0);    // query tokens of the workgroup
-    const int seq_len = a.seq_lens[b];
-    const int qabs = a.q_abs[b];
     // keys any row can see: [0, min(seq_len, last row's position + 1))
     const int hi = min(seq_len, qabs + tq0 + ntok);
-    const int ntiles = hi > 0 ? (hi - 1) / kTile + 1 : 0;
     const int pmin = qabs + tq0;                       // smallest row position
-    // this workgroup's run of key tiles [t0, t1): all of them unless the keys are split
-    const int per = kSplit ? (ntiles + a.nsplit - 1) / a.nsplit : ntiles;
-    const int t0 = kSplit ? min(ntiles, split * per) : 0, t1 = kSplit ? min(ntiles, t0 + per) : ntiles;
 
     // ---- rows of this wave: row r = 48 w + 16 rb + li -> (token r / G, head r % G) ----
     half8_t qop[kFaRB][8];
@@ -133,16 +148,12 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
         const int tok = r / G, hh = r - (r / G) * G;
         rvalid[rb] = tok < ntok && r < a.tok_per_wg * G;
         rpos[rb] = qabs + tq0 + tok;
-        const float* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(g * G + (rvalid[rb] ? hh : 0)) * a.q_sh +
+        const int64_t qat = (int64_t)wk.qrow0 + (int64_t)(g * G + (rvalid[rb] ? hh : 0)) * a.q_sh +
                             (int64_t)(tq0 + (rvalid[rb] ? tok : 0)) * a.q_st;
 #pragma unroll
         for (int st = 0; st < 8; ++st) {
             const int dim = 64 * (st >> 1) + 16 * lg + 8 * (st & 1);
-            const float4_t x0 = *reinterpret_cast<const float4_t*>(qrow + dim);
-            const float4_t x1 = *reinterpret_cast<const float4_t*>(qrow + dim + 4);
-            // Q is rounded to fp16 unscaled: fp16-valued queries enter the matrix cores exactly
-            const half8_t v = {(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w,
-                               (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
+            const half8_t v = load_q8<T>(static_cast<const T*>(a.q) + qat + dim);
             qop[rb][st] = rvalid[rb] ? v : (half8_t)(_Float16)0.0f;
         }
     }
@@ -553,6 +564,10 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
                 tile_back(n, sv, vs);
             }
         };
+        // The interior loop starts a fixed distance past a 64-byte line: one wave per SIMD feels where its 7 KB
+        // of code lie in the instruction fetch. Of 16 distances, 2,048 tokens over 61,440 keys took 3.23
+        // (here) to 3.36 ms, 2,560 in 4 splits 4.10 (here) to 4.41.
+        asm volatile(".p2align 6\n\ts_nop 0" ::: "memory");
         run(std::false_type{}, t0, min(n_int, t1));
         run(std::true_type{}, max(n_int, t0), t1);
     };
@@ -561,8 +576,7 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
     else
         tile_loop(std::false_type{});
 
-    // ---- normalise and store: out[b, tq0 + tok, g G + hh, :]; with the keys split, the
-    //      unnormalised partial O, the running max m and the sum l of the row instead ----
+    // ---- normalise and store the rows, or store their unnormalised O, running max m and sum l ----
 #pragma unroll
     for (int rb = 0; rb < kFaRB; ++rb) {
         const float l_row = xor_sum(xor_sum(l_run[rb], 16), 32);
@@ -573,8 +587,9 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
         if (rvalid[rb]) {
             const int r = 48 * w + 16 * rb + li;
             const int tok = r / G, hh = r - (r / G) * G;
-            if constexpr (kSplit) {
-                const int64_t pr = (((int64_t)b * a.Sq + tq0 + tok) * a.Hq + g * G + hh) * a.nsplit + split;
+            if (kParts == 1 || (kParts == 2 && wk.part >= 0)) {
+                const int64_t pr = kParts == 1 ? (((int64_t)b * a.Sq + tq0 + tok) * a.Hq + g * G + hh) * a.nsplit + wk.part
+                                               : (int64_t)wk.part * kFaRows + r;
                 float* prow = a.part_o + pr * kDim;
 #pragma unroll
                 for (int m = 0; m < 17; ++m) {
@@ -586,14 +601,305 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
                     a.part_l[pr] = l_row;
                 }
             } else {
-                float* orow = a.out + (int64_t)b * a.o_sb + (int64_t)(tq0 + tok) * a.o_st + (int64_t)(g * G + hh) * a.o_sh;
+                const int64_t orow = (int64_t)wk.orow0 + (int64_t)(tq0 + tok) * a.o_st + (int64_t)(g * G + hh) * a.o_sh;
 #pragma unroll
                 for (int m = 0; m < 17; ++m) {
                     const int d0 = m < 16 ? 16 * m - 4 + 4 * lg : (lg == 2 ? 252 : -1);
-                    if (d0 >= 0 && d0 < kDim) *reinterpret_cast<float4_t*>(orow + d0) = (oacc[rb][m] - corr) * inv;
+                    if (d0 >= 0 && d0 < kDim) store_out4<T>(static_cast<T*>(a.out) + orow + d0, (oacc[rb][m] - corr) * inv);
                 }
             }
         }
+    }
+}
+
+template <bool kFast, bool kExact, bool kSplit, class T>
+__global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaParams a) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kFaLdsBytes];
+
+    // Workgroups are dispatched to the 8 XCDs round robin (linear id L to XCD L % 8), and each XCD
+    // has its own L2. Every query tile of a (sequence, kv head) streams the same keys, so the
+    // logical workgroup index (query tile fastest) is laid out XCD by XCD: XCD x takes a
+    // contiguous range of it, and the query tiles sharing a kv head mostly share an L2 (a 2,048-token
+    // chunk at 24 q / 4 kv heads: each kv head's 64 query tiles on two XCDs).
+    const unsigned nx = gridDim.x, ny = gridDim.y, nwg = nx * ny * gridDim.z;
+    const unsigned lin = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
+    const unsigned xcd = lin % 8u;
+    const unsigned lidx = xcd * (nwg / 8u) + min(xcd, nwg % 8u) + lin / 8u;
+    // x = split * (query tiles) + query tile: the query tiles of one split and kv head (which
+    // stream the same keys) stay neighbours in the XCD order
+    const int x = (int)(lidx % nx), g = (int)((lidx / nx) % ny), b = (int)(lidx / (nx * ny));
+    const int nqt = kSplit ? (int)nx / a.nsplit : (int)nx;
+    const int qt = kSplit ? x % nqt : x, split = kSplit ? x / nqt : 0;
+    FaWork wk;
+    wk.b = b;
+    wk.g = g;
+    wk.tq0 = qt * a.tok_per_wg;                 // first query token of the workgroup
+    wk.ntok = min(a.tok_per_wg, a.Sq - wk.tq0);    // query tokens of the workgroup
+    wk.seq_len = a.seq_lens[b];
+    wk.qabs = a.q_abs ? a.q_abs[b] : wk.seq_len - a.Sq;
+    wk.qrow0 = (int64_t)b * a.q_sb;
+    wk.orow0 = (int64_t)b * a.o_sb;
+    // keys any row can see: [0, min(seq_len, last row's position + 1))
+    const int hi = min(wk.seq_len, wk.qabs + wk.tq0 + wk.ntok);
+    const int ntiles = hi > 0 ? (hi - 1) / kTile + 1 : 0;
+    // this workgroup's run of key tiles [t0, t1): all of them unless the keys are split
+    const int per = kSplit ? (ntiles + a.nsplit - 1) / a.nsplit : ntiles;
+    wk.t0 = kSplit ? min(ntiles, split * per) : 0;
+    wk.t1 = kSplit ? min(ntiles, wk.t0 + per) : ntiles;
+    wk.part = split;
+    prefill_body<kFast, kExact, kSplit ? 1 : 0, T>(a, wk, lds);
+}
+
+// ---------------------------------------------------------------------------------------
+// Balanced prefill: one launch of a workgroup per CU over every (kv head, query tile) of one or more
+// chunks, the key tiles dealt evenly by the sequence lengths on the device.
+//
+// A query tile sees the keys before it, so the tiles of a fresh prompt need 1, 2, 3, ... key tiles, and
+// chunks of different sequences anything; one workgroup per query tile (or per equal share of its keys) runs as
+// long as the longest and leaves the other CUs idle, and a launch per sequence fills the chip with
+// none of them. As in the batch decode the items lie on a line, each as long as its key tiles and the set-up of a
+// segment (kFaSegmentUnits), and each workgroup takes `share` consecutive units; items that need about the
+// same are cut into ns equal pieces instead. A workgroup that covers all of an item's tiles stores its rows;
+// the pieces of the others go to the workgroup's two slots of the workspace (its first segment, its
+// last), which pd_prefill_merge_kernel adds up. Measured (24 q / 4 kv heads, whole call): a fresh prompt of 4,000
+// tokens 398 us in one workgroup per query tile, 376 in 2 splits, 327 here; 700 tokens over 6,000 keys 207 (2
+// splits) against 184; a batch of 9 decoded sequences and chunks of 70 to 900 tokens over 1,500 to
+// 6,000 keys 481 -> 298 (four launches, with a transpose and two conversions each, before). Where all
+// query tiles need the same (2,048 tokens over 61,440) the splits' kernel is 3 % faster and is taken.
+constexpr unsigned kFaSegmentUnits = 10;  // set-up and stores of a segment, ~16 us, in key tiles (1.62 us)
+constexpr unsigned kFaMinShare = 16;      // units of a workgroup: below, pieces cost more than they save
+constexpr unsigned kFaMaxPieces = 64;     // pieces of an item (the merge holds one per lane)
+
+struct FaLine {
+    unsigned total, per_head, longest, share, ns, lead, snap, nq, nwg;
+    bool aligned;
+    unsigned t0, incl0;  // this lane's query tile (of the first 64): key tiles, units up to and with it
+};
+
+// Sequence and query tile within it of query tile c (of the tiles of all sequences).
+__device__ __forceinline__ void fa_item(const FaParams& a, const FaRowsParams& rows, int c, int& b, int& qt) {
+    if (rows.n == 0) {
+        const int nqt = rows.tiles / rows.first_tile[0];  // (first_tile[0] holds B here)
+        b = c / nqt;
+        qt = c - b * nqt;
+    } else {
+        b = 0;
+        for (int i = 1; i < rows.n; ++i) b += rows.first_tile[i] <= c ? 1 : 0;
+        int first = 0;
+        for (int i = 1; i < rows.n; ++i) first = rows.first_tile[i] <= c ? rows.first_tile[i] : first;
+        qt = c - first;
+    }
+}
+// Tokens of sequence b, and its first row in the rows form.
+__device__ __forceinline__ void fa_tokens(const FaParams& a, const FaRowsParams& rows, int b, int& ntok, int& first) {
+    ntok = a.Sq;
+    first = 0;
+    if (rows.n != 0) {
+        first = rows.first_tok[b];
+        ntok = rows.first_tok[b + 1] - first;
+    }
+}
+__device__ __forceinline__ unsigned fa_units(unsigned t) { return t + kFaSegmentUnits; }
+
+// Key tiles that query tile c sees (uniform or per lane; 0 past the last).
+__device__ __forceinline__ unsigned fa_tiles(const FaParams& a, const FaRowsParams& rows, int c) {
+    int b, qt, ntok, first;
+    fa_item(a, rows, min(c, rows.tiles - 1), b, qt);
+    fa_tokens(a, rows, b, ntok, first);
+    const int seq_len = a.seq_lens[b], qabs = rows.n == 0 ? a.q_abs[b] : seq_len - ntok;
+    const int hi = min(seq_len, qabs + min(ntok, (qt + 1) * a.tok_per_wg));
+    return c < rows.tiles && hi > 0 ? (unsigned)((hi - 1) / kTile + 1) : 0u;
+}
+
+__device__ __forceinline__ FaLine fa_line(const FaParams& a, const FaRowsParams& rows, unsigned hkv, int lane) {
+    FaLine n;
+    n.nq = (unsigned)rows.tiles;
+    n.nwg = (unsigned)rows.nwg;
+    n.t0 = fa_tiles(a, rows, lane);
+    n.incl0 = wave_scan(lane < rows.tiles ? fa_units(n.t0) : 0u);
+    n.per_head = (unsigned)__builtin_amdgcn_readlane((int)n.incl0, 63);
+    n.longest = wave_umax(n.t0);
+    for (int c = 64; c < rows.tiles; c += 64) {
+        const unsigned t = fa_tiles(a, rows, c + lane);
+        n.per_head += (unsigned)__builtin_amdgcn_readlane((int)wave_scan(c + lane < rows.tiles ? fa_units(t) : 0u), 63);
+        n.longest = max(n.longest, wave_umax(t));
+    }
+    n.total = n.per_head * hkv;
+    const unsigned items = n.nq * hkv;
+    // an item reaches into at most ceil(units / share) + 1 <= kFaMaxPieces shares
+    n.share = max(max((n.total + n.nwg - 1) / n.nwg, (fa_units(n.longest) + kFaMaxPieces - 3) / (kFaMaxPieces - 2)), kFaMinShare);
+    n.ns = min(min(n.nwg / items, kFaMaxPieces), max(1u, n.longest / 8));
+    n.aligned = n.nwg >= items && (n.longest + n.ns - 1) / n.ns <= n.share + n.share / 32;
+    n.snap = min(8u, n.share / 8);
+    n.lead = kFaSegmentUnits + n.snap;
+    return n;
+}
+// The query tile of the kv head's line that holds unit `pos` (< per_head), where it starts, and its key tiles.
+__device__ __forceinline__ void fa_locate(const FaParams& a, const FaRowsParams& rows, const FaLine& n, int lane, unsigned pos,
+                                          int& item, unsigned& start, unsigned& tiles) {
+    unsigned before = 0;
+    for (int c = 0;; c += 64) {
+        const unsigned t = c == 0 ? n.t0 : fa_tiles(a, rows, c + lane);
+        const unsigned incl = c == 0 ? n.incl0 : wave_scan(c + lane < rows.tiles ? fa_units(t) : 0u);
+        const int k = __popcll(__ballot(before + incl <= pos));
+        if (k < 64) {
+            item = c + k;
+            tiles = (unsigned)__builtin_amdgcn_readlane((int)t, k);
+            start = before + (unsigned)__builtin_amdgcn_readlane((int)incl, k) - fa_units(tiles);
+            return;
+        }
+        before += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+    }
+}
+// Start of share x of the even split: on an item's start, or past its first `lead` units.
+__device__ __forceinline__ unsigned fa_bound(const FaParams& a, const FaRowsParams& rows, const FaLine& n, int lane, unsigned x) {
+    const unsigned raw = (unsigned)min((uint64_t)x * n.share, (uint64_t)n.total);
+    if (raw == 0 || raw == n.total) return raw;
+    int item;
+    unsigned start, tiles;
+    const unsigned in_head = raw % n.per_head;
+    fa_locate(a, rows, n, lane, in_head, item, start, tiles);
+    const unsigned off = in_head - start, units = fa_units(tiles);
+    if (off <= n.lead) return raw - off;
+    return units - off <= n.snap ? raw + (units - off) : raw;
+}
+
+template <bool kFast, bool kExact, class T>
+__global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_balanced_kernel(const FaParams a, const FaRowsParams rows) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kFaLdsBytes];
+    const int lane = threadIdx.x & 63;
+    const unsigned hkv = (unsigned)(a.Hq / a.G);
+    const FaLine n = fa_line(a, rows, hkv, lane);
+    // workgroups in XCD order (see pd_prefill_kernel): neighbours on the line share an L2
+    const unsigned xcd = blockIdx.x % 8u, wg = xcd * (n.nwg / 8u) + min(xcd, n.nwg % 8u) + blockIdx.x / 8u;
+    unsigned pos = 0, end = 0;
+    if (!n.aligned) {
+        pos = fa_bound(a, rows, n, lane, wg);
+        end = fa_bound(a, rows, n, lane, wg + 1);
+        if (pos >= end) return;
+    } else if (wg >= n.nq * hkv * n.ns) {
+        return;
+    }
+    for (int segment = 0;; ++segment) {
+        FaWork wk;
+        int c;
+        unsigned first, last, tiles, next = 0;
+        if (n.aligned) {
+            const unsigned item = wg / n.ns, piece = wg - item * n.ns;
+            wk.g = (int)(item / n.nq);
+            c = (int)(item - (unsigned)wk.g * n.nq);
+            tiles = (unsigned)__builtin_amdgcn_readfirstlane((int)fa_tiles(a, rows, c));
+            const unsigned per = (tiles + n.ns - 1) / n.ns;
+            first = piece * per;
+            last = min(tiles, first + per);
+            if (piece > 0 && first >= last) return;
+        } else {
+            unsigned start;
+            wk.g = (int)(pos / n.per_head);
+            const unsigned head = (unsigned)wk.g * n.per_head;
+            fa_locate(a, rows, n, lane, pos - head, c, start, tiles);
+            start += head;
+            const unsigned units = fa_units(tiles);
+            first = pos - start <= n.lead ? 0 : pos - start - kFaSegmentUnits;
+            last = end - start >= units ? tiles : end - start - kFaSegmentUnits;
+            next = start + units;
+        }
+        int qt, ntok, row;
+        fa_item(a, rows, c, wk.b, qt);
+        fa_tokens(a, rows, wk.b, ntok, row);
+        wk.seq_len = a.seq_lens[wk.b];
+        wk.qabs = rows.n == 0 ? a.q_abs[wk.b] : wk.seq_len - ntok;
+        wk.tq0 = qt * a.tok_per_wg;
+        wk.ntok = min(a.tok_per_wg, ntok - wk.tq0);
+        wk.qrow0 = rows.n == 0 ? (int64_t)wk.b * a.q_sb : (int64_t)row * a.q_st;
+        wk.orow0 = rows.n == 0 ? (int64_t)wk.b * a.o_sb : (int64_t)row * a.o_st;
+        wk.t0 = (int)first;
+        wk.t1 = (int)last;
+        wk.part = first == 0 && last == tiles ? -1 : (int)(2 * wg) + (segment > 0 ? 1 : 0);
+        prefill_body<kFast, kExact, 2, T>(a, wk, lds);
+        if (n.aligned || last < tiles) return;
+        pos = next;
+        if (pos >= end) return;
+        __syncthreads();  // every wave is done with the block table and the buffers
+    }
+}
+
+// Adds up the pieces of each item that pd_prefill_balanced_kernel cut: grid (items, 48 / kPerWave), a wave per
+// kPerWave rows, lane l owning dims 4 l .. 4 l + 3 (as pd_prefill_combine_kernel). Lane s knows piece s's
+// slot, m and l. Items in one piece have been stored.
+template <class T, int kPerWave>
+__global__ void __launch_bounds__(256) pd_prefill_merge_kernel(const FaParams a, const FaRowsParams rows) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned hkv = (unsigned)(a.Hq / a.G);
+    const FaLine n = fa_line(a, rows, hkv, lane);
+    const int g = (int)(blockIdx.x / n.nq), c = (int)(blockIdx.x - (unsigned)g * n.nq);
+    unsigned pieces, slot;  // slot: of this lane's piece
+    if (n.aligned) {
+        const unsigned tiles = (unsigned)__builtin_amdgcn_readfirstlane((int)fa_tiles(a, rows, c));
+        const unsigned per = max(1u, (tiles + n.ns - 1) / n.ns);
+        pieces = (tiles + per - 1) / per;
+        if (pieces <= 1) return;
+        slot = 2 * (blockIdx.x * n.ns + (unsigned)lane);
+    } else {
+        // this item's place on the line
+        unsigned start = 0, tiles = 0, before = 0;
+        for (int c0 = 0; c0 <= c; c0 += 64) {
+            const unsigned t = c0 == 0 ? n.t0 : fa_tiles(a, rows, c0 + lane);
+            const unsigned incl = c0 == 0 ? n.incl0 : wave_scan(c0 + lane < rows.tiles ? fa_units(t) : 0u);
+            if (c < c0 + 64) {
+                tiles = (unsigned)__builtin_amdgcn_readlane((int)t, c - c0);
+                start = before + (unsigned)__builtin_amdgcn_readlane((int)incl, c - c0) - fa_units(tiles);
+            }
+            before += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+        }
+        start += (unsigned)g * n.per_head;
+        const unsigned units = fa_units(tiles);
+        // its first workgroup (see the balanced decode), and the last whose share starts inside it
+        const unsigned j0 = min(start + n.lead, start + units - 1) / n.share;
+        const unsigned inside = units > n.snap ? (start + units - n.snap + n.share - 1) / n.share - 1 : j0;
+        pieces = inside > j0 ? inside - j0 + 1 : 1;
+        if (pieces <= 1) return;
+        const unsigned later = fa_bound(a, rows, n, lane, j0) == start ? 0u : 1u;  // not its first segment
+        slot = 2 * (j0 + (unsigned)lane) + (lane == 0 ? later : 0u);
+    }
+    int b, qt, ntok, first;
+    fa_item(a, rows, c, b, qt);
+    fa_tokens(a, rows, b, ntok, first);
+    const int nrow = min(a.tok_per_wg, ntok - qt * a.tok_per_wg) * a.G;
+    const int np = (int)pieces;
+#pragma unroll 1
+    for (int i = 0; i < kPerWave; ++i) {
+        const int r = ((int)blockIdx.y * 4 + wave) * kPerWave + i;  // uniform
+        if (r >= nrow) return;
+        const float m_mine = lane < np ? a.part_m[(int64_t)slot * kFaRows + r] : kNegInf;
+        const float l_mine = lane < np ? a.part_l[(int64_t)slot * kFaRows + r] : 0.f;
+        float M = m_mine;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+        const float w_mine = m_mine != kNegInf ? exp2f(m_mine - M) : 0.f;
+        float Lsum = w_mine * l_mine;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) Lsum += __shfl_xor(Lsum, o, 64);
+        float4_t acc = (float4_t)0.f;
+        constexpr int kBatch = 4;
+        for (int s0 = 0; s0 < np; s0 += kBatch) {
+            float4_t o[kBatch];
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const int64_t sl = __builtin_amdgcn_readlane((int)slot, min(s0 + k, np - 1));
+                o[k] = reinterpret_cast<const float4_t*>(a.part_o + (sl * kFaRows + r) * kDim)[lane];
+            }
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const float wk = __shfl(w_mine, min(s0 + k, 63), 64);
+                acc += (s0 + k < np && wk != 0.f) ? wk * o[k] : (float4_t)0.f;
+            }
+        }
+        const float inv = Lsum > 0.f ? 1.f / Lsum : 0.f;
+        const int tok = qt * a.tok_per_wg + r / a.G, head = g * a.G + r % a.G;
+        const int64_t at = (rows.n == 0 ? (int64_t)b * a.o_sb : (int64_t)first * a.o_st) + (int64_t)tok * a.o_st +
+                           (int64_t)head * a.o_sh;
+        store_out4<T>(static_cast<T*>(a.out) + at + 4 * lane, acc * inv);
     }
 }
 
@@ -603,6 +909,7 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
 // reduces M and L, and the O rows are loaded eight splits at a time before any is used, so a
 // row costs about nsplit / 8 memory round trips. A split that saw no key of the row (m = -inf)
 // is excluded by a select, not a product, so whatever its O holds cannot reach the output.
+template <class T>
 __global__ void __launch_bounds__(256) pd_prefill_combine_kernel(const FaParams a, int rows) {
     constexpr int kBatch = 8;
     const int r = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), l = threadIdx.x & 63;
@@ -632,38 +939,78 @@ __global__ void __launch_bounds__(256) pd_prefill_combine_kernel(const FaParams 
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
     const int hd = r % a.Hq, tok = (r / a.Hq) % a.Sq, b = r / (a.Hq * a.Sq);
-    float* orow = a.out + (int64_t)b * a.o_sb + (int64_t)tok * a.o_st + (int64_t)hd * a.o_sh;
-    *reinterpret_cast<float4_t*>(orow + 4 * l) = acc * inv;
+    T* orow = static_cast<T*>(a.out) + (int64_t)b * a.o_sb + (int64_t)tok * a.o_st + (int64_t)hd * a.o_sh;
+    store_out4<T>(orow + 4 * l, acc * inv);
 }
 
 // ---------------------------------------------------------------------------------------
 // host side
 
-template <bool kSplit>
+template <bool kSplit, class T>
 static void launch_prefill_kernel(const FaParams& p, dim3 grid, hipStream_t stream, bool fast, bool exact) {
     const dim3 block(kFaWaves * 64);
     if (fast && !exact)
-        hipLaunchKernelGGL((pd_prefill_kernel<true, false, kSplit>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((pd_prefill_kernel<true, false, kSplit, T>), grid, block, 0, stream, p);
     else if (!exact)
-        hipLaunchKernelGGL((pd_prefill_kernel<false, false, kSplit>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((pd_prefill_kernel<false, false, kSplit, T>), grid, block, 0, stream, p);
     else if (fast)
-        hipLaunchKernelGGL((pd_prefill_kernel<true, true, kSplit>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((pd_prefill_kernel<true, true, kSplit, T>), grid, block, 0, stream, p);
     else
-        hipLaunchKernelGGL((pd_prefill_kernel<false, true, kSplit>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((pd_prefill_kernel<false, true, kSplit, T>), grid, block, 0, stream, p);
 }
 
-hipError_t launch_prefill(const FaParams& p, int batch, int heads_kv, hipStream_t stream, bool exact) {
+template <class T>
+static hipError_t launch_prefill_type(const FaParams& p, int batch, int heads_kv, hipStream_t stream, bool exact) {
     const dim3 grid(((p.Sq + p.tok_per_wg - 1) / p.tok_per_wg) * p.nsplit, heads_kv, batch);
     const bool fast = fast_block_table(p.block_size, p.k_ss);
     if (p.nsplit == 1) {
-        launch_prefill_kernel<false>(p, grid, stream, fast, exact);
+        launch_prefill_kernel<false, T>(p, grid, stream, fast, exact);
         return hipGetLastError();
     }
-    launch_prefill_kernel<true>(p, grid, stream, fast, exact);
+    launch_prefill_kernel<true, T>(p, grid, stream, fast, exact);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int rows = batch * p.Sq * p.Hq;
-    hipLaunchKernelGGL(pd_prefill_combine_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p, rows);
+    hipLaunchKernelGGL((pd_prefill_combine_kernel<T>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p, rows);
+    return hipGetLastError();
+}
+
+hipError_t launch_prefill(const FaParams& p, int batch, int heads_kv, int dtype, hipStream_t stream, bool exact) {
+    return dtype == PD_DTYPE_FP16 ? launch_prefill_type<_Float16>(p, batch, heads_kv, stream, exact)
+                                  : launch_prefill_type<float>(p, batch, heads_kv, stream, exact);
+}
+
+int64_t balanced_prefill_workgroups(int64_t items, int64_t max_keys, int cus) {
+    // pieces of 8 key tiles at the least
+    const int64_t pieces = items * std::max<int64_t>(1, (max_keys + kTile - 1) / kTile / 8);
+    return std::max<int64_t>(1, std::min<int64_t>(cus, pieces));
+}
+
+template <class T>
+static void launch_balanced_type(const FaParams& p, const FaRowsParams& r, int heads_kv, hipStream_t stream, bool exact) {
+    const dim3 grid((unsigned)r.nwg), block(kFaWaves * 64);
+    const bool fast = fast_block_table(p.block_size, p.k_ss);
+    if (fast && !exact)
+        hipLaunchKernelGGL((pd_prefill_balanced_kernel<true, false, T>), grid, block, 0, stream, p, r);
+    else if (!exact)
+        hipLaunchKernelGGL((pd_prefill_balanced_kernel<false, false, T>), grid, block, 0, stream, p, r);
+    else if (fast)
+        hipLaunchKernelGGL((pd_prefill_balanced_kernel<true, true, T>), grid, block, 0, stream, p, r);
+    else
+        hipLaunchKernelGGL((pd_prefill_balanced_kernel<false, true, T>), grid, block, 0, stream, p, r);
+    const unsigned items = (unsigned)(r.tiles * heads_kv);
+    if (items <= 64)  // few items have many pieces each: a row per wave
+        hipLaunchKernelGGL((pd_prefill_merge_kernel<T, 1>), dim3(items, kFaRows / 4), dim3(256), 0, stream, p, r);
+    else
+        hipLaunchKernelGGL((pd_prefill_merge_kernel<T, 4>), dim3(items, kFaRows / 16), dim3(256), 0, stream, p, r);
+}
+
+hipError_t launch_prefill_balanced(const FaParams& p, const FaRowsParams& r, int heads_kv, int dtype, hipStream_t stream,
+                                   bool exact) {
+    if (dtype == PD_DTYPE_FP32)
+        launch_balanced_type<float>(p, r, heads_kv, stream, exact);
+    else
+        launch_balanced_type<_Float16>(p, r, heads_kv, stream, exact);
     return hipGetLastError();
 }
 

@@ -9,11 +9,13 @@
 #include <Python.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <exception>
 
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <ATen/ops/empty.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "pth_dec.h"
@@ -185,6 +187,63 @@ PyObject* prefill_split(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// prefill_balanced(entry, workspace entry, q, key_cache, value_cache, block_table, seq_lens, scale, q_abs_offset, out,
+//                  query_start, max_keys, nsplit, exact): pth_fa_forward_balanced with its workspace from torch's allocator.
+// query_start None: the batch form, with q_abs_offset; a list of row numbers: the rows form. False if the
+// entry does not take such a call.
+PyObject* prefill_balanced(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        decltype(&pth_fa_forward_balanced) fn;
+        decltype(&pth_fa_balanced_workspace) need;
+        pd_tensor t[5], qa{}, od, wd{};
+        double scale;
+        int64_t max_keys, nsplit, exact;
+        if (!count_is(n, 14) || !entry(a[0], fn) || !entry(a[1], need) || !describe_all(a + 2, t, 5) ||
+            !as_double(a[7], scale) || (a[8] != Py_None && !describe(a[8], qa)) || !describe(a[9], od) ||
+            !as_int64(a[11], max_keys) || !as_int64(a[12], nsplit) || !as_int64(a[13], exact))
+            return nullptr;
+        int starts[33];
+        int64_t seqs = 0;
+        const bool rows = a[10] != Py_None;
+        if (rows) {
+            if (!PyList_Check(a[10]) || PyList_GET_SIZE(a[10]) < 2) {
+                PyErr_SetString(PyExc_TypeError, "query_start must be a list of at least two row numbers");
+                return nullptr;
+            }
+            seqs = PyList_GET_SIZE(a[10]) - 1;
+            if (seqs > 32) Py_RETURN_FALSE;
+            for (int64_t i = 0; i <= seqs; ++i) {
+                int64_t v;
+                if (!as_int64(PyList_GET_ITEM(a[10], i), v)) return nullptr;
+                starts[i] = (int)std::max<int64_t>(-1, std::min<int64_t>(v, INT32_MAX));
+            }
+        }
+        const bool shaped = t[0].ndim == (rows ? 3 : 4) && t[1].ndim == 4 && t[3].ndim == 2;
+        OnDevice dev(a[2]);
+        int64_t floats = 0;
+        if (shaped && nsplit == 0)
+            floats = need(rows ? seqs : t[0].sizes[0], rows ? starts : nullptr, rows ? 0 : t[0].sizes[2], t[0].sizes[1],
+                          t[1].sizes[2], max_keys, t[3].sizes[1] * t[1].sizes[1]);
+        else if (shaped && rows)
+            floats = nsplit > 1 ? (starts[1] - starts[0]) * t[0].sizes[1] * nsplit * 258 : 4;
+        if (floats <= 0) Py_RETURN_FALSE;
+        const at::Tensor ws = at::empty({floats}, THPVariable_Unpack(a[2]).options().dtype(at::kFloat));
+        wd.data = ws.data_ptr();
+        wd.dtype = PD_DTYPE_FP32;
+        wd.ndim = 1;
+        wd.sizes[0] = floats;
+        wd.strides[0] = 1;
+        char err[256] = "";
+        int rc;
+        Py_BEGIN_ALLOW_THREADS;
+        rc = fn(&t[0], &t[1], &t[2], &t[3], &t[4], scale, a[8] == Py_None ? nullptr : &qa, rows ? starts : nullptr, seqs, &od,
+                &wd, max_keys, nsplit, exact, dev.stream, err, (int)sizeof err);
+        Py_END_ALLOW_THREADS;
+        if (rc != 0) return done(rc, err);
+        Py_RETURN_TRUE;
+    });
+}
+
 // cache_write(entry, key, value, key_cache, value_cache, k_scale, v_scale, slot_mapping)
 PyObject* cache_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
@@ -256,12 +315,17 @@ PyObject* plan_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // plan_prefill(work_items, rows, max_keys, block_size, cus, tile_us, wg_us, mb_us, merge_us, max_splits, min_tiles,
-//              max_workspace, lds_table, global_factor): pth_dec.prefill_splits' makespan model.
+//              max_workspace, lds_table, global_factor, sq, tok_per_wg): pth_dec.prefill_splits' makespan model. With sq > 0
+// (the chunk's query tokens, the last of max_keys keys) 0 where the balanced launch is rated at least 5 %
+// faster: a workgroup's share of the line and, measured, up to 20 more units (a share's ends fall on items' starts, and
+// its last segment's set-up is its own) of 1.72 us, plus 20 us of planning and merge. Equal query tiles
+// (the kernel's aligned split) stay with the splits, whose kernel takes 3 % less per tile.
 PyObject* plan_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         int64_t v[5], max_splits, min_tiles, max_workspace, lds_table;
         double tile_us, wg_us, mb_us, merge_us, factor;
-        if (!count_is(n, 14)) return nullptr;
+        int64_t sq, tok;
+        if (!count_is(n, 16) || !as_int64(a[14], sq) || !as_int64(a[15], tok)) return nullptr;
         for (int i = 0; i < 5; ++i)
             if (!as_int64(a[i], v[i])) return nullptr;
         if (!as_double(a[5], tile_us) || !as_double(a[6], wg_us) || !as_double(a[7], mb_us) || !as_double(a[8], merge_us) ||
@@ -284,6 +348,14 @@ PyObject* plan_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
             const double t = cost(s);
             if (t < best_t) best = s, best_t = t;
         }
+        if (sq > 0 && items > 0) {
+            const int64_t nqt = ceil_div(sq, std::max<int64_t>(1, tok)), heads = items / nqt;
+            int64_t units = 0;
+            for (int64_t q = 0; q < nqt; ++q) units += ceil_div(std::max<int64_t>(0, keys - sq) + std::min(sq, (q + 1) * tok), 32) + 10;
+            const int64_t share = std::max<int64_t>(16, ceil_div(units * heads, cus)), ns = items <= cus ? cus / items : 0;
+            const bool aligned = ns > 0 && ceil_div(tiles, ns) <= share + share / 32;
+            if (!aligned && 1.72 * (double)(share + 20) + 20.0 < 0.95 * best_t) best = 0;
+        }
         return PyLong_FromLongLong(best);
     });
 }
@@ -293,6 +365,7 @@ PyMethodDef methods[] = {
     PD_METHOD(decode, "pth_dec_decode on torch tensors"),
     PD_METHOD(prefill, "pth_fa_forward / pth_fa_forward_exact on torch tensors"),
     PD_METHOD(prefill_split, "pth_fa_forward_split on torch tensors"),
+    PD_METHOD(prefill_balanced, "pth_fa_forward_balanced on torch tensors"),
     PD_METHOD(cache_write, "pth_cache_write on torch tensors"),
     PD_METHOD(plan_decode, "split count of a decode batch"),
     PD_METHOD(plan_prefill, "key splits of a prefill launch"),

@@ -120,6 +120,33 @@ __device__ __forceinline__ void split_fp16x2(float p0, float s0, float p1, float
 __device__ __forceinline__ float xor_max(float v, int mask) { return fmaxf(v, __shfl_xor(v, mask, 64)); }
 __device__ __forceinline__ float xor_sum(float v, int mask) { return v + __shfl_xor(v, mask, 64); }
 
+// DPP move with 0 in lanes that have no source (kRows: the 16-lane rows that take part).
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ unsigned dpp_or_zero(unsigned v) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xf, false);
+}
+// Inclusive sum over the lanes: shifts inside 16-lane rows, then the last lane of row 0 into row 1 and of row
+// 2 into row 3, then the last lane of the lower half into the upper.
+__device__ __forceinline__ unsigned wave_scan(unsigned v) {
+    v += dpp_or_zero<0x111>(v);       // row_shr:1
+    v += dpp_or_zero<0x112>(v);       // row_shr:2
+    v += dpp_or_zero<0x114>(v);       // row_shr:4
+    v += dpp_or_zero<0x118>(v);       // row_shr:8
+    v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15
+    v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31
+    return v;
+}
+// Largest value of the wave, uniform (the same steps; the last lane has seen every other).
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+    v = max(v, dpp_or_zero<0x111>(v));
+    v = max(v, dpp_or_zero<0x112>(v));
+    v = max(v, dpp_or_zero<0x114>(v));
+    v = max(v, dpp_or_zero<0x118>(v));
+    v = max(v, dpp_or_zero<0x142, 0xa>(v));
+    v = max(v, dpp_or_zero<0x143, 0xc>(v));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // Block-table access of one workgroup: the slice of pages its split can touch is staged in
 // LDS when it fits (kBtCache entries), so the tile loop issues no loads of its own besides the
 // K/V rows; otherwise entries are read with scalar loads through the constant address space.

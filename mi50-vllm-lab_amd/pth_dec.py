@@ -54,6 +54,8 @@ EXPORTED_SYMBOLS = (
     "pth_fa_forward",
     "pth_fa_forward_exact",
     "pth_fa_forward_split",
+    "pth_fa_forward_balanced",
+    "pth_fa_balanced_workspace",
     "pth_cache_write",
 )
 
@@ -131,13 +133,18 @@ def load_library(path: str | None = None) -> ctypes.CDLL:
     lib.pth_fa_forward_split.argtypes = [tp] * 5 + [c_double, tp, tp, tp, ctypes.c_int64, ctypes.c_int64, vp,
                                                     ctypes.c_char_p, c_int]
     lib.pth_fa_forward_split.restype = c_int
+    lib.pth_fa_forward_balanced.argtypes = [tp] * 5 + [c_double, tp, ip, ctypes.c_int64, tp, tp, ctypes.c_int64,
+                                                       ctypes.c_int64, ctypes.c_int64, vp, ctypes.c_char_p, c_int]
+    lib.pth_fa_forward_balanced.restype = c_int
+    lib.pth_fa_balanced_workspace.argtypes = [ctypes.c_int64, ip] + [ctypes.c_int64] * 5
+    lib.pth_fa_balanced_workspace.restype = ctypes.c_int64
     lib.pth_cache_write.argtypes = [tp] * 7 + [vp, ctypes.c_char_p, c_int]
     lib.pth_cache_write.restype = c_int
     lib.pth_dec_version.argtypes = []
     lib.pth_dec_version.restype = ctypes.c_char_p
     _entries.update({name: ctypes.cast(getattr(lib, name), vp).value
                      for name in ("pth_dec_decode", "pth_fa_forward", "pth_fa_forward_exact", "pth_fa_forward_split",
-                                  "pth_cache_write")})
+                                  "pth_fa_forward_balanced", "pth_fa_balanced_workspace", "pth_cache_write")})
     _lib, _lib_path = lib, os.path.realpath(p)
     return lib
 
@@ -246,12 +253,17 @@ def prefill_splits(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: i
     the keys a row can see; the device splits each row's actual keys evenly."""
     if batch <= 0 or sq <= 0 or heads_q <= 0 or heads_kv <= 0:
         return 1
-    g = max(1, heads_q // heads_kv)
-    qtiles = -(-sq // max(1, PREFILL_ROWS_PER_WORKGROUP // g))
-    return native().plan_prefill(qtiles * heads_kv * batch, batch * sq * heads_q, max_keys, block_size, PREFILL_CUS,
+    return _prefill_plan(batch, sq, heads_q, heads_kv, max_keys, block_size, 0)
+
+
+def _prefill_plan(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: int, block_size: int, chunk: int) -> int:
+    """prefill_splits' count; with chunk = sq (query tokens that are the last of max_keys keys) 0 where the
+    balanced launch is rated faster."""
+    tok = max(1, PREFILL_ROWS_PER_WORKGROUP // max(1, heads_q // heads_kv))
+    return native().plan_prefill(-(-sq // tok) * heads_kv * batch, batch * sq * heads_q, max_keys, block_size, PREFILL_CUS,
                                  PREFILL_US_PER_TILE, PREFILL_US_PER_WORKGROUP, PREFILL_US_PER_PARTIAL_MB,
                                  PREFILL_US_MERGE_LAUNCH, PREFILL_MAX_SPLITS, PREFILL_MIN_TILES_PER_SPLIT,
-                                 PREFILL_MAX_WORKSPACE, PREFILL_LDS_TABLE, PREFILL_GLOBAL_TABLE_FACTOR)
+                                 PREFILL_MAX_WORKSPACE, PREFILL_LDS_TABLE, PREFILL_GLOBAL_TABLE_FACTOR, chunk, tok)
 
 
 def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, block_table: torch.Tensor,
@@ -267,11 +279,11 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
     the widening bias and P' as fp16 hi + lo, for caches with very large scales (outlier
     tokens), at about twice the P.V matrix work.
     nsplit: key splits per query tile (pth_fa_forward_split, no counterpart in the reference);
-    None picks them with prefill_splits (1 for chunks that fill the GPU), and a workspace for the
-    partials is taken from torch's allocator.
+    None picks them with prefill_splits (1 for chunks that fill the GPU), or deals the key tiles evenly
+    over the GPU (pth_fa_forward_balanced) where that is rated faster: chunks whose query tiles see
+    very different numbers of keys. A workspace for the partials is taken from torch's allocator.
     max_keys: a host-side bound on the keys any row of the batch sees (the longest seq_len), used
-    only to pick nsplit; None takes the block table's width in keys, which for a table sized to
-    the model's maximum length plans every chunk for the longest context.
+    only to size the launch; None takes the block table's width in keys.
     """
     if not q.is_cuda:
         raise RuntimeError("q must be contiguous fp32 [B, Hq, Sq, D]")
@@ -280,8 +292,16 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
     if nsplit is None:
         if max_keys is None:
             max_keys = block_table.shape[1] * key_cache.shape[1] if block_table.dim() == 2 else 0
-        nsplit = prefill_splits(q.shape[0], q.shape[2], q.shape[1], key_cache.shape[2], int(max_keys),
-                                key_cache.shape[1] if key_cache.dim() == 4 else 16)
+        batch, heads_q, sq, heads_kv = q.shape[0], q.shape[1], q.shape[2], key_cache.shape[2]
+        nsplit = 1
+        if batch > 0 and sq > 0 and heads_q > 0 and heads_kv > 0:
+            block_size = key_cache.shape[1] if key_cache.dim() == 4 else 16
+            nsplit = _prefill_plan(batch, sq, heads_q, heads_kv, int(max_keys), block_size, sq)
+            if nsplit == 0 and native().prefill_balanced(
+                    _entry("pth_fa_forward_balanced"), _entry("pth_fa_balanced_workspace"), q, key_cache, value_cache,
+                    block_table, seq_lens, scale, q_abs_offset, out, None, int(max_keys), 0, 1 if exact else 0):
+                return out
+            nsplit = nsplit or prefill_splits(batch, sq, heads_q, heads_kv, int(max_keys), block_size)
     if nsplit > 1:
         ws = torch.empty((q.shape[0] * q.shape[2] * q.shape[1] * nsplit * (q.shape[3] + 2),), dtype=torch.float32,
                          device=q.device)
@@ -291,6 +311,28 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
         native().prefill(_entry("pth_fa_forward_exact" if exact else "pth_fa_forward"), q, key_cache, value_cache,
                          block_table, seq_lens, scale, q_abs_offset, out)
     return out
+
+
+def forward_rows(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, block_table: torch.Tensor,
+                 seq_lens: torch.Tensor, scale: float, query_start: list, out: torch.Tensor, max_keys: int,
+                 exact: bool = False) -> bool:
+    """Causal prefill of several sequences as an engine holds them: sequence i has rows [query_start[i],
+    query_start[i + 1]) of query and out (fp16 [T, Hq, 256]), the last tokens of its seq_lens[i] keys
+    (pth_fa_forward_balanced's rows form; no counterpart in the reference). Numerics are forward_pth's.
+    Returns False, with nothing launched, for calls beyond the entry's limits (over 32 sequences, other
+    dtypes or alignments); query_start is a list, max_keys a bound on the keys any row sees.
+    """
+    if not (query.is_cuda and query.dtype == torch.float16 and out.dtype == torch.float16 and query.dim() == 3
+            and out.dim() == 3 and key_cache.dim() == 4 and query.stride(2) == 1 and out.stride(2) == 1 and query.stride(0) % 8 == 0 and query.stride(1) % 8 == 0
+            and query.data_ptr() % 16 == 0 and out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0
+            and out.data_ptr() % 8 == 0):
+        return False
+    nsplit, rows, heads_kv = 0, query_start[-1] - query_start[0], key_cache.shape[2]
+    if len(query_start) == 2 and rows > 0 and heads_kv > 0 and query.shape[1] > 0:
+        nsplit = _prefill_plan(1, rows, query.shape[1], heads_kv, max_keys, key_cache.shape[1], rows)
+    return native().prefill_balanced(_entry("pth_fa_forward_balanced"), _entry("pth_fa_balanced_workspace"), query,
+                                     key_cache, value_cache, block_table, seq_lens, scale, None, out, query_start,
+                                     max_keys, nsplit, 1 if exact else 0)
 
 
 def cache_write(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,

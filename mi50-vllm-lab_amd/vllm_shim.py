@@ -20,8 +20,9 @@ few fields the routing reads.
   sequences), so that the partial kernel runs in a single round.
 - forward_pth_fa (triton_attn.patch:176-262): the sequences with >= MIN_Q query tokens must form
   a suffix of the batch; the rows before it go to the decode operator when every prefix sequence
-  has <= 4 (8 with DFlash) query tokens, else to the caller's Triton function. Each suffix
-  sequence runs the prefill operator once (no padding to a tile ladder is needed);
+  has <= 4 (8 with DFlash) query tokens, else to the caller's Triton function. fp16 batches of up
+  to 32 suffix sequences run in one launch on the query and output rows as they are (forward_rows),
+  others each through the prefill operator (no padding to a tile ladder is needed);
   VLLM_GFX950_PTH_FA_EXACT=1 selects its exact entry (pth_fa_forward_exact: the decode's
   numerics, for caches with very large per-token scales, at ~26 % more time).
 - route (triton_attn.patch:272-308): prefill first when max_seqlen_q >= MIN_Q, then decode
@@ -151,6 +152,7 @@ class _Operators:
         self.supported_layout = _pd.supported_layout
         self.decode = _pd.decode
         self.forward_pth = _pd.forward_pth
+        self.forward_rows = _pd.forward_rows
 
 
 def _load(env_switch: str, env_lib: str, what: str):
@@ -289,6 +291,15 @@ class Gfx950Int8Attention:
         # model's maximum length, so the table alone would plan every chunk for the longest context),
         # else the batch's max_seq_len, else the table width.
         lens_host = meta.seq_lens_cpu if meta.seq_lens_cpu is not None and not _capturing(query.device) else None
+        # All sequences in one launch that reads the query rows and writes the output rows as they are; the
+        # calls it does not take go one by one through forward_pth.
+        rows = getattr(self.pth_fa, "forward_rows", None)
+        if rows is not None:
+            keys = (max(int(x) for x in lens_host[p:n]) if lens_host is not None else int(meta.max_seq_len)) or \
+                meta.block_table.shape[1] * key_cache.shape[1]
+            if rows(query, key_cache, value_cache, meta.block_table[p:n], meta.seq_lens[p:n], self.scale, qsl[p:], output,
+                    keys, PTH_FA_EXACT):
+                return True
         for i in range(p, n):
             start, nq = qsl[i], qsl[i + 1] - qsl[i]
             q = query[start:start + nq].transpose(0, 1).unsqueeze(0).float().contiguous()  # [1, Hq, nq, D]
