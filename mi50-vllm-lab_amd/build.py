@@ -21,7 +21,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libpthdec.so")
 NATIVE_PATH = os.path.join(LIB_DIR, "pd_native.so")
 # the C ABI, then the kernels (each file compiles on its own; they share csrc/pd_*.hpp)
 SOURCES = [os.path.join(HERE, "csrc", f) for f in
-           ("pd_api.hip", "pd_decode.hip", "pd_prefill.hip", "pd_cache_write.hip")]
+           ("pd_api.hip", "pd_decode.hip", "pd_prefill.hip", "pd_prefill_wide.hip",
+            "pd_cache_write.hip")]
 KERNEL_SOURCES = SOURCES[1:]
 ARCH = "gfx950"
 

@@ -19,6 +19,7 @@ constexpr int64_t kSliceKeys = 16384; // decode: largest sequences x window whos
 constexpr int kFaWaves = 4;
 constexpr int kFaRB = 3;                        // row blocks per wave
 constexpr int kFaRows = kFaWaves * kFaRB * 16;  // 192
+constexpr int kFwRows = 256;                    // query rows (token, head) of a workgroup of pd_prefill_wide_kernel
 
 // Split-K decode, partial pass (pd_partial_kernel).
 struct PartialParams {
@@ -151,6 +152,8 @@ hipError_t scratch_address(void** out);
 // exact: K converted to fp16 without the widening bias and P' as fp16 hi + lo (pth_fa_forward_exact)
 // dtype: PD_DTYPE_FP32 or _FP16 of q and out
 hipError_t launch_prefill(const FaParams& p, int batch, int heads_kv, int dtype, hipStream_t stream, bool exact);
+// its 256-row kernel (pd_prefill_wide.hip), without the merge of the splits
+hipError_t launch_prefill_wide(const FaParams& p, int batch, int heads_kv, int dtype, hipStream_t stream, bool exact);
 // the same with the key tiles of all query tiles dealt evenly over r.nwg workgroups; dtype: of q and
 // out (fp32 in the batch form, fp16 in the rows form); partials in p.part_o/m/l (2 slots of kFaRows rows
 // per workgroup)

@@ -80,28 +80,6 @@ __device__ __forceinline__ void wait_quarters(int later, bool tail) {
     }
 }
 
-// Eight consecutive query values as fp16. Q is rounded to fp16 unscaled: fp16-valued queries enter the
-// matrix cores exactly.
-template <class T>
-__device__ __forceinline__ half8_t load_q8(const T* p) {
-    if constexpr (sizeof(T) == 4) {
-        const float4_t x0 = *reinterpret_cast<const float4_t*>(p), x1 = *reinterpret_cast<const float4_t*>(p + 4);
-        return half8_t{(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w,
-                       (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
-    } else {
-        return *reinterpret_cast<const half8_t*>(p);
-    }
-}
-template <class T>
-__device__ __forceinline__ void store_out4(T* p, float4_t v) {
-    if constexpr (sizeof(T) == 4) {
-        *reinterpret_cast<float4_t*>(p) = v;
-    } else {
-        typedef T out4_t __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<out4_t*>(p) = out4_t{(T)v.x, (T)v.y, (T)v.z, (T)v.w};
-    }
-}
-
 // LDS of a prefill workgroup: raw ring, two fp16 buffers, block table.
 constexpr int kFaLdsH = kFaRaw * kSlot;
 constexpr int kFaLdsBt = kFaLdsH + 2 * kFaHBuf;
@@ -963,13 +941,29 @@ template <class T>
 static hipError_t launch_prefill_type(const FaParams& p, int batch, int heads_kv, hipStream_t stream, bool exact) {
     const dim3 grid(((p.Sq + p.tok_per_wg - 1) / p.tok_per_wg) * p.nsplit, heads_kv, batch);
     const bool fast = fast_block_table(p.block_size, p.k_ss);
+    // 256-row workgroups where they take less time for all rounds of one workgroup per CU: a tile of theirs takes
+    // 1.85 us (2.2 exact) against 1.62 (1.9), so they have to save a round (2,048 tokens x 4 splits, 24 q / 4 kv heads:
+    // 3 rounds of 256 against 4, 2.92 ms against 3.30; 2,048 unsplit: one round of either, 3.7 against 3.15)
+    const int64_t cus = std::max(1, compute_units(stream)), each = (int64_t)p.nsplit * heads_kv * batch;
+    const int64_t rounds = ((int64_t)((p.Sq + p.tok_per_wg - 1) / p.tok_per_wg) * each + cus - 1) / cus;
+    const int64_t wide_rounds = (((int64_t)p.Sq * p.G + kFwRows - 1) / kFwRows * each + cus - 1) / cus;
+    const bool wide = (double)wide_rounds * (exact ? 2.2 / 1.9 : 1.85 / 1.62) < (double)rounds;
     if (p.nsplit == 1) {
+        if (wide)
+            return launch_prefill_wide(p, batch, heads_kv, std::is_same<T, float>::value ? PD_DTYPE_FP32 : PD_DTYPE_FP16,
+                                       stream, exact);
         launch_prefill_kernel<false, T>(p, grid, stream, fast, exact);
         return hipGetLastError();
     }
-    launch_prefill_kernel<true, T>(p, grid, stream, fast, exact);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (wide) {
+        const hipError_t e = launch_prefill_wide(p, batch, heads_kv, std::is_same<T, float>::value ? PD_DTYPE_FP32 : PD_DTYPE_FP16,
+                                                 stream, exact);
+        if (e != hipSuccess) return e;
+    } else {
+        launch_prefill_kernel<true, T>(p, grid, stream, fast, exact);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     const int rows = batch * p.Sq * p.Hq;
     hipLaunchKernelGGL((pd_prefill_combine_kernel<T>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p, rows);
     return hipGetLastError();

@@ -315,17 +315,17 @@ PyObject* plan_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // plan_prefill(work_items, rows, max_keys, block_size, cus, tile_us, wg_us, mb_us, merge_us, max_splits, min_tiles,
-//              max_workspace, lds_table, global_factor, sq, tok_per_wg): pth_dec.prefill_splits' makespan model. With sq > 0
+//              max_workspace, lds_table, global_factor, sq, tok_per_wg, rows per kv head): pth_dec.prefill_splits' makespan model. With sq > 0
 // (the chunk's query tokens, the last of max_keys keys) 0 where the balanced launch is rated at least 5 %
 // faster: a workgroup's share of the line and, measured, up to 20 more units (a share's ends fall on items' starts, and
 // its last segment's set-up is its own) of 1.72 us, plus 20 us of planning and merge. Equal query tiles
 // (the kernel's aligned split) stay with the splits, whose kernel takes 3 % less per tile.
 PyObject* plan_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
-        int64_t v[5], max_splits, min_tiles, max_workspace, lds_table;
+        int64_t v[6], max_splits, min_tiles, max_workspace, lds_table;
         double tile_us, wg_us, mb_us, merge_us, factor;
         int64_t sq, tok;
-        if (!count_is(n, 16) || !as_int64(a[14], sq) || !as_int64(a[15], tok)) return nullptr;
+        if (!count_is(n, 17) || !as_int64(a[14], sq) || !as_int64(a[15], tok) || !as_int64(a[16], v[5])) return nullptr;
         for (int i = 0; i < 5; ++i)
             if (!as_int64(a[i], v[i])) return nullptr;
         if (!as_double(a[5], tile_us) || !as_double(a[6], wg_us) || !as_double(a[7], mb_us) || !as_double(a[8], merge_us) ||
@@ -349,6 +349,15 @@ PyObject* plan_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
             if (t < best_t) best = s, best_t = t;
         }
         if (sq > 0 && items > 0) {
+            // the 256-row kernel, which the launch takes where that saves rounds: 1.85 us per tile
+            const int64_t wide_items = ceil_div(v[5], 256) * (items / ceil_div(sq, std::max<int64_t>(1, tok)));
+            for (int64_t s = 1; s <= top && (s == 1 || rows * s * 1032 <= max_workspace); ++s) {
+                const int64_t rounds = ceil_div(wide_items * s, cus), per = ceil_div(tiles, s);
+                if ((double)rounds * (1.85 / 1.62) >= (double)ceil_div(items * s, cus)) continue;
+                double t = (double)rounds * ((double)per * 1.85 + wg_us);
+                if (s > 1) t += merge_us + mb_us * (double)rows * (double)s * 1032 / 1e6;
+                if (t < best_t) best = s, best_t = t;
+            }
             const int64_t nqt = ceil_div(sq, std::max<int64_t>(1, tok)), heads = items / nqt;
             int64_t units = 0;
             for (int64_t q = 0; q < nqt; ++q) units += ceil_div(std::max<int64_t>(0, keys - sq) + std::min(sq, (q + 1) * tok), 32) + 10;

@@ -95,6 +95,28 @@ __device__ __forceinline__ half8_t widen_i8x8_exact(unsigned w0, unsigned w1) {
     return __builtin_bit_cast(half8_t, h);
 }
 
+// Eight consecutive query values as fp16. Q is rounded to fp16 unscaled: fp16-valued queries enter the
+// matrix cores exactly.
+template <class T>
+__device__ __forceinline__ half8_t load_q8(const T* p) {
+    if constexpr (sizeof(T) == 4) {
+        const float4_t x0 = *reinterpret_cast<const float4_t*>(p), x1 = *reinterpret_cast<const float4_t*>(p + 4);
+        return half8_t{(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w,
+                       (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
+    } else {
+        return *reinterpret_cast<const half8_t*>(p);
+    }
+}
+template <class T>
+__device__ __forceinline__ void store_out4(T* p, float4_t v) {
+    if constexpr (sizeof(T) == 4) {
+        *reinterpret_cast<float4_t*>(p) = v;
+    } else {
+        typedef T out4_t __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<out4_t*>(p) = out4_t{(T)v.x, (T)v.y, (T)v.z, (T)v.w};
+    }
+}
+
 // x = p * s as two fp16 parts, hi + lo with ~22 significant bits: hi is the fp32 product rounded
 // to fp16, lo = fp16(p * s - hi) with the product exact (fma). hi must be the same value in both
 // places. The fp32 product is therefore pinned in a register: left to itself the compiler folds

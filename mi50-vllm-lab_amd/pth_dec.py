@@ -263,7 +263,8 @@ def _prefill_plan(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: in
     return native().plan_prefill(-(-sq // tok) * heads_kv * batch, batch * sq * heads_q, max_keys, block_size, PREFILL_CUS,
                                  PREFILL_US_PER_TILE, PREFILL_US_PER_WORKGROUP, PREFILL_US_PER_PARTIAL_MB,
                                  PREFILL_US_MERGE_LAUNCH, PREFILL_MAX_SPLITS, PREFILL_MIN_TILES_PER_SPLIT,
-                                 PREFILL_MAX_WORKSPACE, PREFILL_LDS_TABLE, PREFILL_GLOBAL_TABLE_FACTOR, chunk, tok)
+                                 PREFILL_MAX_WORKSPACE, PREFILL_LDS_TABLE, PREFILL_GLOBAL_TABLE_FACTOR, chunk, tok,
+                                 sq * (heads_q // heads_kv))
 
 
 def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, block_table: torch.Tensor,
