@@ -123,8 +123,8 @@ def summarize_counters(args):
     """Instruction mix and MFMA utilisation per kernel launch from one rocprofv3 --pmc run with
     COUNTERS (medians over the dispatches), per wave and per 32-key tile: the decode partial kernel
     of --profile-only (--counters-kernel partial; a tile is one wave's 32 keys) or the config-5
-    prefill kernel of --profile-prefill (--counters-kernel prefill; a tile is 32 keys that every
-    wave of a workgroup computes for its 48 rows, counted once per wave)."""
+    prefill kernel of --profile-prefill (--counters-kernel prefill, the 256-row kernel; a tile is 32
+    keys that every wave of a workgroup computes for its 64 rows, counted once per wave)."""
     kind = args.counters_kernel
     per = {c: _pmc_dispatches(args.counters_summary, c) for c in COUNTERS}
     med = {}
@@ -141,10 +141,9 @@ def summarize_counters(args):
         what = {"kernel": "decode partial kernel", "workload": "MTP verify 4 x 24/4 heads, ctx 61440+4, bs 16",
                 "nsplit": args.nsplit}
     else:
-        # workgroup q of a kv head: tokens [32 q, 32 q + 32) of the chunk, keys [0, ctx + 32 q + 32)
-        tpw = 192 // 6
-        tiles = 4 * sum(-(-min(PREFILL_CTX + PREFILL_CHUNK, PREFILL_CTX + tpw * (q + 1)) // 32)
-                        for q in range(PREFILL_CHUNK // tpw))
+        # workgroup q of a kv head: rows (token x 6 heads) [256 q, 256 q + 256) of the chunk, keys up to the
+        # last row's token; the key splits share these tiles
+        tiles = 4 * sum(-(-(PREFILL_CTX + (256 * q + 255) // 6 + 1) // 32) for q in range(PREFILL_CHUNK * 6 // 256))
         tiles *= 4  # each of the 4 waves computes every tile of its workgroup
         what = {"kernel": "chunked prefill kernel", "workload": DESCRIPTIONS[5]}
     waves = med["SQ_WAVES"]
@@ -655,8 +654,8 @@ def bench_prefill(torch, wl, pd, dev, stream, reps=20, exact_too=True):
 
 def bench_short_prefill(torch, wl, pd, dev, stream, sq, reps=200):
     """A chunk of sq tokens over the same 61,440 cached tokens, with the key split that forward_pth
-    picks (pth_fa_forward_split): 64 tokens give too few query tiles to fill the GPU, 2,560 give
-    320 workgroups, which unsplit would run as one full round and one part-filled round."""
+    picks (0: dealt evenly, pth_fa_forward_balanced): 64 tokens give too few query tiles to fill the
+    GPU, 2,560 give 320 workgroups of 192 rows (two rounds) or 240 of 256 rows (one)."""
     ctx = PREFILL_CTX
     case = wl.make_case([ctx], [sq], num_q_heads=24, num_kv_heads=4, block_size=16, seed=1005)
     flops = wl.prefill_flops([ctx + sq], [ctx], sq, 24)
@@ -665,11 +664,12 @@ def bench_short_prefill(torch, wl, pd, dev, stream, sq, reps=200):
     q = wl.prefill_query(d)
     qa = torch.tensor([ctx], dtype=torch.int32, device=dev)
     out = torch.empty((1, sq, 24, 256), dtype=torch.float32, device=dev)
-    nsplit = pd.prefill_splits(1, sq, 24, 4, d.block_table.shape[1] * 16)
+    keys = d.block_table.shape[1] * 16
+    nsplit = pd._prefill_plan(1, sq, 24, 4, keys, 16, sq)
 
     def timed(ns, n):
         ops = [lambda c=c: pd.forward_pth(q, c.key_cache, c.value_cache, d.block_table, d.seq_lens, d.scale, qa,
-                                          out=out, nsplit=ns) for c in caches]
+                                          out=out, nsplit=ns, max_keys=keys) for c in caches]
         with torch.cuda.stream(stream):
             for o in ops:
                 o()
@@ -679,7 +679,7 @@ def bench_short_prefill(torch, wl, pd, dev, stream, sq, reps=200):
             g.replay()
             return time_replays(torch, g, n // 2, stream) / n
 
-    ms = timed(nsplit, reps)
+    ms = timed(None, reps)
     ms1 = timed(1, max(2, reps // 20))
     kv = (ctx + sq) * 4 * 520
     return {"tokens": sq, "nsplit": nsplit, "ms_per_chunk": round(ms, 4),
@@ -708,11 +708,11 @@ def bench_prefill_grid(torch, wl, pd, dev, stream, hq, hkv, block_size, reps=20)
         qa = torch.tensor([ctx], dtype=torch.int32, device=dev)
         out = torch.empty((1, sq, hq, 256), dtype=torch.float32, device=dev)
         flops = 4 * 256 * hq * (sq * ctx + sq * (sq + 1) // 2)
-        pick = pd.prefill_splits(1, sq, hq, hkv, ctx + sq, block_size)
+        pick = pd._prefill_plan(1, sq, hq, hkv, ctx + sq, block_size, sq)
 
         def timed(ns, n):
             ops = [lambda c=c: pd.forward_pth(q, c.key_cache, c.value_cache, d.block_table, d.seq_lens, d.scale, qa,
-                                              out=out, nsplit=ns) for c in caches]
+                                              out=out, nsplit=ns, max_keys=ctx + sq) for c in caches]
             with torch.cuda.stream(stream):
                 for o in ops:
                     o()
@@ -723,7 +723,7 @@ def bench_prefill_grid(torch, wl, pd, dev, stream, hq, hkv, block_size, reps=20)
                 return time_replays(torch, g, n // 2, stream) / n
 
         n = reps if ctx <= 65536 else max(4, reps // 2)
-        ms = timed(pick, n)
+        ms = timed(None, n)
         ms1 = ms if pick == 1 else timed(1, n)
         mi50 = PREFILL_GRID_MI50_MS[ctx]
         print(json.dumps({"prefill_grid": True, "heads_q": hq, "heads_kv": hkv, "block_size": block_size,

@@ -8,8 +8,10 @@
 //                the tile's scales) into one of two fp16 buffers while it computes tile n;
 //   MFMA         S^T = K Q^T and O^T += V^T P^T on fp16 MFMA with fp32 accumulation, Q held in
 //                registers, K and V operands read from the fp16 buffer.
-// One barrier per tile orders the three stages. There is no split: each row is normalised in
-// registers and stored once. Q arrives as fp32 and is rounded to fp16 for the MFMA.
+// One barrier per tile orders the three stages. Unsplit, each row is normalised in registers and
+// stored once; a split (pd_prefill_kernel<.., kParts>) or dealt (pd_prefill_balanced_kernel) tile
+// stores its partial sums, which a second launch merges. Q arrives as fp32, rounded to fp16 for the
+// MFMA, or as fp16. Launches that 256-row workgroups finish sooner run pd_prefill_wide_kernel.
 // kExact (pth_fa_forward_exact) gives the decode kernel's numerics: K and V are widened without
 // the bias (so the fp32 accumulators hold only the products' own sums) and P' enters the P.V
 // products as fp16 hi + lo, which doubles them. The default instance keeps the bias in K and V

@@ -243,7 +243,7 @@ def prefill_cost_us(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: 
 
 
 def prefill_splits(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: int, block_size: int = 16) -> int:
-    """Key splits per query tile for a prefill launch: the count in 1..64 that minimises
+    """Key splits per query tile for a prefill launch of 192-row workgroups: the count in 1..64 that minimises
     prefill_cost_us, with at least 8 key tiles (256 keys) of max_keys per split and at most 1 GiB
     of partials. Splitting pays where the query tiles alone leave CUs idle: short chunks (a 64-token
     chunk over 61k keys: 32 splits) and chunks whose workgroups end in a part-filled round (2,560
@@ -280,9 +280,10 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
     the widening bias and P' as fp16 hi + lo, for caches with very large scales (outlier
     tokens), at about twice the P.V matrix work.
     nsplit: key splits per query tile (pth_fa_forward_split, no counterpart in the reference);
-    None picks them with prefill_splits (1 for chunks that fill the GPU), or deals the key tiles evenly
-    over the GPU (pth_fa_forward_balanced) where that is rated faster: chunks whose query tiles see
-    very different numbers of keys. A workspace for the partials is taken from torch's allocator.
+    None picks them as prefill_splits does, counting the 256-row kernel as well (2,048 tokens over 61k
+    keys: 4 splits of it, 2,560: one round unsplit), or deals the key tiles evenly over the GPU
+    (pth_fa_forward_balanced) where that is rated faster: chunks whose query tiles see very different
+    numbers of keys. A workspace for the partials is taken from torch's allocator.
     max_keys: a host-side bound on the keys any row of the batch sees (the longest seq_len), used
     only to size the launch; None takes the block table's width in keys.
     """
@@ -324,8 +325,8 @@ def forward_rows(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
     dtypes or alignments); query_start is a list, max_keys a bound on the keys any row sees.
     """
     if not (query.is_cuda and query.dtype == torch.float16 and out.dtype == torch.float16 and query.dim() == 3
-            and out.dim() == 3 and key_cache.dim() == 4 and query.stride(2) == 1 and out.stride(2) == 1 and query.stride(0) % 8 == 0 and query.stride(1) % 8 == 0
-            and query.data_ptr() % 16 == 0 and out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0
+            and out.dim() == 3 and key_cache.dim() == 4 and query.stride(2) == 1 and out.stride(2) == 1
+            and query.stride(0) % 8 == 0 and query.stride(1) % 8 == 0 and query.data_ptr() % 16 == 0 and out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0
             and out.data_ptr() % 8 == 0):
         return False
     nsplit, rows, heads_kv = 0, query_start[-1] - query_start[0], key_cache.shape[2]
