@@ -97,6 +97,14 @@ __device__ __forceinline__ void settle_values(float4_t (&o)[16]) {
     asm volatile("s_nop 15" : "+a"(o[0]), "+a"(o[1]), "+a"(o[2]), "+a"(o[3]), "+a"(o[4]), "+a"(o[5]), "+a"(o[6]), "+a"(o[7]));
     asm volatile("" : "+a"(o[8]), "+a"(o[9]), "+a"(o[10]), "+a"(o[11]), "+a"(o[12]), "+a"(o[13]), "+a"(o[14]), "+a"(o[15]));
 }
+// The wait before the products of P' (see settle_operand), once for all of its row blocks.
+template <bool kExact>
+__device__ __forceinline__ void settle_weights(half8_t (&p)[kFwRB], half8_t (&lo)[kFwRB]) {
+    if constexpr (kExact)
+        asm volatile("s_nop 1" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(lo[0]), "+v"(lo[1]), "+v"(lo[2]), "+v"(lo[3]));
+    else
+        asm volatile("s_nop 1" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
+}
 
 template <bool kFast, bool kExact, bool kSplit, class T>
 __global__ void __launch_bounds__(kFwWaves * 64, 1) pd_prefill_wide_kernel(const FaParams a) {
@@ -274,6 +282,7 @@ __global__ void __launch_bounds__(kFwWaves * 64, 1) pd_prefill_wide_kernel(const
             vr[m] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_int2*)(S + (m < 8 ? vro_lo : vro_hi) + 16 * m));
         };
         half8_t op = widen_i8x8_exact(kr[0].x, kr[0].y);
+        settle_operand(op);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int u = i >> 2, c = i & 3;
@@ -383,6 +392,7 @@ __global__ void __launch_bounds__(kFwWaves * 64, 1) pd_prefill_wide_kernel(const
             }
             l_run[rb] += psum;
         }
+        settle_weights<kExact>(pop, plo);
 #pragma unroll
         for (int m = 0; m < 16; ++m) {
             if (m + kVAhead < 16) vread(m + kVAhead);

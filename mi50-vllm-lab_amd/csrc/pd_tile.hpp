@@ -79,21 +79,28 @@ __device__ __forceinline__ half8_t widen_i8x8(unsigned w0, unsigned w1) {
 // instruction per value against 0.75 for widen_i8x8, with no bias left in the operand, so the
 // products accumulate without the 1152 sum_d q_d (scores) or 1152 sum_k P'_k (values) that the
 // fp32 accumulator would otherwise carry (and round) along with them. The decode widens K and V
-// this way, and so does the exact prefill.
+// this way, and so does the exact prefill. The low halves are written first: a conversion that keeps
+// the other half of its register may not directly follow the one that wrote it.
 __device__ __forceinline__ half8_t widen_i8x8_exact(unsigned w0, unsigned w1) {
     uint4_t h;
     asm("v_cvt_f16_i16_sdwa %0, sext(%4) dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:BYTE_0\n\t"
-        "v_cvt_f16_i16_sdwa %0, sext(%4) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_1\n\t"
         "v_cvt_f16_i16_sdwa %1, sext(%4) dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:BYTE_2\n\t"
-        "v_cvt_f16_i16_sdwa %1, sext(%4) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_3\n\t"
         "v_cvt_f16_i16_sdwa %2, sext(%5) dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:BYTE_0\n\t"
-        "v_cvt_f16_i16_sdwa %2, sext(%5) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_1\n\t"
         "v_cvt_f16_i16_sdwa %3, sext(%5) dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:BYTE_2\n\t"
+        "v_cvt_f16_i16_sdwa %0, sext(%4) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_1\n\t"
+        "v_cvt_f16_i16_sdwa %1, sext(%4) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_3\n\t"
+        "v_cvt_f16_i16_sdwa %2, sext(%5) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_1\n\t"
         "v_cvt_f16_i16_sdwa %3, sext(%5) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_3"
         : "=&v"(h.x), "=&v"(h.y), "=&v"(h.z), "=&v"(h.w)
         : "v"(w0), "v"(w1));
     return __builtin_bit_cast(half8_t, h);
 }
+
+// A matrix instruction needs two wait states after the vector instruction that wrote one of its operands. The
+// compiler keeps them between its own instructions only: an operand that goes from one asm block to the
+// products of another passes through here. (Operands of the compiler's own products do not: it puts one wait state
+// behind the asm itself, and a second one made the windowed decode of 4 x 8 rows 17.7 -> 18.3 us.)
+__device__ __forceinline__ void settle_operand(half8_t& x) { asm("s_nop 1" : "+v"(x)); }
 
 // Eight consecutive query values as fp16. Q is rounded to fp16 unscaled: fp16-valued queries enter the
 // matrix cores exactly.

@@ -82,3 +82,68 @@ def test_no_packed_fp32_instructions(gfx950_asm):
     # the build disables the packed-FP32 VALU forms; none may appear in the code
     for asm in gfx950_asm:
         assert not re.search(r"\bv_pk_(add|mul|fma)_f32\b", asm)
+
+
+def _registers(operand):
+    """{("v" or "a", number)} of a vector register operand, empty for any other."""
+    m = re.fullmatch(r"([va])(?:(\d+)|\[(\d+):(\d+)\])", operand.split(" ")[0])
+    if not m:
+        return set()
+    first, last = (m.group(2), m.group(2)) if m.group(2) else m.group(3, 4)
+    return {(m.group(1), i) for i in range(int(first), int(last) + 1)}
+
+
+def early_matrix_reads(asm, states_needed):
+    """(vector instruction, matrix instruction) pairs where the second reads what the first wrote fewer than
+    `states_needed` (1 or 2) wait states before it."""
+    found, recent = [], []  # recent: wait states and registers written, of the last instructions
+    for line in asm.splitlines():
+        text = line.split(";")[0].strip()
+        if not re.match(r"[a-z]\w+(\s|$)", text) or text.endswith(":"):
+            continue
+        name, rest = (text.split(None, 1) + [""])[:2]
+        operands = [x.strip() for x in re.split(r",(?![^\[]*\])", rest)]
+        written = set()
+        if name.startswith("v_mfma"):
+            read, waited = set().union(*(_registers(x) for x in operands[1:4])), 0
+            for states, regs, who in reversed(recent):
+                if waited >= states_needed:
+                    break
+                if regs & read:
+                    found.append((who, text))
+                    break
+                waited += states
+        elif name.startswith("v_"):
+            written = _registers(operands[0])
+            if name.startswith(("v_permlane", "v_swap")):
+                written |= _registers(operands[1])
+        recent = recent[-2:] + [(int(operands[0]) + 1 if name == "s_nop" else 1, written, text)]
+    return found
+
+
+def test_matrix_operands_have_settled(gfx950_asm):
+    # inline asm is outside the compiler's own hazard checks. The 256-row prefill writes operands and products both
+    # in asm, so it keeps the two wait states between them itself; elsewhere the products are the compiler's
+    close = ["v_cvt_f16_i16_sdwa v5, sext(v1) dst_sel:WORD_1", "s_nop 0", "v_mfma_f32_16x16x32_f16 a[0:3], v[2:5], v[8:11], a[0:3]"]
+    close = "\n".join("\t" + x for x in close)
+    assert len(early_matrix_reads(close, 2)) == 1 and not early_matrix_reads(close, 1)
+    assert not early_matrix_reads(close.replace("s_nop 0", "s_nop 1"), 2)
+    kernels = {}
+    for asm in gfx950_asm:
+        wide = "pd_prefill_wide_kernel" in asm
+        kernels[wide] = kernels.get(wide, 0) + asm.count("v_mfma")
+        assert early_matrix_reads(asm, 2 if wide else 1) == []
+    assert kernels[True] > 0 and kernels[False] > 0
+
+
+def test_halves_of_a_register_are_not_written_back_to_back(gfx950_asm):
+    # a conversion that preserves the other half reads the register: one wait state after the one that wrote it
+    for asm in gfx950_asm:
+        last = ""
+        for line in asm.splitlines():
+            text = line.split(";")[0].strip()
+            if not re.match(r"[a-z]\w+(\s|$)", text):
+                continue
+            if "UNUSED_PRESERVE" in text and "_sdwa" in last:
+                assert text.split()[1] != last.split()[1], (last, text)
+            last = text
