@@ -14,8 +14,8 @@
 // MFMA, or as fp16. Launches that 256-row workgroups finish sooner run pd_prefill_wide_kernel.
 // kExact (pth_fa_forward_exact) gives the decode kernel's numerics: K and V are widened without
 // the bias (so the fp32 accumulators hold only the products' own sums) and P' enters the P.V
-// products as fp16 hi + lo, which doubles them. The default instance keeps the bias in K and V
-// and removes it per row (sum_d q_d (k_d + 1152) - 1152 sum_d q_d, sum_k P'_k (v_k + 1152) -
+// products as fp16 hi + lo, which doubles them. The default instances of pd_prefill_kernel keep the bias in K
+// and V and remove it per row (sum_d q_d (k_d + 1152) - 1152 sum_d q_d, sum_k P'_k (v_k + 1152) -
 // 1152 sum_k P'_k).
 #include <algorithm>
 #include <type_traits>
@@ -108,6 +108,11 @@ __device__ __forceinline__ void prefill_body(const FaParams& a, const FaWork& wk
     // tokens x 4 splits, fma_mix being the part that costs it) and keep per-store addresses and
     // a multiply and a conversion for P'.
     constexpr bool kPinned = !kExact && kParts == 0;
+    // K and V carry the widening bias (see the head of the file), whose rounding grows with the run of key tiles
+    // that one accumulator sums. The dealt instance's runs are as long as the deal makes them, so it widens exactly:
+    // error of four chunks of 70 to 900 tokens over 1,500 to 6,000 keys 4.4e-4 -> 2.9e-4 of the result (302 us
+    // with 9 decoded sequences, 297 biased), of chunks over 30,000 to 60,000 keys on 10 workgroups 5.2e-3 -> 2.9e-4.
+    constexpr bool kBias = !kExact && kParts != 2;
     const int b = wk.b, g = wk.g, tq0 = wk.tq0, ntok = wk.ntok, seq_len = wk.seq_len, qabs = wk.qabs;
     const int t0 = wk.t0, t1 = wk.t1;
     const int tid = threadIdx.x, l = tid & 63, lg = l >> 4, li = l & 15;
@@ -185,7 +190,7 @@ __device__ __forceinline__ void prefill_body(const FaParams& a, const FaWork& wk
             }
         }
     }
-    {
+    if constexpr (kBias) {
         const half8_t nb = (half8_t)(_Float16)(-kWidenBias);
 #pragma unroll
         for (int rb = 0; rb < kFaRB; ++rb) {
@@ -284,24 +289,24 @@ __device__ __forceinline__ void prefill_body(const FaParams& a, const FaWork& wk
         if (j < 4) {
             const int u = j >> 1, hh = j & 1;
             half8_t kf;
-            if constexpr (kExact)
-                kf = hh == 0 ? widen_i8x8_exact(r.kr[u].x, r.kr[u].y) : widen_i8x8_exact(r.kr[u].z, r.kr[u].w);
-            else
+            if constexpr (kBias)
                 kf = hh == 0 ? widen_i8x8(r.kr[u].x, r.kr[u].y) : widen_i8x8(r.kr[u].z, r.kr[u].w);
+            else
+                kf = hh == 0 ? widen_i8x8_exact(r.kr[u].x, r.kr[u].y) : widen_i8x8_exact(r.kr[u].z, r.kr[u].w);
             lds_u8* const d = kPinned ? r.hk + (2 * hh + u) * 1024 : H + ((2 * w + hh) * 2 + u) * 1024 + 16 * l;
             *(lds_half8*)d = kf;
         } else if (j < 8) {
-            // kExact: V widened exactly (no bias), so the fp32 P.V accumulators hold only the
-            // products' own sums; else with the bias, removed per row at the end
+            // widened exactly (no bias) the fp32 P.V accumulators hold only the products' own sums; else
+            // with the bias, removed per row at the end
             const int2_t vr = r.vr[j - 4];
             lds_u8* const d = kPinned ? r.hv + 4096 * (j - 4) : H + kFaHK + (w + 4 * (j - 4)) * 1024 + 16 * l;
             *(lds_half8*)d =
-                kExact ? widen_i8x8_exact((unsigned)vr.x, (unsigned)vr.y) : widen_i8x8((unsigned)vr.x, (unsigned)vr.y);
+                kBias ? widen_i8x8((unsigned)vr.x, (unsigned)vr.y) : widen_i8x8_exact((unsigned)vr.x, (unsigned)vr.y);
         } else if (j == 8) {
-            // rows 12..15 of the tail block are the v_scale bytes. kExact: the O^T rows they feed
+            // rows 12..15 of the tail block are the v_scale bytes. Widened exactly, the O^T rows they feed
             // (lane group 3 of accumulator block 16) are never stored. Else they are widened from
             // 0 to exactly 1152, so those rows accumulate 1152 * sum of P', the bias to remove
-            if constexpr (kExact) {
+            if constexpr (!kBias) {
                 *(lds_half8*)(H + kFaHK + 16 * 1024 + 16 * l) = widen_i8x8_exact((unsigned)r.vr[4].x, (unsigned)r.vr[4].y);
             } else {
                 const int2_t vt = li >= 12 ? int2_t{0, 0} : r.vr[4];
@@ -357,7 +362,7 @@ __device__ __forceinline__ void prefill_body(const FaParams& a, const FaWork& wk
 #pragma unroll
                 for (int rb = 0; rb < kFaRB; ++rb)
                     sacc[rb][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[st & 1][u], qop[rb][st],
-                                                                         st ? sacc[rb][u] : (float4_t)(kExact ? 0.f : qneg[rb]), 0, 0, 0);
+                                                                         st ? sacc[rb][u] : (float4_t)(kBias ? qneg[rb] : 0.f), 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
         const int kb = n * kTile;
@@ -562,7 +567,7 @@ __device__ __forceinline__ void prefill_body(const FaParams& a, const FaWork& wk
         const float l_row = xor_sum(xor_sum(l_run[rb], 16), 32);
         const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
         // the V widening bias of the row, 1152 * sum of its P' (0 when V is widened exactly)
-        const float corr = kExact ? 0.f : __shfl(oacc[rb][16].x, 48 + li, 64);
+        const float corr = kBias ? __shfl(oacc[rb][16].x, 48 + li, 64) : 0.f;
 
         if (rvalid[rb]) {
             const int r = 48 * w + 16 * rb + li;
@@ -644,7 +649,7 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
 // last), which pd_prefill_merge_kernel adds up. Measured (24 q / 4 kv heads, whole call): a fresh prompt of 4,000
 // tokens 398 us in one workgroup per query tile, 376 in 2 splits, 327 here; 700 tokens over 6,000 keys 207 (2
 // splits) against 184; a batch of 9 decoded sequences and chunks of 70 to 900 tokens over 1,500 to
-// 6,000 keys 481 -> 298 (four launches, with a transpose and two conversions each, before). Where all
+// 6,000 keys 481 -> 302 (four launches, with a transpose and two conversions each, before). Where all
 // query tiles need the same (2,048 tokens over 61,440) the splits' kernel is 3 % faster and is taken.
 constexpr unsigned kFaSegmentUnits = 10;  // set-up and stores of a segment, ~16 us, in key tiles (1.62 us)
 constexpr unsigned kFaMinShare = 16;      // units of a workgroup: below, pieces cost more than they save

@@ -137,3 +137,28 @@ def test_rows_graph_replays():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("wgs", [None, 10], ids=["all", "10"])
+def test_error_does_not_grow_with_the_run(wgs):
+    """Chunks over long prefixes, each workgroup on a run of hundreds of key tiles (10 workgroups: thousands, across
+    items). The default numerics round the weights to fp16, and the output is fp16: each at most 2^-11 / sqrt(3) =
+    2.8e-4 of the result's norm, 4e-4 together; nothing that grows with the keys may come on top."""
+    ctxs, news = [60000, 30011, 45000, 52000], [200, 77, 130, 100]
+    c = kvc.make_case(ctxs, news, num_q_heads=6, num_kv_heads=1, block_size=16, seed=11)
+    d = c.to("cuda")
+    out = torch.full_like(d.q, float("nan"))
+    starts = [sum(news[:i]) for i in range(5)]
+    balanced(d.q, d, d.seq_lens, out, starts, False, wgs and wgs * SLOT)
+    o = out.double().cpu().numpy()
+    assert np.isfinite(o).all()
+    num = den = 0.0
+    for i, n in enumerate(news):
+        rows = [0, n // 2, n - 1]
+        qi = c.q[starts[i]:starts[i + 1]].transpose(0, 1).unsqueeze(0).float().contiguous()
+        ref, _ = orc.paged_prefill(qi, c.cache.key_cache, c.cache.value_cache, c.cache.k_scale, c.cache.v_scale,
+                                   c.block_table[i:i + 1], c.seq_lens[i:i + 1], c.scale, torch.tensor([ctxs[i]]), rows)
+        e = o[starts[i]:starts[i + 1]][rows] - ref[0][rows]
+        num, den = num + (e ** 2).sum(), den + (ref[0][rows] ** 2).sum()
+    print(f"  wgs={wgs} error {np.sqrt(num / den):.2e} of the result", flush=True)
+    assert np.sqrt(num / den) <= 4e-4
