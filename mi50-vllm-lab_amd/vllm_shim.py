@@ -286,30 +286,26 @@ class Gfx950Int8Attention:
                                      output[:qsl[p]], max_q_prefix, meta,
                                      None if meta.seq_lens_cpu is None else meta.seq_lens_cpu[:p])):
             triton_fallback(0, qsl[p], 0, p, max_q_prefix)
-        # The split count of each prefill is planned for the keys its sequence sees: the host length
-        # when it is known and no graph is being captured (vLLM's block table is as wide as the
-        # model's maximum length, so the table alone would plan every chunk for the longest context),
-        # else the batch's max_seq_len, else the table width.
-        lens_host = meta.seq_lens_cpu if meta.seq_lens_cpu is not None and not _capturing(query.device) else None
+        # A launch is planned for the keys that its sequences see: the host lengths when they are known and
+        # no graph is being captured (vLLM's block table is as wide as the model's maximum length, so the table
+        # alone would plan every chunk for the longest context), else the batch's max_seq_len, else the
+        # table width. A capture's lengths are those of a dummy batch: the table's width alone bounds the replays.
+        lens_host, max_seq_len = meta.seq_lens_cpu, max(0, int(meta.max_seq_len))
+        if _capturing(query.device):
+            lens_host, max_seq_len = None, 0
         # All sequences in one launch that reads the query rows and writes the output rows as they are; the
         # calls it does not take go one by one through forward_pth.
         rows = getattr(self.pth_fa, "forward_rows", None)
         if rows is not None:
-            keys = (max(int(x) for x in lens_host[p:n]) if lens_host is not None else int(meta.max_seq_len)) or \
-                meta.block_table.shape[1] * key_cache.shape[1]
+            keys = max(int(x) for x in lens_host[p:n]) if lens_host is not None else max_seq_len
             if rows(query, key_cache, value_cache, meta.block_table[p:n], meta.seq_lens[p:n], self.scale, qsl[p:], output,
-                    keys, PTH_FA_EXACT):
+                    keys or meta.block_table.shape[1] * key_cache.shape[1], PTH_FA_EXACT):
                 return True
         for i in range(p, n):
             start, nq = qsl[i], qsl[i + 1] - qsl[i]
             q = query[start:start + nq].transpose(0, 1).unsqueeze(0).float().contiguous()  # [1, Hq, nq, D]
             seq_len = meta.seq_lens[i:i + 1]
-            if lens_host is not None:
-                max_keys = int(lens_host[i])
-            elif meta.max_seq_len > 0 and not _capturing(query.device):
-                max_keys = int(meta.max_seq_len)
-            else:
-                max_keys = None
+            max_keys = int(lens_host[i]) if lens_host is not None else (max_seq_len or None)
             out = self.pth_fa.forward_pth(q, key_cache, value_cache, meta.block_table[i:i + 1], seq_len, self.scale,
                                           seq_len - nq, max_keys=max_keys,
                                           **({"exact": True} if PTH_FA_EXACT else {}))

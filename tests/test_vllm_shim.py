@@ -32,6 +32,13 @@ class FakeOps:
         self.max_keys = getattr(self, "max_keys", []) + [max_keys]
         return torch.full((1, q.shape[2], q.shape[1], q.shape[3]), 2.0)
 
+    def forward_rows(self, q, kc, vc, bt, sl, scale, query_start, out, max_keys, exact=False):
+        if q.dtype != torch.float16 or len(query_start) > 33:
+            return False
+        self.calls.append(("rows", tuple(query_start), sl.tolist(), bt.shape[0], max_keys, exact))
+        out[query_start[0]:query_start[-1]] = 3.0
+        return True
+
 
 @pytest.fixture
 def ops(monkeypatch):
@@ -293,6 +300,55 @@ def test_prefill_exact_switch(ops, monkeypatch, exact):
     m = meta([100, 70], [1100, 70])
     assert a.route(q, kc, kc, None, None, m, out, 100, 170, lambda *x: pytest.fail("fallback"))
     assert ops.exact == [exact, exact]
+
+
+def half_tensors(T):
+    q, out, kc = tensors(T)
+    return q.half(), out.half(), kc
+
+
+@pytest.mark.parametrize("exact", [False, True])
+def test_fp16_suffix_is_one_rows_call(ops, monkeypatch, exact):
+    """What engines run: fp16 rows, every suffix sequence in one launch sized by the longest host length."""
+    monkeypatch.setattr(shim, "PTH_FA_EXACT", exact)
+    q, out, kc = half_tensors(2 + 100 + 70)
+    m = meta([1, 1, 100, 70], [5000, 40, 1100, 70])
+    m.seq_lens_cpu = [5000, 40, 1100, 70]
+    assert impl().route(q, kc, kc, None, None, m, out, 100, 172, lambda *x: pytest.fail("fallback"))
+    assert [c[0] for c in ops.calls] == ["layout", "decode", "rows"]
+    assert ops.calls[-1] == ("rows", (2, 102, 172), [1100, 70], 2, 1100, exact)
+    assert (out[:2] == 1).all() and (out[2:] == 3).all()
+
+
+@pytest.mark.parametrize("qlens,seqs", [([77], [300]), ([100, 70], [1100, 70])], ids=["one", "two"])
+def test_fp16_suffix_is_sized_as_the_loop_is(ops, monkeypatch, qlens, seqs):
+    """The launch is sized by the host lengths, else max_seq_len, and while a graph is captured, whose lengths are a
+    dummy batch's, by the table: sized for the dummy lengths it would stay frozen for short contexts."""
+    q, out, kc = half_tensors(sum(qlens))
+    m = meta(qlens, seqs)
+    m.block_table = torch.zeros((len(seqs), 131072 // 16), dtype=torch.int32)
+
+    def keys():
+        assert impl().route(q, kc, kc, None, None, m, out, max(qlens), sum(qlens), lambda *x: pytest.fail("fallback"))
+        assert ops.calls[-1][0] == "rows"
+        return ops.calls[-1][4]
+    assert keys() == max(seqs)  # max_seq_len
+    m.seq_lens_cpu, m.max_seq_len = seqs, 100000
+    assert keys() == max(seqs)
+    with monkeypatch.context() as capture:
+        capture.setattr(shim, "_capturing", lambda device: True)
+        assert keys() == 131072
+        m.seq_lens_cpu = None
+        assert keys() == 131072
+    m.max_seq_len = 0
+    assert keys() == 131072
+
+
+def test_fp16_suffix_of_many_sequences_goes_one_by_one(ops):
+    q, out, kc = half_tensors(33 * 64)
+    m = meta([64] * 33, [64] * 33)
+    assert impl().route(q, kc, kc, None, None, m, out, 64, 33 * 64, lambda *x: pytest.fail("fallback"))
+    assert [c[0] for c in ops.calls] == ["prefill"] * 33 and (out == 2).all()
 
 
 def test_prefill_prefix_too_long_for_decode_goes_to_triton(ops):
