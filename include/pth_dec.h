@@ -212,7 +212,7 @@ int pth_fa_forward_split(const pd_tensor* q, const pd_tensor* key_cache, const p
  *   query_start (host, int[num_seqs + 1], num_seqs <= 32): q fp16 [T, Hq, 256] with unit dim stride, rows
  *     16-byte aligned; sequence i has rows [query_start[i], query_start[i + 1]) of q and out, the last tokens
  *     of its seq_lens[i] keys; block_table and seq_lens have a row per sequence; out fp16 [T, Hq, 256],
- *     rows 8-byte aligned. The rows outside the sequences are left alone. q_abs_offset is ignored.
+ *     rows 8-byte aligned, T its own (both hold the sequences' rows). The rows outside the sequences are left alone. q_abs_offset is ignored.
  *   workspace  fp32, contiguous, 16-byte aligned, of pth_fa_balanced_workspace floats (fewer, down to
  *              2 x 192 x 258, only lower the number of workgroups)
  *   max_keys   a bound on the keys any row sees, to size the launch; a wrong one costs time only

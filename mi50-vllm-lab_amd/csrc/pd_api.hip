@@ -408,8 +408,8 @@ static int fa_forward_rows(const pd_tensor* q, const pd_tensor* kc, const pd_ten
     if (!(q->ndim == 3 && q->dtype == PD_DTYPE_FP16 && q->sizes[2] == kDim &&
           q->strides[2] == 1 && q->sizes[0] <= INT32_MAX && q->sizes[1] <= INT32_MAX))
         return fail(err, errlen, "q must be fp16 [T, Hq, 256] with unit dim stride");
-    if (!(out->ndim == 3 && out->dtype == q->dtype && out->sizes[0] == q->sizes[0] && out->sizes[1] == q->sizes[1] &&
-          out->sizes[2] == kDim && out->strides[2] == 1))
+    if (!(out->ndim == 3 && out->dtype == q->dtype && out->sizes[1] == q->sizes[1] && out->sizes[2] == kDim &&
+          out->strides[2] == 1))
         return fail(err, errlen, "out must be fp16 [T, Hq, 256] with unit dim stride");
     if (!(reinterpret_cast<uintptr_t>(q->data) % 16 == 0 && q->strides[0] % 8 == 0 && q->strides[1] % 8 == 0 &&
           reinterpret_cast<uintptr_t>(out->data) % 8 == 0 && out->strides[0] % 4 == 0 && out->strides[1] % 4 == 0))
@@ -426,8 +426,9 @@ static int fa_forward_rows(const pd_tensor* q, const pd_tensor* kc, const pd_ten
     const int64_t T = q->sizes[0], Hq = q->sizes[1], bs = kc->sizes[1], Hkv = kc->sizes[2];
     if (!(Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && Hq / Hkv <= kFaRows))
         return fail(err, errlen, "heads_q must be a multiple of heads_kv, at most 192 times");
-    if (!(num_seqs >= 1 && num_seqs <= kFaMaxSeqs && query_start[0] >= 0 && query_start[num_seqs] <= T))
-        return fail(err, errlen, "1 to 32 sequences within the rows of q");
+    if (!(num_seqs >= 1 && num_seqs <= kFaMaxSeqs && query_start[0] >= 0 && query_start[num_seqs] <= T &&
+          query_start[num_seqs] <= out->sizes[0]))
+        return fail(err, errlen, "1 to 32 sequences within the rows of q and out");
     for (int64_t i = 0; i < num_seqs; ++i)
         if (query_start[i] > query_start[i + 1]) return fail(err, errlen, "query_start must not decrease");
     if (!(bt->dtype == PD_DTYPE_INT32 && bt->ndim == 2 && bt->sizes[0] >= num_seqs && bt->strides[1] == 1 &&

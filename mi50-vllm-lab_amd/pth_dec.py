@@ -322,12 +322,13 @@ def forward_rows(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
     query_start[i + 1]) of query and out (fp16 [T, Hq, 256]), the last tokens of its seq_lens[i] keys
     (pth_fa_forward_balanced's rows form; no counterpart in the reference). Numerics are forward_pth's.
     Returns False, with nothing launched, for calls beyond the entry's limits (over 32 sequences, other
-    dtypes or alignments); query_start is a list, max_keys a bound on the keys any row sees.
+    dtypes or alignments, out on another device, strided seq_lens); query_start is a list, max_keys a bound on the
+    keys any row sees. query and out may have different numbers of rows.
     """
     if not (query.is_cuda and query.dtype == torch.float16 and out.dtype == torch.float16 and query.dim() == 3
             and out.dim() == 3 and key_cache.dim() == 4 and query.stride(2) == 1 and out.stride(2) == 1
             and query.stride(0) % 8 == 0 and query.stride(1) % 8 == 0 and query.data_ptr() % 16 == 0 and out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0
-            and out.data_ptr() % 8 == 0):
+            and out.data_ptr() % 8 == 0 and out.device == query.device and seq_lens.is_contiguous()):
         return False
     nsplit, rows, heads_kv = 0, query_start[-1] - query_start[0], key_cache.shape[2]
     if len(query_start) == 2 and rows > 0 and heads_kv > 0 and query.shape[1] > 0:

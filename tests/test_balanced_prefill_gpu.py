@@ -162,3 +162,25 @@ def test_error_does_not_grow_with_the_run(wgs):
         num, den = num + (e ** 2).sum(), den + (ref[0][rows] ** 2).sum()
     print(f"  wgs={wgs} error {np.sqrt(num / den):.2e} of the result", flush=True)
     assert np.sqrt(num / den) <= 4e-4
+
+
+def test_rows_calls_that_the_loop_takes():
+    """Calls that one forward_pth per sequence takes are taken as well, or left to it (False): out with more or
+    fewer rows than query, strided lengths, an output on the host."""
+    c = kvc.make_case([300, 0], [70, 65], num_q_heads=24, num_kv_heads=4, block_size=16, seed=6).to("cuda")
+    k, starts = c.cache, [0, 70, 135]
+
+    def call(q, out, lens=c.seq_lens):
+        return pth_dec.forward_rows(q, k.key_cache, k.value_cache, c.block_table, lens, c.scale, starts, out, 370)
+    want = torch.zeros_like(c.q)
+    assert call(c.q, want)
+    longer = torch.full((150, 24, 256), 7.0, dtype=torch.float16, device="cuda")
+    assert call(c.q, longer) and torch.equal(longer[:135], want) and (longer[135:] == 7).all()
+    shorter = torch.zeros_like(want)
+    assert call(torch.cat([c.q, c.q[:9]]), shorter) and torch.equal(shorter, want)
+    untouched = torch.full_like(want, 7.0)
+    lens = torch.stack([c.seq_lens, c.seq_lens], 1)[:, 0]
+    assert not lens.is_contiguous() and not call(c.q, untouched, lens) and (untouched == 7).all()
+    assert not call(c.q, torch.empty(want.shape, dtype=torch.float16))
+    with pytest.raises(RuntimeError, match="within the rows of q and out"):
+        call(c.q, untouched[:134])
