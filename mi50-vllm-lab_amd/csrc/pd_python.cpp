@@ -189,8 +189,8 @@ PyObject* prefill_split(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // prefill_balanced(entry, workspace entry, q, key_cache, value_cache, block_table, seq_lens, scale, q_abs_offset, out,
 //                  query_start, max_keys, nsplit, exact): pth_fa_forward_balanced with its workspace from torch's allocator.
-// query_start None: the batch form, with q_abs_offset; a list of row numbers: the rows form. False if the
-// entry does not take such a call.
+// query_start None: the batch form, with q_abs_offset; a list of row numbers: the rows form. False, with nothing
+// launched, if the entry does not take such a call or its workspace cannot be had.
 PyObject* prefill_balanced(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         decltype(&pth_fa_forward_balanced) fn;
@@ -227,7 +227,12 @@ PyObject* prefill_balanced(PyObject*, PyObject* const* a, Py_ssize_t n) {
         else if (shaped && rows)
             floats = nsplit > 1 ? (starts[1] - starts[0]) * t[0].sizes[1] * nsplit * 258 : 4;
         if (floats <= 0) Py_RETURN_FALSE;
-        const at::Tensor ws = at::empty({floats}, THPVariable_Unpack(a[2]).options().dtype(at::kFloat));
+        at::Tensor ws;
+        try {
+            ws = at::empty({floats}, THPVariable_Unpack(a[2]).options().dtype(at::kFloat));
+        } catch (const c10::OutOfMemoryError&) {
+            Py_RETURN_FALSE;
+        }
         wd.data = ws.data_ptr();
         wd.dtype = PD_DTYPE_FP32;
         wd.ndim = 1;

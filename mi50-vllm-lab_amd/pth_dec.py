@@ -283,7 +283,8 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
     None picks them as prefill_splits does, counting the 256-row kernel as well (2,048 tokens over 61k
     keys: 4 splits of it, 2,560: one round unsplit), or deals the key tiles evenly over the GPU
     (pth_fa_forward_balanced) where that is rated faster: chunks whose query tiles see very different
-    numbers of keys. A workspace for the partials is taken from torch's allocator.
+    numbers of keys. A workspace for the partials is taken from torch's allocator (203 MB for 2,048 tokens over 61k
+    keys at 24 q heads, 101 MB for a dealt call); where a planned call cannot have it, it runs unsplit, without one.
     max_keys: a host-side bound on the keys any row of the batch sees (the longest seq_len), used
     only to size the launch; None takes the block table's width in keys.
     """
@@ -291,7 +292,8 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
         raise RuntimeError("q must be contiguous fp32 [B, Hq, Sq, D]")
     if out is None:
         out = torch.empty((q.shape[0], q.shape[2], q.shape[1], q.shape[3]), dtype=torch.float32, device=q.device)
-    if nsplit is None:
+    planned = nsplit is None
+    if planned:
         if max_keys is None:
             max_keys = block_table.shape[1] * key_cache.shape[1] if block_table.dim() == 2 else 0
         batch, heads_q, sq, heads_kv = q.shape[0], q.shape[1], q.shape[2], key_cache.shape[2]
@@ -304,9 +306,15 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
                     block_table, seq_lens, scale, q_abs_offset, out, None, int(max_keys), 0, 1 if exact else 0):
                 return out
             nsplit = nsplit or prefill_splits(batch, sq, heads_q, heads_kv, int(max_keys), block_size)
+    ws = None
     if nsplit > 1:
-        ws = torch.empty((q.shape[0] * q.shape[2] * q.shape[1] * nsplit * (q.shape[3] + 2),), dtype=torch.float32,
-                         device=q.device)
+        try:
+            ws = torch.empty((q.shape[0] * q.shape[2] * q.shape[1] * nsplit * (q.shape[3] + 2),), dtype=torch.float32,
+                             device=q.device)
+        except torch.OutOfMemoryError:
+            if not planned:
+                raise
+    if ws is not None:
         native().prefill_split(_entry("pth_fa_forward_split"), q, key_cache, value_cache, block_table, seq_lens, scale,
                                q_abs_offset, out, ws, int(nsplit), 1 if exact else 0)
     else:
@@ -322,7 +330,8 @@ def forward_rows(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
     query_start[i + 1]) of query and out (fp16 [T, Hq, 256]), the last tokens of its seq_lens[i] keys
     (pth_fa_forward_balanced's rows form; no counterpart in the reference). Numerics are forward_pth's.
     Returns False, with nothing launched, for calls beyond the entry's limits (over 32 sequences, other
-    dtypes or alignments, out on another device, strided seq_lens); query_start is a list, max_keys a bound on the
+    dtypes or alignments, out on another device, strided seq_lens) and for several sequences whose workspace
+    (101 MB) cannot be had; a single one then runs unsplit. query_start is a list, max_keys a bound on the
     keys any row sees. query and out may have different numbers of rows.
     """
     if not (query.is_cuda and query.dtype == torch.float16 and out.dtype == torch.float16 and query.dim() == 3
@@ -333,9 +342,13 @@ def forward_rows(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
     nsplit, rows, heads_kv = 0, query_start[-1] - query_start[0], key_cache.shape[2]
     if len(query_start) == 2 and rows > 0 and heads_kv > 0 and query.shape[1] > 0:
         nsplit = _prefill_plan(1, rows, query.shape[1], heads_kv, max_keys, key_cache.shape[1], rows)
-    return native().prefill_balanced(_entry("pth_fa_forward_balanced"), _entry("pth_fa_balanced_workspace"), query,
+    one = len(query_start) == 2 and rows > 0
+    for n in (nsplit, 1) if one and nsplit != 1 else (nsplit,):  # (a single chunk without its workspace: unsplit)
+        if native().prefill_balanced(_entry("pth_fa_forward_balanced"), _entry("pth_fa_balanced_workspace"), query,
                                      key_cache, value_cache, block_table, seq_lens, scale, None, out, query_start,
-                                     max_keys, nsplit, 1 if exact else 0)
+                                     max_keys, n, 1 if exact else 0):
+            return True
+    return False
 
 
 def cache_write(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,

@@ -184,3 +184,39 @@ def test_rows_calls_that_the_loop_takes():
     assert not call(c.q, torch.empty(want.shape, dtype=torch.float16))
     with pytest.raises(RuntimeError, match="within the rows of q and out"):
         call(c.q, untouched[:134])
+
+
+def test_planned_calls_without_memory_for_their_workspace():
+    """With no room for the partials a planned call runs unsplit, several chunks are left to the loop, and a split
+    count that the caller asked for raises torch's error. The room is limited in torch's allocator."""
+    c = kvc.make_case([3000], [1501], num_q_heads=24, num_kv_heads=4, block_size=16, seed=8).to("cuda")
+    k, q, starts = c.cache, kvc.prefill_query(c), [0, 1501]
+    q_abs = torch.tensor([3000], dtype=torch.int32, device="cuda")
+    out, rows = torch.empty((1, 1501, 24, 256), device="cuda"), torch.empty_like(c.q)
+
+    def batch(nsplit, max_keys):
+        pth_dec.forward_pth(q, k.key_cache, k.value_cache, c.block_table, c.seq_lens, c.scale, q_abs, out=out,
+                            nsplit=nsplit, max_keys=max_keys)
+        return out.clone()
+
+    def chunk(starts, max_keys):
+        rows.fill_(7)
+        return pth_dec.forward_rows(c.q, k.key_cache, k.value_cache, c.block_table.expand(len(starts) - 1, -1),
+                                    c.seq_lens.expand(len(starts) - 1).contiguous(), c.scale, starts, rows, max_keys)
+    unsplit, plans = batch(1, 4501), [pth_dec._prefill_plan(1, 1501, 24, 4, m, 16, 1501) for m in (4501, 200000)]
+    assert plans[0] == 0 and plans[1] > 1  # dealt, and split
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + (64 << 20)
+    torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        for max_keys in (4501, 200000):
+            assert torch.equal(batch(None, max_keys), unsplit)
+            assert chunk(starts, max_keys)
+            assert (rows.cpu().float() - unsplit[0].cpu()).abs().max() <= 2e-3
+        assert not chunk([0, 300, 1501], 4501) and (rows.cpu() == 7).all()
+        with pytest.raises(torch.OutOfMemoryError):
+            batch(8, 4501)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert chunk([0, 300, 1501], 4501)
