@@ -70,9 +70,9 @@ typedef struct pd_tensor {
  * Returns hipErrorInvalidValue unless heads_q == 6 * heads_kv, 1 <= qmax <= 4,
  * 1 <= nsplit <= nseg and num_seqs >= 1.
  * Here and in the other entries that run both kernels, a batch of several sequences for which
- * nsplit * heads_kv * num_seqs is above the CU count (and nseg >= 2, at most 32 rows per kv head)
- * is dealt evenly over the GPU by seq_lens instead: it may then use up to min(nseg, 128) segments
- * of the partial buffers rather than nsplit of them.
+ * nsplit * heads_kv * num_seqs is above the CU count (and at most 32 rows per kv head, and
+ * min(nseg, 128) > nsplit + nsplit / 8 or nsplit >= 16) is dealt evenly over the GPU by seq_lens instead: it
+ * may then use up to min(nseg, 128) segments of the partial buffers rather than nsplit of them.
  */
 hipError_t pth_dec_launch(const void* q, int q_st, const void* kc, int k_sb, int k_ss, int k_sh,
                           const int* block_table, int bt_stride, const int* seq_lens, const int* qsl,

@@ -1260,14 +1260,20 @@ static hipError_t launch_balanced_nrb(const PartialParams& p, int wgs, hipStream
 // (16 x 300 keys at 4 splits 11.5 us against 12.6, 64 x 4,096 at 1 split 109.2 against 111.3); past one
 // round the balanced kernel won at every batch measured (the figures at
 // pd_balanced_kernel) but at many short equal ones (128 x 1,024 keys at 1 split 74.4 against 77.3). More than one
-// sequence, since one alone is dealt evenly by pd_partial_kernel; at least two segments for the shares' ends;
+// sequence, since one alone is dealt evenly by pd_partial_kernel; segments to spare;
 // at most two row blocks (three do not fit the registers beside the line's state); and, with a block table of this width, a line of tiles that 32 bits number.
 static int balanced_segments(const LaunchArgs& x, int cus) {
     if ((int64_t)x.nsplit * x.heads_kv * x.num_seqs <= cus) return 0;
     const int64_t tiles = ((int64_t)x.bt_stride * x.block_size + kTile - 1) / kTile + 1;
     if (x.num_seqs < 2 || x.nseg < 2 || x.bt_stride < 1 || x.qmax * (x.heads_q / x.heads_kv) > 32) return 0;
     if (tiles > INT32_MAX || tiles * x.num_seqs > INT32_MAX / x.heads_kv) return 0;
-    return x.nseg < kMaxBalancedSegments ? x.nseg : kMaxBalancedSegments;
+    const int cap = x.nseg < kMaxBalancedSegments ? x.nseg : kMaxBalancedSegments;
+    // An item's pieces reach into one share more than they fill, so `cap` segments cut the longest sequence into
+    // cap - 1 full shares: below nsplit of them (and an eighth) it runs longer than in its nsplit splits
+    // (60,000 keys and 64 x 100, us, at nsplit = cap: 2: 475 against 823 dealt, 4: 236 / 290, 8: 123 / 133, 12: 72.5 / 81).
+    // From 16 splits on the empty splits of the short sequences cost more (16: 112 / 63).
+    if (x.nsplit < 16 && cap - 1 < x.nsplit + x.nsplit / 8) return 0;
+    return cap;
 }
 
 // The partial pass. `balanced` (may be null): allows pd_balanced_kernel, and says how many segments per row it

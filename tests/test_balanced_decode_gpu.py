@@ -88,3 +88,26 @@ def test_batches(name, causal):
     torch.cuda.synchronize()
     sel = torch.from_numpy(written).cuda()
     assert torch.equal(again[sel], out[sel])
+
+
+def dealt(parts, nsplit):
+    """Whether the call ran pd_balanced_kernel: only that writes more than nsplit segments of the partial buffers."""
+    return not parts[1][:, :, nsplit:].isnan().all().item()
+
+
+# segments, splits, whether the batch (65 sequences x 4 kv heads: past one round at any count) is dealt
+ROUTES = [(3, 2, True), (5, 4, True), (9, 8, False), (10, 8, True), (13, 12, False), (14, 12, True), (16, 15, False), (17, 16, True),
+          (100, 4, True)]
+
+
+@pytest.mark.parametrize("nseg,nsplit,deal", ROUTES)
+def test_few_segments_stay_with_the_splits(nseg, nsplit, deal):
+    """One long sequence among short ones is cut by the deal into at most one share less than there are segments: with
+    no segments to spare for that the launch keeps its splits."""
+    c = kvc.make_case([2000] + [5] * 64, [1] * 65, num_q_heads=24, num_kv_heads=4, block_size=16, seed=nseg)
+    d, out, parts = decode(c, nseg, nsplit)
+    assert dealt(parts, nsplit) == deal
+    ref, written = orc.paged_decode(c.q, c.cache.key_cache, c.cache.value_cache, c.cache.k_scale, c.cache.v_scale,
+                                    c.block_table, c.seq_lens, c.query_start_loc, c.num_seqs, c.scale, c.window, c.causal)
+    emax, emean, over, over_mean = kvc.fp16_output_errors(out.double().cpu().numpy()[written], ref[written])
+    assert over <= 0 and over_mean <= 2e-4, (emax, emean)
