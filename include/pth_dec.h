@@ -70,7 +70,7 @@ typedef struct pd_tensor {
  * Returns hipErrorInvalidValue unless heads_q == 6 * heads_kv, 1 <= qmax <= 4,
  * 1 <= nsplit <= nseg and num_seqs >= 1.
  * Here and in the other entries that run both kernels, a batch of several sequences for which
- * nsplit * heads_kv * num_seqs is above the CU count (and at most 32 rows per kv head, and
+ * nsplit * heads_kv * num_seqs is above the CU count (and nsplit >= 2, at most 32 rows per kv head, and
  * min(nseg, 128) > nsplit + nsplit / 8 or nsplit >= 16) is dealt evenly over the GPU by seq_lens instead: it
  * may then use up to min(nseg, 128) segments of the partial buffers rather than nsplit of them.
  */

@@ -1257,15 +1257,20 @@ static hipError_t launch_balanced_nrb(const PartialParams& p, int wgs, hipStream
 
 // Segments per item that a balanced launch may use (0: the batch is not one for it). A split count whose
 // workgroups fit one round of the CUs has been planned for the batch's lengths, and its kernel starts ~1.5 us earlier
-// (16 x 300 keys at 4 splits 11.5 us against 12.6, 64 x 4,096 at 1 split 109.2 against 111.3); past one
-// round the balanced kernel won at every batch measured (the figures at
-// pd_balanced_kernel) but at many short equal ones (128 x 1,024 keys at 1 split 74.4 against 77.3). More than one
+// (16 x 300 keys at 4 splits 11.5 us against 12.6, 64 x 4,096 at 1 split 109.2 against 111.3). Past one
+// round the balanced kernel won at every batch measured with two splits or more (24 q / 4 kv heads, us: 48 x 4,096 keys at
+// 2 splits 100 against 92, 64 of 500 to 4,000 at 2 58 / 48, 32 of 200 to 32,768 at 8 129 / 89). One split per
+// sequence past one round says that there are many sequences, where the hardware's own order of workgroups
+// is as even if they are short or alike (128 x 1,024 keys 57.5 against 59.9, 904 to 1,024 keys 55.7 / 64.2, 128 x 64
+// 21.3 / 25.9) and not if they are ragged or leave a round part-filled (160 of 100 to 3,000 keys 90 / 78, 70 x 8,192 316 / 228):
+// that only a caller that knows the lengths can tell, and it asks for the deal by passing 2 splits. More than one
 // sequence, since one alone is dealt evenly by pd_partial_kernel; segments to spare;
-// at most two row blocks (three do not fit the registers beside the line's state); and, with a block table of this width, a line of tiles that 32 bits number.
+// at most two row blocks (three do not fit the registers beside the line's state); and, with a block table of this
+// width, a line of tiles that 32 bits number.
 static int balanced_segments(const LaunchArgs& x, int cus) {
-    if ((int64_t)x.nsplit * x.heads_kv * x.num_seqs <= cus) return 0;
+    if (x.nsplit < 2 || (int64_t)x.nsplit * x.heads_kv * x.num_seqs <= cus) return 0;
     const int64_t tiles = ((int64_t)x.bt_stride * x.block_size + kTile - 1) / kTile + 1;
-    if (x.num_seqs < 2 || x.nseg < 2 || x.bt_stride < 1 || x.qmax * (x.heads_q / x.heads_kv) > 32) return 0;
+    if (x.num_seqs < 2 || x.bt_stride < 1 || x.qmax * (x.heads_q / x.heads_kv) > 32) return 0;
     if (tiles > INT32_MAX || tiles * x.num_seqs > INT32_MAX / x.heads_kv) return 0;
     const int cap = x.nseg < kMaxBalancedSegments ? x.nseg : kMaxBalancedSegments;
     // An item's pieces reach into one share more than they fill, so `cap` segments cut the longest sequence into

@@ -12,6 +12,9 @@
 #include <climits>
 #include <cmath>
 #include <exception>
+#include <functional>
+#include <queue>
+#include <vector>
 
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -267,8 +270,41 @@ PyObject* cache_write(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// The lengths of a batch on the host: a contiguous int32 or int64 CPU tensor.
+class Lengths {
+public:
+    // false with a Python error set
+    bool take(PyObject* o, int64_t num_seqs, int64_t max_q, int64_t window) {
+        if (!THPVariable_Check(o)) {
+            PyErr_SetString(PyExc_TypeError, "lens must be a tensor");
+            return false;
+        }
+        const at::Tensor& lens = THPVariable_Unpack(o);
+        wide_ = lens.scalar_type() == at::kLong;
+        if (!lens.device().is_cpu() || !lens.is_contiguous() || (!wide_ && lens.scalar_type() != at::kInt)) {
+            PyErr_SetString(PyExc_ValueError, "lens must be a contiguous int32 or int64 CPU tensor");
+            return false;
+        }
+        data_ = lens.const_data_ptr();
+        count = std::min<int64_t>(lens.numel(), num_seqs);
+        most_ = window > 0 ? window + max_q : INT64_MAX;
+        return true;
+    }
+    // visible keys of sequence i in 32-key tiles (+ 1: alignment)
+    int64_t tiles(int64_t i) const {
+        const int64_t len = std::min<int64_t>(wide_ ? static_cast<const int64_t*>(data_)[i] : static_cast<const int32_t*>(data_)[i], most_);
+        return len > 0 ? ceil_div(len, 32) + 1 : 0;
+    }
+    int64_t count = 0;
+
+private:
+    const void* data_ = nullptr;
+    bool wide_ = false;
+    int64_t most_ = INT64_MAX;
+};
+
 // plan_decode(lens, num_seqs, num_kv_heads, rows, max_q, window, cap, cus, tile_us, fixed_us, empty_us, merge_us_per_mb,
-//             row_bytes): vllm_shim.decode_splits' makespan model; lens is a contiguous int32 or int64 CPU tensor.
+//             row_bytes): vllm_shim.decode_splits' makespan model.
 PyObject* plan_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         int64_t num_seqs, hkv, rows, max_q, window, cap, cus;
@@ -278,33 +314,17 @@ PyObject* plan_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
             !as_double(a[8], tile_us) || !as_double(a[9], fixed_us) || !as_double(a[10], empty_us) ||
             !as_double(a[11], merge_us) || !as_double(a[12], row_bytes))
             return nullptr;
-        if (!THPVariable_Check(a[0])) {
-            PyErr_SetString(PyExc_TypeError, "lens must be a tensor");
-            return nullptr;
-        }
-        const at::Tensor& lens = THPVariable_Unpack(a[0]);
-        const bool wide = lens.scalar_type() == at::kLong;
-        if (!lens.device().is_cpu() || !lens.is_contiguous() || (!wide && lens.scalar_type() != at::kInt)) {
-            PyErr_SetString(PyExc_ValueError, "lens must be a contiguous int32 or int64 CPU tensor");
-            return nullptr;
-        }
-        const void* data = lens.const_data_ptr();
-        const int64_t count = std::min<int64_t>(lens.numel(), num_seqs);
-        // visible keys in 32-key tiles (+ 1: alignment)
-        auto tiles_of = [&](int64_t i) -> int64_t {
-            int64_t len = wide ? static_cast<const int64_t*>(data)[i] : static_cast<const int32_t*>(data)[i];
-            if (window > 0) len = std::min(len, window + max_q);
-            return len > 0 ? ceil_div(len, 32) + 1 : 0;
-        };
+        Lengths lens;
+        if (!lens.take(a[0], num_seqs, max_q, window)) return nullptr;
         bool live = false;
-        for (int64_t i = 0; i < count; ++i) live = live || tiles_of(i) > 0;
+        for (int64_t i = 0; i < lens.count; ++i) live = live || lens.tiles(i) > 0;
         if (!live) return PyLong_FromLong(1);
         int64_t best_s = cap;
         double best_t = HUGE_VAL;
         for (int64_t s = 1;; s = s * 2 < cap ? s * 2 : cap) {  // powers of two, and the cap
             double total = 0.0, longest = 0.0;
-            for (int64_t i = 0; i < count; ++i) {
-                const int64_t t = tiles_of(i), per = std::max<int64_t>(ceil_div(t, s), 1);
+            for (int64_t i = 0; i < lens.count; ++i) {
+                const int64_t t = lens.tiles(i), per = std::max<int64_t>(ceil_div(t, s), 1);
                 const int64_t filled = t > 0 ? ceil_div(t, per) : 0;  // splits holding tiles
                 const double us = fixed_us + tile_us * (double)ceil_div(per, 4);
                 total += (double)filled * us + (double)(s - filled) * empty_us;
@@ -316,6 +336,42 @@ PyObject* plan_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
             if (s >= cap) break;
         }
         return PyLong_FromLongLong(best_s);
+    });
+}
+
+// deal_pays(lens, num_seqs, num_kv_heads, max_q, window, cus): whether pd_balanced_kernel is rated faster than one unsplit
+// workgroup per (sequence, kv head), of which there are more than CUs. In tiles (a workgroup's set-up and
+// merge are kSegmentUnits = 12): the workgroups run in order on the CU that is free first, the kv heads of a
+// sequence side by side; the deal takes an equal share and, measured, 15 % and 8 tiles more (a share's ends, its second
+// segment, the planning on the device). us, unsplit against dealt (24 q / 4 kv heads), with the two ratings: 100 x 512
+// keys 34.8 / 38.1 (58 : 60), 160 x 1,024 91.7 / 91.7 (135 : 137), 96 x 2,048 100 / 94 (154 : 141), 256 of 16 to 4,096
+// 289 / 248, 70 x 8,192 316 / 228.
+PyObject* deal_pays(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return guarded([&]() -> PyObject* {
+        int64_t num_seqs, hkv, max_q, window, cus;
+        if (!count_is(n, 6) || !as_int64(a[1], num_seqs) || !as_int64(a[2], hkv) || !as_int64(a[3], max_q) ||
+            !as_int64(a[4], window) || !as_int64(a[5], cus))
+            return nullptr;
+        Lengths lens;
+        if (!lens.take(a[0], num_seqs, max_q, window)) return nullptr;
+        constexpr int64_t kSegment = 12;
+        const int64_t lanes = std::max<int64_t>(1, cus / std::max<int64_t>(1, hkv));
+        std::priority_queue<int64_t, std::vector<int64_t>, std::greater<int64_t>> busy;  // until when, of each lane
+        int64_t total = 0, span = 0;
+        for (int64_t i = 0; i < lens.count; ++i) {
+            const int64_t t = lens.tiles(i);
+            if (t == 0) continue;
+            int64_t at = t + kSegment;
+            total += at;
+            if ((int64_t)busy.size() == lanes) {
+                at += busy.top();
+                busy.pop();
+            }
+            busy.push(at);
+            span = std::max(span, at);
+        }
+        const double share = (double)total * (double)hkv / (double)cus;
+        return PyBool_FromLong((double)span > 1.15 * share + 8.0);
     });
 }
 
@@ -382,6 +438,7 @@ PyMethodDef methods[] = {
     PD_METHOD(prefill_balanced, "pth_fa_forward_balanced on torch tensors"),
     PD_METHOD(cache_write, "pth_cache_write on torch tensors"),
     PD_METHOD(plan_decode, "split count of a decode batch"),
+    PD_METHOD(deal_pays, "whether a batch of unsplit sequences is dealt instead"),
     PD_METHOD(plan_prefill, "key splits of a prefill launch"),
     {nullptr, nullptr, 0, nullptr},
 };

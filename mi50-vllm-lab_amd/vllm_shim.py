@@ -105,6 +105,27 @@ def sliced_splits(window: int, max_q: int, group: int, num_kv_heads: int, num_se
     return s if s >= 2 else 0
 
 
+def _host_lengths(lens) -> torch.Tensor:
+    """Host lengths as the planners read them: a contiguous int32 or int64 CPU tensor."""
+    if isinstance(lens, torch.Tensor) and lens.dtype in (torch.int32, torch.int64) and lens.device.type == "cpu" \
+            and lens.is_contiguous():
+        return lens
+    return torch.from_numpy(np.array(lens, dtype=np.int64).reshape(-1))
+
+
+def launched_splits(nsplit: int, nseg: int, window: int, num_kv_heads: int, num_seqs: int, device, seq_lens_host, max_q: int,
+                    num_q_heads: int) -> int:
+    """The split count to call the operator with where decode_splits plans `nsplit`: 2, which makes it deal the tiles of
+    all sequences over the GPU, instead of 1 for a batch of more than one round of workgroups that is rated faster
+    dealt. The operator leaves a split count of 1 to one workgroup per sequence and kv head, since it cannot
+    see the lengths."""
+    if (nsplit != 1 or seq_lens_host is None or min(nseg, PTH_DEC_SPLITS + 1) < 3 or num_kv_heads * num_seqs <= cu_count(device)
+            or max_q * (num_q_heads // num_kv_heads) > 32):
+        return nsplit
+    dealt = _pd.native().deal_pays(_host_lengths(seq_lens_host), num_seqs, num_kv_heads, max_q, window, cu_count(device))
+    return 2 if dealt else 1
+
+
 def decode_splits(nseg: int, window: int, num_kv_heads: int, num_seqs: int, device, seq_lens_host=None,
                   max_q: int = 1, num_q_heads: Optional[int] = None) -> int:
     """Splits per sequence for the decode operator, at most min(VLLM_GFX950_PTH_DEC_SPLITS, nseg).
@@ -128,10 +149,7 @@ def decode_splits(nseg: int, window: int, num_kv_heads: int, num_seqs: int, devi
         if window > 0:
             return max(1, min(cap, cus // max(1, num_kv_heads * num_seqs)))
         return cap
-    lens = seq_lens_host
-    if not (isinstance(lens, torch.Tensor) and lens.dtype in (torch.int32, torch.int64) and lens.device.type == "cpu"
-            and lens.is_contiguous()):
-        lens = torch.from_numpy(np.array(seq_lens_host, dtype=np.int64).reshape(-1))
+    lens = _host_lengths(seq_lens_host)
     rows = num_seqs * max(1, max_q) * (num_q_heads if num_q_heads else 6 * num_kv_heads)
     return _pd.native().plan_decode(lens, num_seqs, num_kv_heads, rows, max_q, window, cap, cus, SPLIT_TILE_US,
                                     SPLIT_FIXED_US, SPLIT_EMPTY_US, COMBINE_US_PER_MB, PARTIAL_ROW_BYTES)
@@ -256,12 +274,12 @@ class Gfx950Int8Attention:
         # for windowed rows).
         if seq_lens_host is not None and _capturing(query.device):
             seq_lens_host = None
+        batch = (segm_o.shape[2], self.window, self.num_kv_heads, seq_lens.shape[0], query.device, seq_lens_host,
+                 max(1, max_q), query.shape[1])
         self.pth_dec.decode(query, key_cache, value_cache, k_scale_cache, v_scale_cache, block_table, seq_lens,
                             query_start_loc, output, self.scale, segm_o, meta.softmax_segm_max,
                             meta.softmax_segm_expsum, seq_lens.shape[0], max(1, max_q),
-                            decode_splits(segm_o.shape[2], self.window, self.num_kv_heads, seq_lens.shape[0],
-                                          query.device, seq_lens_host, max(1, max_q), query.shape[1]),
-                            window=self.window, causal=True)
+                            launched_splits(decode_splits(*batch), *batch), window=self.window, causal=True)
         return True
 
     # -------------------------------------------------------------------------------------

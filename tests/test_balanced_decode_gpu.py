@@ -97,13 +97,14 @@ def dealt(parts, nsplit):
 
 # segments, splits, whether the batch (65 sequences x 4 kv heads: past one round at any count) is dealt
 ROUTES = [(3, 2, True), (5, 4, True), (9, 8, False), (10, 8, True), (13, 12, False), (14, 12, True), (16, 15, False), (17, 16, True),
-          (100, 4, True)]
+          (100, 4, True), (64, 1, False), (64, 2, True)]
 
 
 @pytest.mark.parametrize("nseg,nsplit,deal", ROUTES)
 def test_few_segments_stay_with_the_splits(nseg, nsplit, deal):
     """One long sequence among short ones is cut by the deal into at most one share less than there are segments: with
-    no segments to spare for that the launch keeps its splits."""
+    no segments to spare for that the launch keeps its splits. So does one split, past one round, of sequences whose
+    lengths only the caller knows."""
     c = kvc.make_case([2000] + [5] * 64, [1] * 65, num_q_heads=24, num_kv_heads=4, block_size=16, seed=nseg)
     d, out, parts = decode(c, nseg, nsplit)
     assert dealt(parts, nsplit) == deal

@@ -47,6 +47,49 @@ def test_decode_plan_equals_its_model(seed):
             assert shim.decode_splits(nseg, window, hkv, n, "cpu", given, max_q) == want
 
 
+def deal_model(lens, hkv, max_q, window, cus):
+    """pd_native.deal_pays: the workgroups in order on the CU that is free first, against an equal share."""
+    tiles = [-(-min(x, window + max_q if window > 0 else x) // 32) + 1 for x in lens if x > 0]
+    free = [0] * max(1, cus // hkv)
+    for t in tiles:
+        at = free.index(min(free))
+        free[at] += t + 12
+    return max(free) > 1.15 * hkv * sum(t + 12 for t in tiles) / cus + 8
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_deal_rating_equals_its_model(seed):
+    r = random.Random(seed)
+    seen = set()
+    for _ in range(150):
+        n, top = r.randint(1, r.choice([20, 130, 400])), r.choice([100, 1500, 20000])
+        lens = [r.choice([0, top, r.randint(1, top), top - r.randint(0, top // 8)]) for _ in range(n)] if r.random() < 0.5 else [top] * n
+        hkv, max_q, window, cus = r.choice([1, 2, 3, 8]), r.choice([1, 4]), r.choice([-1, 900]), r.choice([1, 40, 256])
+        want = deal_model(lens, hkv, max_q, window, cus)
+        for given in (torch.tensor(lens), torch.tensor(lens, dtype=torch.int32)):
+            assert pth_dec.native().deal_pays(given, n, hkv, max_q, window, cus) == want
+        seen.add(want)
+    assert seen == {False, True}
+
+
+# sequences' keys (24 q / 4 kv heads, one token), us in one workgroup per sequence and kv head, us dealt
+UNSPLIT_BATCHES = [([1024] * 128, 57.5, 59.9), ([64] * 128, 21.3, 25.9), ([512] * 256, 77.6, 82.3), ([256] * 512, 128.1, 144.9),
+                   ([1024 - 32 * (i % 16) for i in range(128)], 49.7, 55.4), ([1000] * 65, 46.6, 37.4), ([2048] * 96, 100.3, 94.2),
+                   ([8192] * 70, 316, 228), ([100 + 18 * (i * 37 % 160) for i in range(160)], None, 0)]
+
+
+@pytest.mark.parametrize("lens,unsplit,dealt", UNSPLIT_BATCHES)
+def test_unsplit_batches_are_launched_as_measured(lens, unsplit, dealt):
+    batch = (64, -1, 4, len(lens), "cpu", lens, 1, 24)
+    assert shim.decode_splits(*batch) == 1
+    want = 2 if unsplit is None or dealt < unsplit else 1
+    assert shim.launched_splits(1, *batch) == want
+    assert shim.launched_splits(1, 2, *batch[1:]) == 1            # no segments for the deal
+    assert shim.launched_splits(1, *batch[:5], None, 1, 24) == 1  # no lengths
+    assert shim.launched_splits(4, *batch) == 4
+    assert shim.launched_splits(1, *batch[:6], 8, 48) == 1        # more than 32 rows per kv head
+
+
 @pytest.mark.parametrize("seed", range(8))
 def test_prefill_plan_equals_its_model(seed):
     r = random.Random(seed)

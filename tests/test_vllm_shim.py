@@ -211,6 +211,20 @@ def test_graph_capture_ignores_host_lengths(ops, monkeypatch):
     assert ops.calls[-1][4] == 256 // (4 * nseq)  # windowed: one round of workgroups
 
 
+@pytest.mark.parametrize("lens,launched", [([1024] * 128, 1), ([100 + 18 * (i * 37 % 160) for i in range(160)], 2)],
+                         ids=["equal", "ragged"])
+def test_unsplit_batches_ask_for_the_deal_where_it_pays(ops, monkeypatch, lens, launched):
+    n = len(lens)
+    q, out, kc = tensors(n)
+    m = meta([1] * n, lens, nseg=16)
+    m.seq_lens_cpu = lens
+    assert impl().route(q, kc, kc, None, None, m, out, 1, n, lambda *x: pytest.fail("fallback"))
+    assert ops.calls[-1][4] == launched
+    monkeypatch.setattr(shim, "_capturing", lambda device: True)  # no lengths while capturing: the cap
+    assert impl().route(q, kc, kc, None, None, m, out, 1, n, lambda *x: pytest.fail("fallback"))
+    assert ops.calls[-1][4] == 16
+
+
 @pytest.mark.parametrize("why", ["no_segm", "too_many_tokens", "q_stride", "layout", "mid_q", "noncausal"])
 def test_decode_fallbacks(monkeypatch, why):
     f = FakeOps(layout_ok=why != "layout")
