@@ -901,7 +901,7 @@ __global__ void __launch_bounds__(kThreads, 1) pd_partial_kernel(const PartialPa
 // segments. 120,000 + 7 x 2,048 keys (4 tokens): 119 / 90.7 / 70.3 us. Equal lengths take the aligned split, which
 // has no second segment (16 x 8,192 keys, 4 tokens: 192 / 68.4 / 65.9).
 // Segment s of an item is its s-th workgroup; the last one marks the item's other segments (up to
-// a.nsplit) empty, so the partial buffers mean the same as after pd_partial_kernel.
+// a.nsplit) empty (m = -inf, l = 0), so the partial buffers mean the same as after pd_partial_kernel.
 constexpr unsigned kSegmentUnits = 12;  // set-up and merge of a segment, ~10 us, in tiles of a workgroup (~0.8 us each)
 constexpr unsigned kSnapTiles = 6;      // a share's end this close to an item's boundary moves onto it
 
@@ -1012,14 +1012,16 @@ __global__ void __launch_bounds__(kThreads, 1) pd_balanced_kernel(const PartialP
         wk.te = wk.t_first + (int)last;
         wk.W = 0;
         wk.interleave = false;
+        partial_body<NRB, kFast>(a, wk, lds);
         if (last == (unsigned)wk.ntiles) {  // the item's last workgroup: no other segments
             const int R = min(16 * NRB, min(wk.q_len, a.qmax) * a.G), spare = a.nsplit - 1 - wk.seg;
             for (int k = threadIdx.x; k < R * spare; k += kThreads) {
                 const int r = k / spare, i = r / a.G, hh = r - i * a.G;
-                a.part_m[((int64_t)(wk.q0 + i) * a.Hq + (wk.g * a.G + hh)) * a.nseg + wk.seg + 1 + (k - r * spare)] = kNegInf;
+                const int64_t pr = ((int64_t)(wk.q0 + i) * a.Hq + (wk.g * a.G + hh)) * a.nseg + wk.seg + 1 + (k - r * spare);
+                a.part_m[pr] = kNegInf;
+                a.part_l[pr] = 0.f;
             }
         }
-        partial_body<NRB, kFast>(a, wk, lds);
         if (aligned || last < (unsigned)wk.ntiles) return;
         pos = (first ? pos - first - kSegmentUnits : pos) + units_of((unsigned)wk.ntiles);  // the next item
         if (pos >= end) return;

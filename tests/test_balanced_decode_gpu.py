@@ -112,3 +112,7 @@ def test_few_segments_stay_with_the_splits(nseg, nsplit, deal):
                                     c.block_table, c.seq_lens, c.query_start_loc, c.num_seqs, c.scale, c.window, c.causal)
     emax, emean, over, over_mean = kvc.fp16_output_errors(out.double().cpu().numpy()[written], ref[written])
     assert over <= 0 and over_mean <= 2e-4, (emax, emean)
+    # either way every segment of the launch is written, the empty ones with m = -inf and l = 0
+    m, l = (t[:, :, :min(nseg, 128) if deal else nsplit] for t in parts[1:])
+    assert not m.isnan().any() and not l.isnan().any()
+    assert (nsplit == 1 or (m == float("-inf")).any()) and (l[m == float("-inf")] == 0).all() and (l[m > float("-inf")] > 0).all()
