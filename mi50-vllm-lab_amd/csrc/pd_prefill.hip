@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "pd_plan.hpp"
 #include "pd_tile.hpp"
 #include "pth_dec.h"
 
@@ -651,8 +652,6 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
 // splits) against 184; a batch of 9 decoded sequences and chunks of 70 to 900 tokens over 1,500 to
 // 6,000 keys 481 -> 302 (four launches, with a transpose and two conversions each, before). Where all
 // query tiles need the same (2,048 tokens over 61,440) the splits' kernel is 3 % faster and is taken.
-constexpr unsigned kFaSegmentUnits = 10;  // set-up and stores of a segment, ~16 us, in key tiles (1.62 us)
-constexpr unsigned kFaMinShare = 16;      // units of a workgroup: below, pieces cost more than they save
 constexpr unsigned kFaMaxPieces = 64;     // pieces of an item (the merge holds one per lane)
 
 struct FaLine {
@@ -714,7 +713,7 @@ __device__ __forceinline__ FaLine fa_line(const FaParams& a, const FaRowsParams&
     // an item reaches into at most ceil(units / share) + 1 <= kFaMaxPieces shares
     n.share = max(max((n.total + n.nwg - 1) / n.nwg, (fa_units(n.longest) + kFaMaxPieces - 3) / (kFaMaxPieces - 2)), kFaMinShare);
     n.ns = min(min(n.nwg / items, kFaMaxPieces), max(1u, n.longest / 8));
-    n.aligned = n.nwg >= items && (n.longest + n.ns - 1) / n.ns <= n.share + n.share / 32;
+    n.aligned = n.nwg >= items && (n.longest + n.ns - 1) / n.ns <= n.share + n.share / kFaAlignedPart;
     n.snap = min(8u, n.share / 8);
     n.lead = kFaSegmentUnits + n.snap;
     return n;
@@ -948,13 +947,10 @@ template <class T>
 static hipError_t launch_prefill_type(const FaParams& p, int batch, int heads_kv, hipStream_t stream, bool exact) {
     const dim3 grid(((p.Sq + p.tok_per_wg - 1) / p.tok_per_wg) * p.nsplit, heads_kv, batch);
     const bool fast = fast_block_table(p.block_size, p.k_ss);
-    // 256-row workgroups where they take less time for all rounds of one workgroup per CU: a tile of theirs takes
-    // 1.85 us (2.2 exact) against 1.62 (1.9), so they have to save a round (2,048 tokens x 4 splits, 24 q / 4 kv heads:
-    // 3 rounds of 256 against 4, 2.92 ms against 3.30; 2,048 unsplit: one round of either, 3.7 against 3.15)
     const int64_t cus = std::max(1, compute_units(stream)), each = (int64_t)p.nsplit * heads_kv * batch;
     const int64_t rounds = ((int64_t)((p.Sq + p.tok_per_wg - 1) / p.tok_per_wg) * each + cus - 1) / cus;
     const int64_t wide_rounds = (((int64_t)p.Sq * p.G + kFwRows - 1) / kFwRows * each + cus - 1) / cus;
-    const bool wide = (double)wide_rounds * (exact ? 2.2 / 1.9 : 1.85 / 1.62) < (double)rounds;
+    const bool wide = fa_wide_saves(wide_rounds, rounds, exact);
     if (p.nsplit == 1) {
         if (wide)
             return launch_prefill_wide(p, batch, heads_kv, std::is_same<T, float>::value ? PD_DTYPE_FP32 : PD_DTYPE_FP16,

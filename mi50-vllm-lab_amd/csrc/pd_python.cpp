@@ -21,6 +21,7 @@
 #include <ATen/ops/empty.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include "pd_plan.hpp"
 #include "pth_dec.h"
 
 namespace {
@@ -375,56 +376,54 @@ PyObject* deal_pays(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
-// plan_prefill(work_items, rows, max_keys, block_size, cus, tile_us, wg_us, mb_us, merge_us, max_splits, min_tiles,
-//              max_workspace, lds_table, global_factor, sq, tok_per_wg, rows per kv head): pth_dec.prefill_splits' makespan model. With sq > 0
-// (the chunk's query tokens, the last of max_keys keys) 0 where the balanced launch is rated at least 5 %
-// faster: a workgroup's share of the line and, measured, up to 20 more units (a share's ends fall on items' starts, and
-// its last segment's set-up is its own) of 1.72 us, plus 20 us of planning and merge. Equal query tiles
-// (the kernel's aligned split) stay with the splits, whose kernel takes 3 % less per tile.
+// plan_prefill(work_items, rows, max_keys, block_size, cus, wg_us, mb_us, merge_us, max_splits, min_tiles, max_workspace,
+//              lds_table, global_factor, sq, tok_per_wg, rows per kv head, exact): pth_dec.prefill_splits' makespan model, with
+// the tile times of pd_plan.hpp. With sq > 0 (the chunk's query tokens, the last of max_keys keys) the 256-row kernel, at the
+// counts where the launch takes it, is rated as well, and the result is 0 where the balanced launch is rated
+// faster. Equal query tiles (the kernel's aligned split) stay with the splits, whose kernel takes less per tile.
 PyObject* plan_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
-        int64_t v[6], max_splits, min_tiles, max_workspace, lds_table;
-        double tile_us, wg_us, mb_us, merge_us, factor;
-        int64_t sq, tok;
-        if (!count_is(n, 17) || !as_int64(a[14], sq) || !as_int64(a[15], tok) || !as_int64(a[16], v[5])) return nullptr;
-        for (int i = 0; i < 5; ++i)
-            if (!as_int64(a[i], v[i])) return nullptr;
-        if (!as_double(a[5], tile_us) || !as_double(a[6], wg_us) || !as_double(a[7], mb_us) || !as_double(a[8], merge_us) ||
-            !as_int64(a[9], max_splits) || !as_int64(a[10], min_tiles) || !as_int64(a[11], max_workspace) ||
-            !as_int64(a[12], lds_table) || !as_double(a[13], factor))
+        int64_t items, rows, max_keys, block_size, cus, max_splits, min_tiles, max_workspace, lds_table, sq, tok, head_rows, exact;
+        double wg_us, mb_us, merge_us, factor;
+        if (!count_is(n, 17) || !as_int64(a[0], items) || !as_int64(a[1], rows) || !as_int64(a[2], max_keys) ||
+            !as_int64(a[3], block_size) || !as_int64(a[4], cus) || !as_double(a[5], wg_us) || !as_double(a[6], mb_us) ||
+            !as_double(a[7], merge_us) || !as_int64(a[8], max_splits) || !as_int64(a[9], min_tiles) ||
+            !as_int64(a[10], max_workspace) || !as_int64(a[11], lds_table) || !as_double(a[12], factor) || !as_int64(a[13], sq) ||
+            !as_int64(a[14], tok) || !as_int64(a[15], head_rows) || !as_int64(a[16], exact))
             return nullptr;
-        const int64_t items = v[0], rows = v[1], keys = std::max<int64_t>(0, v[2]), bs = std::max<int64_t>(1, v[3]), cus = v[4];
-        const int64_t tiles = ceil_div(keys, 32);
-        auto cost = [&](int64_t s) {
-            const int64_t rounds = ceil_div(items * s, cus), per = ceil_div(tiles, s);
-            const bool in_lds = v[3] % 16 == 0 ? 2 * per <= lds_table : ceil_div(keys, bs) <= lds_table;
+        const pd::FaTimes& times = pd::fa_times(exact != 0);
+        const int64_t keys = std::max<int64_t>(0, max_keys), bs = std::max<int64_t>(1, block_size), tiles = ceil_div(keys, 32);
+        // `count` workgroups per split, of which each takes `tile_us` per tile
+        auto cost = [&](int64_t count, int64_t s, double tile_us) {
+            const int64_t rounds = ceil_div(count * s, cus), per = ceil_div(tiles, s);
+            const bool in_lds = block_size % 16 == 0 ? 2 * per <= lds_table : ceil_div(keys, bs) <= lds_table;
             double t = (double)rounds * ((double)per * (tile_us * (in_lds ? 1.0 : factor)) + wg_us);
             if (s > 1) t += merge_us + mb_us * (double)rows * (double)s * 1032 / 1e6;
             return t;
         };
-        int64_t best = 1;
-        double best_t = cost(1);
         const int64_t top = std::max<int64_t>(1, std::min(max_splits, tiles / min_tiles));
-        for (int64_t s = 2; s <= top && rows * s * 1032 <= max_workspace; ++s) {
-            const double t = cost(s);
+        auto fits = [&](int64_t s) { return s == 1 || rows * s * 1032 <= max_workspace; };
+        int64_t best = 1;
+        double best_t = cost(items, 1, times.tile);
+        for (int64_t s = 2; s <= top && fits(s); ++s) {
+            const double t = cost(items, s, times.tile);
             if (t < best_t) best = s, best_t = t;
         }
         if (sq > 0 && items > 0) {
-            // the 256-row kernel, which the launch takes where that saves rounds: 1.85 us per tile
-            const int64_t wide_items = ceil_div(v[5], 256) * (items / ceil_div(sq, std::max<int64_t>(1, tok)));
-            for (int64_t s = 1; s <= top && (s == 1 || rows * s * 1032 <= max_workspace); ++s) {
-                const int64_t rounds = ceil_div(wide_items * s, cus), per = ceil_div(tiles, s);
-                if ((double)rounds * (1.85 / 1.62) >= (double)ceil_div(items * s, cus)) continue;
-                double t = (double)rounds * ((double)per * 1.85 + wg_us);
-                if (s > 1) t += merge_us + mb_us * (double)rows * (double)s * 1032 / 1e6;
+            const int64_t nqt = ceil_div(sq, std::max<int64_t>(1, tok)), heads = items / nqt;
+            const int64_t wide_items = ceil_div(head_rows, 256) * heads;
+            for (int64_t s = 1; s <= top && fits(s); ++s) {
+                if (!pd::fa_wide_saves(ceil_div(wide_items * s, cus), ceil_div(items * s, cus), exact != 0)) continue;
+                const double t = cost(wide_items, s, times.wide_tile);
                 if (t < best_t) best = s, best_t = t;
             }
-            const int64_t nqt = ceil_div(sq, std::max<int64_t>(1, tok)), heads = items / nqt;
             int64_t units = 0;
-            for (int64_t q = 0; q < nqt; ++q) units += ceil_div(std::max<int64_t>(0, keys - sq) + std::min(sq, (q + 1) * tok), 32) + 10;
-            const int64_t share = std::max<int64_t>(16, ceil_div(units * heads, cus)), ns = items <= cus ? cus / items : 0;
-            const bool aligned = ns > 0 && ceil_div(tiles, ns) <= share + share / 32;
-            if (!aligned && 1.72 * (double)(share + 20) + 20.0 < 0.95 * best_t) best = 0;
+            for (int64_t q = 0; q < nqt; ++q)
+                units += ceil_div(std::max<int64_t>(0, keys - sq) + std::min(sq, (q + 1) * tok), 32) + pd::kFaSegmentUnits;
+            const int64_t share = std::max<int64_t>(pd::kFaMinShare, ceil_div(units * heads, cus)), ns = items <= cus ? cus / items : 0;
+            const bool aligned = ns > 0 && ceil_div(tiles, ns) <= share + share / pd::kFaAlignedPart;
+            const double dealt = times.deal_unit * (double)(share + pd::kFaDealSpareUnits) + pd::kFaDealFixedUs;
+            if (!aligned && dealt < pd::kFaDealMargin * best_t) best = 0;
         }
         return PyLong_FromLongLong(best);
     });

@@ -256,15 +256,15 @@ def prefill_splits(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: i
     return _prefill_plan(batch, sq, heads_q, heads_kv, max_keys, block_size, 0)
 
 
-def _prefill_plan(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: int, block_size: int, chunk: int) -> int:
-    """prefill_splits' count; with chunk = sq (query tokens that are the last of max_keys keys) 0 where the
-    balanced launch is rated faster."""
+def _prefill_plan(batch: int, sq: int, heads_q: int, heads_kv: int, max_keys: int, block_size: int, chunk: int,
+                  exact: bool = False) -> int:
+    """prefill_splits' count; with chunk = sq (query tokens that are the last of max_keys keys) the count for either
+    kernel in the call's numerics, 0 where the balanced launch is rated faster."""
     tok = max(1, PREFILL_ROWS_PER_WORKGROUP // max(1, heads_q // heads_kv))
     return native().plan_prefill(-(-sq // tok) * heads_kv * batch, batch * sq * heads_q, max_keys, block_size, PREFILL_CUS,
-                                 PREFILL_US_PER_TILE, PREFILL_US_PER_WORKGROUP, PREFILL_US_PER_PARTIAL_MB,
-                                 PREFILL_US_MERGE_LAUNCH, PREFILL_MAX_SPLITS, PREFILL_MIN_TILES_PER_SPLIT,
-                                 PREFILL_MAX_WORKSPACE, PREFILL_LDS_TABLE, PREFILL_GLOBAL_TABLE_FACTOR, chunk, tok,
-                                 sq * (heads_q // heads_kv))
+                                 PREFILL_US_PER_WORKGROUP, PREFILL_US_PER_PARTIAL_MB, PREFILL_US_MERGE_LAUNCH,
+                                 PREFILL_MAX_SPLITS, PREFILL_MIN_TILES_PER_SPLIT, PREFILL_MAX_WORKSPACE, PREFILL_LDS_TABLE,
+                                 PREFILL_GLOBAL_TABLE_FACTOR, chunk, tok, sq * (heads_q // heads_kv), 1 if exact else 0)
 
 
 def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, block_table: torch.Tensor,
@@ -300,7 +300,7 @@ def forward_pth(q: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Ten
         nsplit = 1
         if batch > 0 and sq > 0 and heads_q > 0 and heads_kv > 0:
             block_size = key_cache.shape[1] if key_cache.dim() == 4 else 16
-            nsplit = _prefill_plan(batch, sq, heads_q, heads_kv, int(max_keys), block_size, sq)
+            nsplit = _prefill_plan(batch, sq, heads_q, heads_kv, int(max_keys), block_size, sq, exact)
             if nsplit == 0 and native().prefill_balanced(
                     _entry("pth_fa_forward_balanced"), _entry("pth_fa_balanced_workspace"), q, key_cache, value_cache,
                     block_table, seq_lens, scale, q_abs_offset, out, None, int(max_keys), 0, 1 if exact else 0):
@@ -341,7 +341,7 @@ def forward_rows(query: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
         return False
     nsplit, rows, heads_kv = 0, query_start[-1] - query_start[0], key_cache.shape[2]
     if len(query_start) == 2 and rows > 0 and heads_kv > 0 and query.shape[1] > 0:
-        nsplit = _prefill_plan(1, rows, query.shape[1], heads_kv, max_keys, key_cache.shape[1], rows)
+        nsplit = _prefill_plan(1, rows, query.shape[1], heads_kv, max_keys, key_cache.shape[1], rows, exact)
     one = len(query_start) == 2 and rows > 0
     for n in (nsplit, 1) if one and nsplit != 1 else (nsplit,):  # (a single chunk without its workspace: unsplit)
         if native().prefill_balanced(_entry("pth_fa_forward_balanced"), _entry("pth_fa_balanced_workspace"), query,

@@ -2,7 +2,9 @@
 Python exceptions that the operators document. The calls themselves are covered by every GPU test.
 """
 import math
+import os
 import random
+import re
 
 import numpy as np
 import pytest
@@ -101,6 +103,70 @@ def test_prefill_plan_equals_its_model(seed):
         top = max(1, min(pth_dec.PREFILL_MAX_SPLITS, -(-a[4] // 32) // pth_dec.PREFILL_MIN_TILES_PER_SPLIT))
         counts = [s for s in range(1, top + 1) if s == 1 or a[0] * a[1] * a[2] * s * 1032 <= pth_dec.PREFILL_MAX_WORKSPACE]
         assert pth_dec.prefill_splits(*a, bs) == min(counts, key=lambda s: pth_dec.prefill_cost_us(*a, s, bs))
+
+
+PLAN = open(os.path.join(os.path.dirname(pth_dec.__file__), "csrc", "pd_plan.hpp")).read()
+TIMES = {e: [float(x) for x in re.search(r"constexpr FaTimes %s = \{(.*?)\}" % n, PLAN).group(1).split(",")]
+         for e, n in ((False, "kFaTimes"), (True, "kFaTimesExact"))}
+SEGMENT, MIN_SHARE, ALIGNED, SPARE, DEAL_US, MARGIN = (
+    float(re.search(r"constexpr \w+ %s = ([\d.]+);" % n, PLAN).group(1))
+    for n in ("kFaSegmentUnits", "kFaMinShare", "kFaAlignedPart", "kFaDealSpareUnits", "kFaDealFixedUs", "kFaDealMargin"))
+
+
+def chunk_model(batch, sq, hq, hkv, keys, bs, exact, cus=256):
+    """pd_native.plan_prefill for a chunk whose tokens are the last of `keys` keys: {split count: (us, kernel)}, and the
+    us of the dealt launch (None where it would cut the query tiles evenly)."""
+    tile, wide, unit = TIMES[exact]
+    g, tiles = hq // hkv, -(-keys // 32)
+    tok = 192 // g
+    qtiles = -(-sq // tok)
+    items, wide_items, rows = qtiles * hkv * batch, -(-sq * g // 256) * hkv * batch, batch * sq * hq
+    out = {}
+    for s in range(1, max(1, min(64, tiles // 8)) + 1):
+        if s > 1 and rows * s * 1032 > pth_dec.PREFILL_MAX_WORKSPACE:
+            break
+        per = -(-tiles // s)
+        table = 2 * per if bs % 16 == 0 else -(-keys // bs)
+        slow = 1.0 if table <= pth_dec.PREFILL_LDS_TABLE else pth_dec.PREFILL_GLOBAL_TABLE_FACTOR
+        rounds, wide_rounds = -(-items * s // cus), -(-wide_items * s // cus)
+        merge = pth_dec.PREFILL_US_MERGE_LAUNCH + pth_dec.PREFILL_US_PER_PARTIAL_MB * rows * s * 1032 / 1e6 if s > 1 else 0.0
+        times = {192: rounds * (per * tile * slow + pth_dec.PREFILL_US_PER_WORKGROUP) + merge}
+        if wide_rounds * wide < rounds * tile:
+            times[256] = wide_rounds * (per * wide * slow + pth_dec.PREFILL_US_PER_WORKGROUP) + merge
+        out[s] = min((t, k) for k, t in times.items())
+    units = sum(-(-(max(0, keys - sq) + min(sq, (q + 1) * tok)) // 32) + SEGMENT for q in range(qtiles)) * hkv * batch
+    share = max(MIN_SHARE, -(-units // cus))
+    ns = cus // items
+    if ns and -(-tiles // ns) <= share + share // ALIGNED:
+        return out, None
+    return out, unit * (share + SPARE) + DEAL_US
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["default", "exact"])
+@pytest.mark.parametrize("seed", range(4))
+def test_chunk_plan_equals_its_model(seed, exact):
+    r, seen = random.Random(seed), set()
+    for _ in range(120):
+        hkv = r.choice([1, 2, 4, 8])
+        batch, hq, sq = r.choice([1, 1, 3]), hkv * r.choice([1, 4, 6, 8]), r.choice([r.randint(1, 100), r.randint(1, 6000), 2048])
+        keys, bs = sq + r.choice([0, r.randint(1, 2000), r.randint(1, 300000)]), r.choice([1, 8, 16, 48, 1584])
+        counts, dealt = chunk_model(batch, sq, hq, hkv, keys, bs, exact)
+        best = min(t for t, _ in counts.values())
+        got = pth_dec._prefill_plan(batch, sq, hq, hkv, keys, bs, sq, exact)
+        assert (got == 0) == (dealt is not None and dealt < MARGIN * best), (counts, dealt, got)
+        if got:
+            assert counts[got][0] == pytest.approx(best, rel=1e-12)
+        seen.add(0 if got == 0 else counts[got][1])
+    assert seen == {0, 192, 256}  # every kernel is planned somewhere
+
+
+def test_plan_and_launch_share_the_tile_times():
+    assert TIMES[False][0] == pth_dec.PREFILL_US_PER_TILE
+    csrc = os.path.join(os.path.dirname(pth_dec.__file__), "csrc")
+    assert "fa_wide_saves(wide_rounds, rounds, exact)" in open(os.path.join(csrc, "pd_prefill.hip")).read()
+    # an exact call is rated with its own times: here a 256-row count that saves a round by the default's ratio only
+    tile, wide, _ = TIMES[True]
+    assert wide / tile > TIMES[False][1] / TIMES[False][0]
 
 
 def test_errors_become_python_exceptions():
