@@ -550,10 +550,11 @@ __device__ __forceinline__ void prefill_body(const FaParams& a, const FaWork& wk
                 tile_back(n, sv, vs);
             }
         };
-        // The interior loop starts a fixed distance past a 64-byte line: one wave per SIMD feels where its 7 KB
-        // of code lie in the instruction fetch. Of 16 distances, 2,048 tokens over 61,440 keys took 3.23
-        // (here) to 3.36 ms, 2,560 in 4 splits 4.10 (here) to 4.41.
-        asm volatile(".p2align 6\n\ts_nop 0" ::: "memory");
+        // pd_prefill_kernel starts the interior loop a fixed distance past a 64-byte line: one wave per SIMD feels where
+        // its 7 KB of code lie in the instruction fetch. us without and with, of launches that run it: 900 tokens over
+        // 20,000 keys 590 / 551, 900 over 900 84 / 81, 2,000 fresh ones 122 / 118, exact 2,048 over 16,384 (12 / 2
+        // heads) 625 / 623. The dealt launch showed no difference (300.8 with and without).
+        if constexpr (kParts != 2) asm volatile(".p2align 6\n\ts_nop 0" ::: "memory");
         run(std::false_type{}, t0, min(n_int, t1));
         run(std::true_type{}, max(n_int, t0), t1);
     };
