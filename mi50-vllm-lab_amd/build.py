@@ -46,6 +46,7 @@ def build(save_temps: str | None = None, verbose: bool = False) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     tmp = LIB_PATH + ".tmp"
     if save_temps:
+        save_temps = os.path.abspath(save_temps)  # the compilers run in it
         os.makedirs(save_temps, exist_ok=True)
     with tempfile.TemporaryDirectory() as objdir:
         # one compiler per source, side by side (the prefill kernels take longest)

@@ -147,3 +147,21 @@ def test_halves_of_a_register_are_not_written_back_to_back(gfx950_asm):
             if "UNUSED_PRESERVE" in text and "_sdwa" in last:
                 assert text.split()[1] != last.split()[1], (last, text)
             last = text
+
+
+def test_save_temps_takes_a_relative_directory(tmp_path, monkeypatch):
+    # a stand-in compiler that writes its output where it runs and links only what is there
+    cc = tmp_path / "hipcc"
+    cc.write_text('#!/bin/sh\nfor a in "$@"; do case "$a" in *.o) [ "$last" = -o ] || [ -f "$a" ] || exit 3;; esac; last=$a; done\n'
+                  'while [ "$1" != -o ]; do shift; done\necho built > "$2"\n')
+    cc.chmod(0o755)
+    monkeypatch.setenv("HIPCC", str(cc))
+    monkeypatch.syspath_prepend(PKG_DIR)
+    monkeypatch.chdir(tmp_path)
+    import build as pd_build
+    monkeypatch.setattr(pd_build, "LIB_DIR", str(tmp_path / "lib"))
+    monkeypatch.setattr(pd_build, "LIB_PATH", str(tmp_path / "lib" / "libpthdec.so"))
+    for d in ("temps", str(tmp_path / "absolute"), None):
+        assert open(pd_build.build(d)).read() == "built\n"
+        if d:
+            assert len([f for f in os.listdir(tmp_path / d) if f.endswith(".o")]) == len(pd_build.SOURCES)
