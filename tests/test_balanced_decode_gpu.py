@@ -5,7 +5,8 @@ split-per-sequence launches pth_dec_launch_partial and pth_dec_launch_combine.
 The batches are those at whose edges the deal can go wrong: sequences of one key, of exactly one
 tile and of one key more, empty ones, one long sequence among short ones (its segments at the cap of the
 partial buffers), equal lengths (cut evenly, one workgroup each), more sequences than a wave's lanes, more
-items than workgroups. Every partial buffer starts as NaN: a segment that nobody wrote must not be read.
+items than workgroups. Each is launched at a split count that the operator deals, which the test sees in the segments
+written. Every partial buffer starts as NaN: a segment that nobody wrote must not be read.
 """
 import numpy as np
 import pytest
@@ -19,22 +20,22 @@ pytestmark = pytest.mark.gpu
 
 MIXED = [1, 31, 32, 33, 700, 5000, 97, 12000]
 BATCHES = {
-    # name: contexts, query tokens, (q heads, kv heads), block size, segments, window
-    "mixed": (MIXED, [1] * 8, (24, 4), 16, 64, -1),
-    "mixed_mtp_two_row_blocks": (MIXED, [4, 0, 1, 2, 4, 3, 0, 4], (24, 4), 16, 64, -1),
-    "long_among_short_at_two_segments": ([40000, 10, 900, 64], [1, 1, 1, 1], (12, 2), 16, 2, -1),
-    "long_among_short_at_five_segments": ([30000, 10, 900, 64], [2, 1, 2, 1], (24, 4), 32, 5, -1),
-    "more_segments_than_lanes": ([60000, 10, 300], [1, 1, 1], (6, 1), 16, 100, -1),
-    "equal": ([2048] * 6, [1] * 6, (24, 4), 16, 64, -1),
-    "equal_reference_blocks": ([3000] * 3, [4] * 3, (12, 2), 1584, 16, -1),
-    "nearly_equal_many_items": ([500 + 3 * (i % 7) for i in range(70)], [1] * 70, (32, 8), 16, 64, -1),
-    "lanes_plus_one": ([(i * 37) % 400 for i in range(65)], [1 + i % 2 for i in range(65)], (8, 2), 16, 64, -1),
-    "more_than_two_waves_of_sequences": ([(i * 53) % 230 + 1 for i in range(130)], [1] * 130, (8, 2), 16, 16, -1),
-    "no_query_tokens_but_one": ([500, 900, 40], [0, 3, 0], (24, 4), 16, 64, -1),
-    "pages_not_of_16": (MIXED, [1] * 8, (24, 4), 8, 64, -1),
-    "pages_of_one": ([1, 31, 33, 2000, 97], [2] * 5, (24, 4), 1, 7, -1),
-    "window": (MIXED, [1, 2, 1, 2, 1, 2, 1, 2], (24, 4), 16, 64, 512),
-    "window_past_the_sliced_size": ([9000, 100, 20000, 31], [4] * 4, (24, 4), 16, 64, 8192),
+    # name: contexts, query tokens, (q heads, kv heads), block size, segments, splits (x kv heads x sequences above 256), window
+    "mixed": (MIXED, [1] * 8, (24, 4), 16, 64, 16, -1),
+    "mixed_mtp_two_row_blocks": (MIXED, [4, 0, 1, 2, 4, 3, 0, 4], (24, 4), 16, 64, 16, -1),
+    "long_among_short_at_three_segments": ([40000, 10, 900, 64] + [9] * 130, [1] * 134, (12, 2), 16, 3, 2, -1),
+    "long_among_short_at_five_segments": ([30000, 10, 900, 64] + [40] * 13, [2, 1, 2, 1] + [1] * 13, (24, 4), 32, 5, 4, -1),
+    "more_segments_than_lanes": ([60000, 10, 300], [1, 1, 1], (6, 1), 16, 128, 100, -1),
+    "equal": ([2048] * 6, [1] * 6, (24, 4), 16, 64, 16, -1),
+    "equal_reference_blocks": ([3000] * 3, [4] * 3, (12, 2), 1584, 64, 48, -1),
+    "nearly_equal_many_items": ([500 + 3 * (i % 7) for i in range(70)], [1] * 70, (32, 8), 16, 64, 4, -1),
+    "lanes_plus_one": ([(i * 37) % 400 for i in range(65)], [1 + i % 2 for i in range(65)], (8, 2), 16, 64, 4, -1),
+    "more_than_two_waves_of_sequences": ([(i * 53) % 230 + 1 for i in range(130)], [1] * 130, (8, 2), 16, 16, 4, -1),
+    "no_query_tokens_but_one": ([500, 900, 40], [0, 3, 0], (24, 4), 16, 64, 32, -1),
+    "pages_not_of_16": (MIXED, [1] * 8, (24, 4), 8, 64, 16, -1),
+    "pages_of_one": ([1, 31, 33, 2000, 97] + [20 + i for i in range(15)], [2] * 20, (24, 4), 1, 7, 5, -1),
+    "window": (MIXED, [1, 2, 1, 2, 1, 2, 1, 2], (24, 4), 16, 64, 16, 512),
+    "window_past_the_sliced_size": ([9000, 100, 20000, 31], [4] * 4, (24, 4), 16, 64, 32, 8192),
 }
 
 
@@ -47,6 +48,11 @@ def decode(c, nseg, nsplit):
                    d.seq_lens, d.query_start_loc, out, d.scale, *parts, d.num_seqs, d.qmax, nsplit, d.window, d.causal)
     torch.cuda.synchronize()
     return d, out, parts
+
+
+def dealt(parts, nsplit):
+    """Whether the call ran pd_balanced_kernel: only that writes more than nsplit segments of the partial buffers."""
+    return not parts[1][:, :, nsplit:].isnan().all().item()
 
 
 def general_path(d, nseg, nsplit):
@@ -65,14 +71,14 @@ def general_path(d, nseg, nsplit):
 @pytest.mark.parametrize("causal", [True, False], ids=["causal", "all_keys"])
 @pytest.mark.parametrize("name", list(BATCHES))
 def test_batches(name, causal):
-    ctxs, qlens, (hq, hkv), bs, nseg, window = BATCHES[name]
+    ctxs, qlens, (hq, hkv), bs, nseg, nsplit, window = BATCHES[name]
     c = kvc.make_case(ctxs, qlens, num_q_heads=hq, num_kv_heads=hkv, block_size=bs, seed=len(name), window=window,
                       causal=causal, layout="NHD" if len(name) % 2 else "HND", outlier_frac=0.01)
     ref, written = orc.paged_decode(c.q, c.cache.key_cache, c.cache.value_cache, c.cache.k_scale, c.cache.v_scale,
                                     c.block_table, c.seq_lens, c.query_start_loc, c.num_seqs, c.scale, c.window, c.causal)
     print(f"balanced {name} causal={causal}", flush=True)
-    nsplit = min(nseg, 4)
     d, out, parts = decode(c, nseg, nsplit)
+    assert dealt(parts, nsplit), "this batch does not run the kernel"
     o = out.double().cpu().numpy()
     emax, emean, over, over_mean = kvc.fp16_output_errors(o[written], ref[written])
     print(f"  max-abs {emax:.2e} mean-abs {emean:.2e}", flush=True)
@@ -88,11 +94,6 @@ def test_batches(name, causal):
     torch.cuda.synchronize()
     sel = torch.from_numpy(written).cuda()
     assert torch.equal(again[sel], out[sel])
-
-
-def dealt(parts, nsplit):
-    """Whether the call ran pd_balanced_kernel: only that writes more than nsplit segments of the partial buffers."""
-    return not parts[1][:, :, nsplit:].isnan().all().item()
 
 
 # segments, splits, whether the batch (65 sequences x 4 kv heads: past one round at any count) is dealt
