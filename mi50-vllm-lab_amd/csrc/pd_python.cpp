@@ -412,18 +412,47 @@ PyObject* plan_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (sq > 0 && items > 0) {
             const int64_t nqt = ceil_div(sq, std::max<int64_t>(1, tok)), heads = items / nqt;
             const int64_t wide_items = ceil_div(head_rows, 256) * heads;
+            auto wide = [&](int64_t s) { return pd::fa_wide_saves(ceil_div(wide_items * s, cus), ceil_div(items * s, cus), exact != 0); };
             for (int64_t s = 1; s <= top && fits(s); ++s) {
-                if (!pd::fa_wide_saves(ceil_div(wide_items * s, cus), ceil_div(items * s, cus), exact != 0)) continue;
+                if (!wide(s)) continue;
                 const double t = cost(wide_items, s, times.wide_tile);
                 if (t < best_t) best = s, best_t = t;
             }
+            // key tiles that a workgroup whose last token is `last` - 1 sees
+            auto seen = [&](int64_t last) { return ceil_div(std::max<int64_t>(0, keys - sq) + std::min(sq, last), 32); };
+            // A launch of s splits as the hardware runs it (pd_prefill_kernel's order): each of the 8 XCDs has a contiguous
+            // part of the workgroups, a query tile's splits apart and the tiles ascending, and starts the next one on
+            // the CU that is free first. The workgroups' lengths differ by the causal triangle, which the rounds above do
+            // not see: 3 chunks of 1,000 fresh tokens run 109 us unsplit (114 here, 137 in rounds) and 133 dealt.
+            auto ordered = [&](int64_t s, int64_t sequences) {
+                const bool w = wide(s);
+                const int64_t nq = w ? ceil_div(head_rows, 256) : nqt, group = std::max<int64_t>(1, head_rows / sq);
+                const int64_t total = nq * s * sequences, lanes = std::max<int64_t>(1, cus / 8);
+                if (total > 64 * cus) return 0.0;  // many rounds: as even as dealt
+                double span = 0.0;
+                for (int64_t xcd = 0, i = 0; xcd < 8; ++xcd) {
+                    std::priority_queue<double, std::vector<double>, std::greater<double>> busy;
+                    for (const int64_t end = i + total / 8 + (xcd < total % 8 ? 1 : 0); i < end; ++i) {
+                        const int64_t x = i % (nq * s), q = x % nq, split = x / nq;
+                        const int64_t t = seen(w ? std::min((q + 1) * 256 - 1, head_rows - 1) / group + 1 : (q + 1) * tok);
+                        const int64_t per = ceil_div(t, s), mine = std::max<int64_t>(0, std::min(per, t - split * per));
+                        double at = (double)mine * (w ? times.wide_tile : times.tile) + wg_us;
+                        if ((int64_t)busy.size() == lanes) {
+                            at += busy.top();
+                            busy.pop();
+                        }
+                        busy.push(at);
+                        span = std::max(span, at);
+                    }
+                }
+                return s > 1 ? span + merge_us + mb_us * (double)rows * (double)s * 1032 / 1e6 : span;
+            };
             int64_t units = 0;
-            for (int64_t q = 0; q < nqt; ++q)
-                units += ceil_div(std::max<int64_t>(0, keys - sq) + std::min(sq, (q + 1) * tok), 32) + pd::kFaSegmentUnits;
+            for (int64_t q = 0; q < nqt; ++q) units += seen((q + 1) * tok) + pd::kFaSegmentUnits;
             const int64_t share = std::max<int64_t>(pd::kFaMinShare, ceil_div(units * heads, cus)), ns = items <= cus ? cus / items : 0;
             const bool aligned = ns > 0 && ceil_div(tiles, ns) <= share + share / pd::kFaAlignedPart;
             const double dealt = times.deal_unit * (double)(share + pd::kFaDealSpareUnits) + pd::kFaDealFixedUs;
-            if (!aligned && dealt < pd::kFaDealMargin * best_t) best = 0;
+            if (!aligned && dealt < pd::kFaDealMargin * best_t && dealt < pd::kFaDealMargin * ordered(best, heads)) best = 0;
         }
         return PyLong_FromLongLong(best);
     });

@@ -1,6 +1,7 @@
 """pd_native (csrc/pd_python.cpp) on the CPU: the split plans equal their models, and errors come back as the
 Python exceptions that the operators document. The calls themselves are covered by every GPU test.
 """
+import heapq
 import math
 import os
 import random
@@ -114,8 +115,9 @@ SEGMENT, MIN_SHARE, ALIGNED, SPARE, DEAL_US, MARGIN = (
 
 
 def chunk_model(batch, sq, hq, hkv, keys, bs, exact, cus=256):
-    """pd_native.plan_prefill for a chunk whose tokens are the last of `keys` keys: {split count: (us, kernel)}, and the
-    us of the dealt launch (None where it would cut the query tiles evenly)."""
+    """pd_native.plan_prefill for a chunk whose tokens are the last of `keys` keys: {split count: (us, kernel)}, the us of
+    the dealt launch (None where it would cut the query tiles evenly), and the us of a split count in the order of its
+    workgroups."""
     tile, wide, unit = TIMES[exact]
     g, tiles = hq // hkv, -(-keys // 32)
     tok = 192 // g
@@ -137,9 +139,32 @@ def chunk_model(batch, sq, hq, hkv, keys, bs, exact, cus=256):
     units = sum(-(-(max(0, keys - sq) + min(sq, (q + 1) * tok)) // 32) + SEGMENT for q in range(qtiles)) * hkv * batch
     share = max(MIN_SHARE, -(-units // cus))
     ns = cus // items
-    if ns and -(-tiles // ns) <= share + share // ALIGNED:
-        return out, None
-    return out, unit * (share + SPARE) + DEAL_US
+    dealt = None if ns and -(-tiles // ns) <= share + share // ALIGNED else unit * (share + SPARE) + DEAL_US
+
+    def ordered(s):
+        w = -(-wide_items * s // cus) * wide < -(-items * s // cus) * tile
+        nq = -(-sq * g // 256) if w else qtiles
+        launch = []
+        for _ in range(hkv * batch):
+            for split in range(s):
+                for q in range(nq):
+                    last = min((q + 1) * 256 - 1, sq * g - 1) // g + 1 if w else min(sq, (q + 1) * tok)
+                    t = -(-(max(0, keys - sq) + last) // 32)
+                    per = -(-t // s)
+                    launch.append(max(0, min(per, t - split * per)) * (wide if w else tile) + pth_dec.PREFILL_US_PER_WORKGROUP)
+        if len(launch) > 64 * cus:
+            return 0.0
+        span = at = 0
+        for xcd in range(8):
+            free = [0.0] * (cus // 8)
+            n = len(launch) // 8 + (xcd < len(launch) % 8)
+            for us in launch[at:at + n]:
+                span = max(span, us + free[0])
+                heapq.heapreplace(free, us + free[0])
+            at += n
+        merge = pth_dec.PREFILL_US_MERGE_LAUNCH + pth_dec.PREFILL_US_PER_PARTIAL_MB * rows * s * 1032 / 1e6 if s > 1 else 0.0
+        return span + merge
+    return out, dealt, ordered
 
 
 @pytest.mark.parametrize("exact", [False, True], ids=["default", "exact"])
@@ -150,14 +175,28 @@ def test_chunk_plan_equals_its_model(seed, exact):
         hkv = r.choice([1, 2, 4, 8])
         batch, hq, sq = r.choice([1, 1, 3]), hkv * r.choice([1, 4, 6, 8]), r.choice([r.randint(1, 100), r.randint(1, 6000), 2048])
         keys, bs = sq + r.choice([0, r.randint(1, 2000), r.randint(1, 300000)]), r.choice([1, 8, 16, 48, 1584])
-        counts, dealt = chunk_model(batch, sq, hq, hkv, keys, bs, exact)
+        counts, dealt, ordered = chunk_model(batch, sq, hq, hkv, keys, bs, exact)
         best = min(t for t, _ in counts.values())
         got = pth_dec._prefill_plan(batch, sq, hq, hkv, keys, bs, sq, exact)
-        assert (got == 0) == (dealt is not None and dealt < MARGIN * best), (counts, dealt, got)
+        first = min(s for s, (t, _) in counts.items() if t == min(t for t, _ in counts.values()))
+        deal = dealt is not None and dealt < MARGIN * best and dealt < MARGIN * ordered(first)
+        assert (got == 0) == deal, (counts, dealt, got)
         if got:
             assert counts[got][0] == pytest.approx(best, rel=1e-12)
         seen.add(0 if got == 0 else counts[got][1])
     assert seen == {0, 192, 256}  # every kernel is planned somewhere
+
+
+# batch, tokens, cached keys (24 q / 4 kv heads), exact, us unsplit, us dealt
+FRESH_BATCHES = [(3, 1000, 0, False, 109.3, 133.0), (2, 1900, 0, False, 169.4, 201.7), (4, 1600, 0, False, 236.4, 280.9),
+                 (2, 2000, 1000, False, 282.1, 320.1), (2, 3000, 0, False, 340.1, 372.5), (3, 1000, 0, True, 127.2, 145.8),
+                 (1, 4000, 0, False, 371, 303), (1, 3000, 0, True, 337, 228), (1, 6000, 0, False, 776, 593)]
+
+
+@pytest.mark.parametrize("batch,sq,ctx,exact,unsplit,dealt", FRESH_BATCHES)
+def test_fresh_batches_are_planned_as_measured(batch, sq, ctx, exact, unsplit, dealt):
+    got = pth_dec._prefill_plan(batch, sq, 24, 4, ctx + sq, 16, sq, exact)
+    assert (got == 0) == (dealt < unsplit)
 
 
 def test_plan_and_launch_share_the_tile_times():
