@@ -13,8 +13,8 @@
 //   groups of more than 16 rows are instead sliced into 16-row workgroups (grid z = slice x
 //   sequence) when nsplit x Hkv x num_seqs x slices fits the CUs and num_seqs x window is at most
 //   16,384 keys: then the slices' repeated reads of the tiles cost less than the split partials
-//   they save. Batches of several sequences beyond one round of the CUs run pd_balanced_kernel
-//   instead: one workgroup per CU, each an even share of all (sequence, kv head) tiles.
+//   they save. Batches of several sequences whose splits take more than one round of the CUs run
+//   pd_balanced_kernel instead: one workgroup per CU, each an even share of all (sequence, kv head) tiles.
 //
 // Memory path: HBM -> LDS by DMA (global_load_lds_dwordx4), double-buffered per wave, no VGPR
 //   holding data in flight. A tile is 17 DMA instructions of 1 KiB: 8 for K (4 rows x 256

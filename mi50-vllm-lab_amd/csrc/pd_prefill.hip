@@ -648,11 +648,12 @@ __global__ void __launch_bounds__(kFaWaves * 64, 1) pd_prefill_kernel(const FaPa
 // segment (kFaSegmentUnits), and each workgroup takes `share` consecutive units; items that need about the
 // same are cut into ns equal pieces instead. A workgroup that covers all of an item's tiles stores its rows;
 // the pieces of the others go to the workgroup's two slots of the workspace (its first segment, its
-// last), which pd_prefill_merge_kernel adds up. Measured (24 q / 4 kv heads, whole call): a fresh prompt of 4,000
-// tokens 398 us in one workgroup per query tile, 376 in 2 splits, 327 here; 700 tokens over 6,000 keys 207 (2
-// splits) against 184; a batch of 9 decoded sequences and chunks of 70 to 900 tokens over 1,500 to
+// last), which pd_prefill_merge_kernel adds up. Measured (24 q / 4 kv heads, fp16 rows): a fresh prompt of 4,000
+// tokens 371 us in one workgroup per query tile, 314 in 2 splits, 303 here; 1,501 tokens over 3,000 keys 239, 219 (3
+// splits), 214; a batch of 9 decoded sequences and chunks of 70 to 900 tokens over 1,500 to
 // 6,000 keys 481 -> 302 (four launches, with a transpose and two conversions each, before). Where all
-// query tiles need the same (2,048 tokens over 61,440) the splits' kernel is 3 % faster and is taken.
+// query tiles need the same (2,048 tokens over 61,440) the splits' kernel takes less per tile (1.62 us against 1.75)
+// and is taken.
 constexpr unsigned kFaMaxPieces = 64;     // pieces of an item (the merge holds one per lane)
 
 struct FaLine {

@@ -136,7 +136,8 @@ def decode_splits(nseg: int, window: int, num_kv_heads: int, num_seqs: int, devi
     6 q heads per kv head when not given). Few splits for many sequences, many for one long
     sequence. Without the lengths: a sliding window bounds every sequence to about window + qmax
     keys, so the grid is sized to one workgroup per CU; otherwise the cap (the reference's
-    rule). Before either: windowed groups of more than 16 rows take the count at which the
+    rule). A count whose workgroups take more than one round of the CUs is no more than the sign for the
+    operator to deal the tiles itself (see launched_splits for 1). Before either: windowed groups of more than 16 rows take the count at which the
     operator slices them into one round of 16-row workgroups (sliced_splits), when that is at
     least 2."""
     cap = max(1, min(PTH_DEC_SPLITS, nseg))
