@@ -1,5 +1,5 @@
 // Internal interface of libpthdec.so between the C ABI (pd_api.hip) and the kernel files
-// (pd_decode.hip, pd_prefill.hip, pd_cache_write.hip): the parameter block each kernel takes and
+// (pd_decode.hip, pd_prefill.hip, pd_prefill_wide.hip, pd_cache_write.hip): the parameter block each kernel takes and
 // the host functions that launch them. The public interface is include/pth_dec.h; nothing here
 // is exported from the library.
 #pragma once
